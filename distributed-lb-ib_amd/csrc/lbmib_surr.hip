@@ -779,309 +779,411 @@ __global__ void k_flip(const uint16_t *__restrict__ w, uint16_t *__restrict__ wt
 //
 // dw[co][t][ci] = sum_v dy[v][co] x[v + o(t)][ci]: per tap a GEMM whose
 // reduction runs over voxels.  A block owns a 32 x 32 (co, ci) tile (16 for
-// 16-channel tensors) and all 27 taps, spread over its 4 waves (taps
-// w, w + 4, ...: 7 accumulator tiles per wave), and a contiguous range of
-// 32-voxel chunks (the last one zero-filled past the end).  Per chunk it stages dy[32 voxels][co tile] and, for
-// every tap, x[neighbour][ci tile] in LDS with natural (channel-fastest)
-// 16-byte pieces; the MFMA operands need 8 consecutive voxels per lane, so
-// lanes gather them with 2-byte LDS reads.  A row pitch of 36 elements
-// (72 bytes) puts the four 8-voxel groups of a fragment on distinct banks.
-constexpr int kWgPitch = 36;
-constexpr int kWgChunk = 32;
-constexpr int kWgBox = kWgChunk + 2;  // a chunk's voxels and one more on each side
+// 16-channel tensors), the 9 taps of one dz and a contiguous range of units;
+// its 4 waves each multiply a quarter of a unit's voxels for all 9 taps (9 x
+// NA x NB accumulator fragments), and add up through LDS at the end.
+//
+// A unit is up to 128 voxels as 16 runs of 8 consecutive x (lane group kq =
+// lane >> 4 of wave w takes run 4w + kq as its 8 reduction slots): R whole
+// lines of a z-plane, P whole planes where a plane is small, or R lines of a
+// 32-voxel x segment where a line is longer than 64.  The unit's dy and the
+// lines of x around it at plane z + dz are staged in LDS channel-fastest, as
+// they lie in memory, zeros outside the volume; ds_read_b64_tr_b16 hands each
+// lane 4 consecutive voxels of its channel, so an operand fragment is two
+// 8-byte reads where gathering it takes eight 2-byte ones and the packing.
+// Three such reads hold the 12 voxels from one before the run on: taps dx =
+// -1 and +1 are registers of them as they are, dx = 0 four v_alignbit.
+//
+// 36 MFMAs per wave and unit against 22 LDS reads; the next unit's loads are
+// in flight meanwhile and go into the other LDS buffer (one barrier per
+// unit), and what bounds it is their latency.  Measured, this kernel against
+// the form that gathered its operands with 2-byte LDS reads: 154 against 539
+// us at batch 4 x 64^3, 32 -> 32 channels (376 TFLOP/s), 43 against 150 us at
+// batch 4 x 16^3, 128 -> 128.
+constexpr int kWgRuns = 16;
+constexpr int kWgXP = 4, kWgYP = 2;  // 16-byte pieces per thread of a unit's x and dy at most
 
-__global__ void __launch_bounds__(256) k_conv_wgrad(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy,
-                                                    float *__restrict__ part, int D, int H, int W, long M, int Cin,
-                                                    int Cout, int ci_tiles, int chunks_per_split, long nchunks) {
-  // the chunk's neighbourhood: for each (dz, dy), interval j = 3 (dz + 1) +
-  // dy + 1 of kWgBox linear voxel indices starting one before the chunk's
-  // first voxel shifted by dz HW + dy W; tap (dz, dy, dx) of voxel p is slot
-  // p + 1 + dx of interval j wherever that neighbour lies in the volume
-  __shared__ uint16_t sx[9 * kWgBox * kWgPitch];
-  __shared__ uint16_t sdy[kWgChunk * kWgPitch];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 15, kq = lane >> 4;
-  const int ci0 = (blockIdx.x % ci_tiles) * 32, co0 = (blockIdx.x / ci_tiles) * 32;
-  const int nci = Cin - ci0 >= 32 ? 2 : 1;  // 16-channel fragments in the tile
-  const int nco = Cout - co0 >= 32 ? 2 : 1;
-  const long HW = (long)H * W;
-  const int K = 27 * Cin;
-  f32x4 acc[7][2][2];
-#pragma unroll
-  for (int tt = 0; tt < 7; ++tt)
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) acc[tt][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const long c_begin = (long)blockIdx.y * chunks_per_split;
-  long c_end = c_begin + chunks_per_split;
-  if (c_end > nchunks) c_end = nchunks;
-  const int lgxp = nci == 2 ? 2 : 1;  // log2 of the 8-channel pieces per voxel in the ci tile
-  const int npx = 9 * kWgBox << lgxp;
-  const int npy = kWgChunk * nco * 2;
-  // the chunk's voxels: x, y, z within the sample, and 1 if the voxel exists
-  __shared__ int svc[kWgChunk][4];
-  constexpr int kXRounds = (9 * kWgBox * 4 + 255) / 256;  // x pieces per thread at most
-  for (long c = c_begin; c < c_end; ++c) {
-    const long v0 = c * kWgChunk;
-    if (tid < kWgChunk) {
-      const long v = v0 + tid;
-      int cv[4] = {0, 0, 0, 0};
-      if (v < M) {
-        long rr = v;
-        cv[0] = (int)(rr % W);
-        rr /= W;
-        cv[1] = (int)(rr % H);
-        rr /= H;
-        cv[2] = (int)(rr % D);
-        cv[3] = 1;
-      }
-#pragma unroll
-      for (int a = 0; a < 4; ++a) svc[tid][a] = cv[a];
-    }
-    // every piece's load is issued before any is stored: an unconditional
-    // load from a valid address (the tensor's start for an index outside
-    // [0, M)), the value zeroed after it
-    u32x4 px[kXRounds];
-    bool pok[kXRounds];
-#pragma unroll
-    for (int r = 0; r < kXRounds; ++r) {
-      const int e = tid + 256 * r;
-      const uint16_t *src = x;
-      bool ok = false;
-      if (e < npx) {
-        const int q = e & ((1 << lgxp) - 1), rest = e >> lgxp, sl = rest % kWgBox, j = rest / kWgBox;
-        const long li = v0 - 1 + sl + (long)(j / 3 - 1) * HW + (long)(j % 3 - 1) * W;
-        ok = li >= 0 && li < M;
-        if (ok) src = x + li * Cin + ci0 + q * 8;
-      }
-      px[r] = *(const u32x4 *)src;
-      pok[r] = ok;
-    }
-#pragma unroll
-    for (int r = 0; r < kXRounds; ++r) {
-      const int e = tid + 256 * r;
-      if (e < npx) {
-        const int q = e & ((1 << lgxp) - 1), rest = e >> lgxp;
-        const u32x4 val = pok[r] ? px[r] : u32x4{0u, 0u, 0u, 0u};
-        uint16_t *dst = sx + rest * kWgPitch + q * 8;
-        *(u32x2 *)dst = u32x2{val[0], val[1]};
-        *(u32x2 *)(dst + 4) = u32x2{val[2], val[3]};
-      }
-    }
-    u32x4 py = {0u, 0u, 0u, 0u};
-    bool yok = false;
-    {
-      const int q = tid % (nco * 2), p = tid / (nco * 2);
-      const uint16_t *src = dy;
-      if (tid < npy && v0 + p < M) {
-        src = dy + (v0 + p) * Cout + co0 + q * 8;
-        yok = true;
-      }
-      py = *(const u32x4 *)src;
-    }
-    if (tid < npy) {
-      const int q = tid % (nco * 2), p = tid / (nco * 2);
-      const u32x4 val = yok ? py : u32x4{0u, 0u, 0u, 0u};
-      uint16_t *dst = sdy + p * kWgPitch + q * 8;
-      *(u32x2 *)dst = u32x2{val[0], val[1]};
-      *(u32x2 *)(dst + 4) = u32x2{val[2], val[3]};
-    }
-    __syncthreads();
-    // which of this lane's voxels p = 8 kq + e have their neighbour at
-    // offset d - 1 along x, y, z inside the volume (bit e); mz also carries
-    // whether the voxel exists
-    uint32_t mx[3] = {0u, 0u, 0u}, my[3] = {0u, 0u, 0u}, mz[3] = {0u, 0u, 0u};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int *cv = svc[kq * 8 + e];
-      const int vx = cv[0], vy = cv[1], vz = cv[2], ex = cv[3];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        mx[d] |= (uint32_t)((unsigned)(vx + d - 1) < (unsigned)W) << e;
-        my[d] |= (uint32_t)((unsigned)(vy + d - 1) < (unsigned)H) << e;
-        mz[d] |= (uint32_t)(ex && (unsigned)(vz + d - 1) < (unsigned)D) << e;
-      }
-    }
-    // A: dy^T fragments (row co = 16 a + col, voxels 8 kq .. + 8)
-    bf16x8 fa[2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      uint16_t h[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) h[e] = sdy[(kq * 8 + e) * kWgPitch + a * 16 + col];
-      u32x4 pk;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) pk[e] = (uint32_t)h[2 * e] | ((uint32_t)h[2 * e + 1] << 16);
-      fa[a] = __builtin_bit_cast(bf16x8, pk);
-    }
-#pragma unroll
-    for (int tt = 0; tt < 7; ++tt) {
-      const int t = wave + 4 * tt;
-      if (t >= 27) break;
-      const int tz = t / 9, ty = (t / 3) % 3, tx = t % 3;
-      const uint32_t vm = mx[tx] & my[ty] & mz[tz];
-      const uint16_t *row = sx + ((tz * 3 + ty) * kWgBox + kq * 8 + tx) * kWgPitch;
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        if (b >= nci) break;
-        uint16_t h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint16_t v = row[e * kWgPitch + b * 16 + col];
-          h[e] = (vm >> e) & 1u ? v : (uint16_t)0;
-        }
-        u32x4 pk;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pk[e] = (uint32_t)h[2 * e] | ((uint32_t)h[2 * e + 1] << 16);
-        const bf16x8 fb = __builtin_bit_cast(bf16x8, pk);
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          if (a >= nco) break;
-          acc[tt][a][b] = mfma16(fa[a], fb, acc[tt][a][b]);
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // partials: lane holds (co = co0 + 16 a + 4 kq + r, ci = ci0 + 16 b + col)
-  float *dst = part + (long)blockIdx.y * Cout * K;
-#pragma unroll
-  for (int tt = 0; tt < 7; ++tt) {
-    const int t = wave + 4 * tt;
-    if (t >= 27) break;
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      if (a >= nco) break;
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        if (b >= nci) break;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int co = co0 + a * 16 + 4 * kq + r, ci = ci0 + b * 16 + col;
-          dst[(long)co * K + t * Cin + ci] = acc[tt][a][b][r];
-        }
-      }
-    }
-  }
-}
-
-// out[e] = sum over s < ns of part[s][e], in order of s
-// out[e] = sum over k < ns of part[k][e], in a fixed order.  A block covers
-// 64 consecutive e (one per lane, so every wave reads 256 contiguous bytes
-// per k) and its 4 waves split k: wave g sums k = g, g + 8, g + 16, ... and
-// k = g + 4, g + 12, ... in two running sums; the four waves' sums are then
-// added through LDS as (w0 + w1) + (w2 + w3).  Launch with kSumBlock
-// threads and ceil(n / 64) blocks.
-constexpr int kSumBlock = 256;
-__global__ void __launch_bounds__(kSumBlock) k_sum_parts(const float *__restrict__ part, float *__restrict__ out,
-                                                         long n, int ns) {
-  __shared__ float red[4][64];
-  const int el = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const long e = (long)blockIdx.x * 64 + el;
-  float s0 = 0.f, s1 = 0.f;
-  if (e < n) {
-    int k = g;
-    for (; k + 4 < ns; k += 8) {
-      s0 += part[(long)k * n + e];
-      s1 += part[(long)(k + 4) * n + e];
-    }
-    if (k < ns) s0 += part[(long)k * n + e];
-  }
-  red[g][el] = s0 + s1;
-  __syncthreads();
-  if (g == 0 && e < n) out[e] = (red[0][el] + red[1][el]) + (red[2][el] + red[3][el]);
-}
-
-// bias gradient partials: part[blk][co] = sum of dy[v][co] over the block's
-// voxel range.  A thread sums 8 channels of every G-th voxel (16-byte
-// loads; G = 256 / (C / 8) voxel lanes), then the G lanes of each channel
-// group are added through LDS in lane order.  C is a multiple of 16 and at
-// most 512.
-__global__ void __launch_bounds__(256) k_colsum(const uint16_t *__restrict__ dy, float *__restrict__ part, long M,
-                                                int C, long per_block) {
-  __shared__ float red[256][9];
-  const int ng = C / 8, G = 256 / ng;  // channel groups, voxel lanes
-  const int tid = threadIdx.x, cg = tid % ng, vl = tid / ng;
-  const long v0 = (long)blockIdx.x * per_block;
-  long v1 = v0 + per_block;
-  if (v1 > M) v1 = M;
-  for (int c0 = 0; c0 < C; c0 += 8 * ng) {  // one pass: 8 ng = C
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (vl < G)
-      for (long v = v0 + vl; v < v1; v += G) {
-        const u32x4 q = *(const u32x4 *)(dy + v * C + c0 + 8 * cg);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[2 * r] += bf2f((uint16_t)(q[r] & 0xffff));
-          s[2 * r + 1] += bf2f((uint16_t)(q[r] >> 16));
-        }
-      }
-#pragma unroll
-    for (int r = 0; r < 8; ++r) red[tid][r] = s[r];
-    __syncthreads();
-    for (int ch = tid; ch < 8 * ng; ch += 256) {
-      const int g = ch / 8, r = ch % 8;
-      float t = 0.f;
-      for (int k = 0; k < G; ++k) t += red[k * ng + g][r];
-      part[(long)blockIdx.x * C + c0 + ch] = t;
-    }
-    __syncthreads();
-  }
-}
-
-// Split of the voxel reduction: chunks per split, chosen from the shape only
-// (so every entry point that shares it gives the same bits), capped so that
-// the partials fit in `cap_bytes`.
-struct WgradPlan {
-  int ci_tiles, co_tiles, splits, cps;
-  long nchunks;
-  size_t part_bytes;
+struct WgGeo {
+  int TX, nr, R, P;  // voxels of a line segment, its runs of 8, lines per plane, planes
+  int halo;          // 1: segments of a longer line, loaded with their x neighbours
+  int nlx, l0;       // x lines loaded per plane, and the LDS line of the first: R + 2, 0, or R, 1 where R = H
+  int LP;            // LDS voxels per line: index i is x = xs + i - 1
+  int nseg, nyb;     // segments per line, line groups per plane
+  long planes, nunits;
+  int xbytes, ybytes;  // of one LDS buffer
 };
 
-WgradPlan wgrad_plan(long M, int Cin, int Cout, size_t cap_bytes) {
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// 4 voxels of one channel: lane i of each 16 passes the address of row
+// (i & 15) >> 2 (a voxel), channels 4 (i & 3) .. + 3, and receives rows 0..3
+// of channel i & 15.
+__device__ __forceinline__ u32x2 lds_tr4(const char *p) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p));
+}
+
+template <int NA, int NB, bool BIG>
+__global__ void __launch_bounds__(256, 2)
+    k_conv_wgrad(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part,
+                 float *__restrict__ bpart, WgGeo q, int D, int H, int W, int Cin, int Cout, int ci_tiles, int tiles,
+                 int splits, long units_per_split) {
+  constexpr int VX = 32 * NB, VY = 32 * NA;  // bytes per voxel in LDS
+  constexpr uint32_t kNone = 0x80000000u;    // past the end of the resources: loads zeros
+  extern __shared__ __attribute__((aligned(16))) char sm[];  // two buffers of x and dy, then 12 voxels of zeros
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kq = lane >> 4;
+  // Workgroup b runs on XCD b % 8: the three dz of a split and tile, which
+  // read the same dy and neighbouring planes of x, follow each other there.
+  const int jobs = tiles * 3 * splits, per = (jobs + 7) / 8;
+  const int job = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || job >= jobs) return;
+  const int dzi = job % 3, tile = (job / 3) % tiles, split = job / (3 * tiles);
+  const int ci0 = (tile % ci_tiles) * 32, co0 = (tile / ci_tiles) * 32;
+  const int buf_bytes = q.xbytes + q.ybytes;
+
+  // this thread's pieces: where they lie in memory relative to the unit, and
+  // (in one register each) line, plane and x within it, which decide whether
+  // they exist, and the LDS piece they go to
+  uint32_t xo[kWgXP], yo[kWgYP], xl[kWgXP], yl[kWgYP];
+  constexpr uint32_t kNoPiece = 0x80000000u;
+  auto pack = [](int l, int p, int ix, int at) { return (uint32_t)(l | p << 5 | ix << 10 | (at >> 4) << 17); };
+  auto line_of = [](uint32_t v) { return (int)(v & 31); };
+  auto plane_of = [](uint32_t v) { return (int)(v >> 5 & 31); };
+  auto x_of = [](uint32_t v) { return (int)(v >> 10 & 127); };
+  auto at_of = [](uint32_t v) { return (int)(v >> 17 << 4); };
+  const int SX = min(W, q.TX) + 2 * q.halo, TXs = min(W, q.TX);
+#pragma unroll
+  for (int r = 0; r < kWgXP; ++r) {
+    const int e = tid + 256 * r, pc = e & (2 * NB - 1), v = e / (2 * NB);
+    const int ix = v % SX, ln = v / SX, l = ln % q.nlx, p = ln / q.nlx;
+    const int L = p * (q.R + 2) + l + q.l0, i = ix + 1 - q.halo;
+    const int s = NB == 2 ? ((i >> 3) + L) & 1 : 0;
+    xo[r] = (uint32_t)((((long)p * H + l) * W + ix) * Cin * 2 + pc * 16);
+    xl[r] = p < q.P ? pack(l, p, ix, (L * q.LP + i) * VX + (((pc >> 1) ^ s) * 32) + (pc & 1) * 16) : kNoPiece;
+  }
+#pragma unroll
+  for (int r = 0; r < kWgYP; ++r) {
+    const int e = tid + 256 * r, pc = e & (2 * NA - 1), v = e / (2 * NA);
+    const int ix = v % TXs, ln = v / TXs, l = ln % q.R, p = ln / q.R;
+    const int run = (p * q.R + l) * q.nr + (ix >> 3);
+    yo[r] = co0 + pc * 8 < Cout ? (uint32_t)((((long)p * H + l) * W + ix) * Cout * 2 + pc * 16) : kNone;
+    const int h = NA == 2 ? (pc >> 1) ^ (run & 1) : 0;
+    yl[r] = p < q.P ? pack(l, p, ix, q.xbytes + (run * 8 + (ix & 7)) * VY + h * 32 + (pc & 1) * 16) : kNoPiece;
+  }
+  // this lane's run: LDS addresses of its x (line dy = -1) and dy operands
+  const int run = 4 * wave + kq, rx = run % q.nr, rl = (run / q.nr) % q.R, rp = run / (q.nr * q.R);
+  const bool has_run = rp < q.P;
+  const int rowb = (lane & 15) >> 2, colb = (lane & 3) * 8;
+  const int L0 = rp * (q.R + 2) + rl;
+  const int xa0 = (L0 * q.LP + 8 * rx + rowb) * VX + colb, xs0 = NB == 2 ? ((rx + L0) & 1) * 32 : 0;
+  const int ya0 = q.xbytes + (run * 8 + rowb) * VY + colb, ys0 = NA == 2 ? (run & 1) * 32 : 0;
+  const int zero_at = 2 * buf_bytes + rowb * VX + colb;
+  const bool tails = q.halo || (W & 7);  // lines whose last run is not full
+
+  // the unit sequence: plane group, line group, segment
+  long u = (long)split * units_per_split;
+  const long u_end = min(u + units_per_split, q.nunits);
+  int sg = (int)(u % q.nseg), yb = (int)(u / q.nseg % q.nyb);
+  long pg = u / q.nseg / q.nyb;
+  int z0 = (int)(pg * q.P % D);  // the first plane's z
+  auto step = [&]() {
+    ++u;
+    if (++sg == q.nseg) {
+      sg = 0;
+      if (++yb == q.nyb) {
+        yb = 0;
+        ++pg;
+        for (z0 += q.P; z0 >= D;) z0 -= D;
+      }
+    }
+  };
+  // (a single plane whose z + dz lies outside the volume adds nothing)
+  auto skip = [&]() {
+    while (u < u_end && q.P == 1 && (unsigned)(z0 + dzi - 1) >= (unsigned)D) step();
+  };
+  u32x4 px[kWgXP], py[kWgYP];
+  auto fetch = [&]() {
+    const long pl = pg * q.P;
+    const int y0 = yb * q.R, xs = sg * q.TX, yx = y0 - (1 - q.l0);
+    const uint16_t *bx = x + (((pl + dzi - 1) * H + yx) * W + xs - q.halo) * Cin + ci0;
+    const uint16_t *by = dy + ((pl * H + y0) * W + xs) * Cout + co0;
+    const __amdgpu_buffer_rsrc_t rx_ = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(bx), (short)0, 0x7fffffff,
+                                                                        0x00020000);
+    const __amdgpu_buffer_rsrc_t ry_ = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(by), (short)0, 0x7fffffff,
+                                                                        0x00020000);
+#pragma unroll
+    for (int r = 0; r < kWgXP; ++r) {
+      const int l = line_of(xl[r]), p = plane_of(xl[r]), ix = x_of(xl[r]);
+      bool ok = xl[r] != kNoPiece && (unsigned)(yx + l) < (unsigned)H && (unsigned)(xs + ix - q.halo) < (unsigned)W;
+      if (q.P > 1) ok = ok && pl + p < q.planes && (unsigned)((z0 + p) % D + dzi - 1) < (unsigned)D;
+      if constexpr (BIG) {
+        const int pc = (tid + 256 * r) & (2 * NB - 1);
+        const uint16_t *src = ok ? bx + (((long)p * H + l) * W + ix) * Cin + pc * 8 : x;
+        px[r] = ok ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
+      } else {
+        px[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx_, ok ? xo[r] : kNone, 0, 0));
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kWgYP; ++r) {
+      const int l = line_of(yl[r]), p = plane_of(yl[r]), ix = x_of(yl[r]);
+      const bool ok = yl[r] != kNoPiece && y0 + l < H && xs + ix < W && pl + p < q.planes;
+      if constexpr (BIG) {
+        const int pc = (tid + 256 * r) & (2 * NA - 1);
+        const bool in = ok && yo[r] != kNone;
+        const uint16_t *src = in ? by + (((long)p * H + l) * W + ix) * Cout + pc * 8 : dy;
+        py[r] = in ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
+      } else {
+        py[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ry_, ok ? yo[r] : kNone, 0, 0));
+      }
+    }
+  };
+  auto put = [&](char *b) {
+#pragma unroll
+    for (int r = 0; r < kWgXP; ++r)
+      if (xl[r] != kNoPiece) *(u32x4 *)(b + at_of(xl[r])) = px[r];
+#pragma unroll
+    for (int r = 0; r < kWgYP; ++r)
+      if (yl[r] != kNoPiece) *(u32x4 *)(b + at_of(yl[r])) = py[r];
+  };
+
+  f32x4 acc[9][NA][NB], accb[NA];
+#pragma unroll
+  for (int a = 0; a < NA; ++a) {
+    accb[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[t][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const bool want_b = bpart && dzi == 1 && ci0 == 0;  // this block also sums dy over the voxels
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+
+  // what no piece fills stays zero: the neighbours outside a line, lines
+  // outside the plane, slots past the unit's runs
+  for (int k = tid * 16; k < 2 * buf_bytes + 12 * VX; k += 256 * 16) *(u32x4 *)(sm + k) = u32x4{0u, 0u, 0u, 0u};
+  skip();
+  if (u < u_end) fetch();
+  __syncthreads();
+  if (u < u_end) put(sm);
+  __syncthreads();
+  int buf = 0;
+  while (u < u_end) {
+    // the lanes whose run lies past the unit or the plane multiply zeros by zeros
+    const bool in = has_run && yb * q.R + rl < H;
+    const int boff = buf * buf_bytes;
+    const int xa = in ? boff + xa0 : zero_at, lstep = in ? q.LP * VX : 0, xs1 = in ? xs0 : 0;
+    u32x4 tm = {~0u, ~0u, ~0u, ~0u};  // clears x[last voxel] where dx = -1 pairs it with a voxel past the line
+    if (tails) {
+      const int e0 = W - sg * q.TX - 8 * rx;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (e0 == k) tm[k >> 1] = k & 1 ? 0x0000ffffu : 0xffff0000u;
+    }
+    step();
+    skip();
+    const bool more = u < u_end;
+    if (more) fetch();
+    bf16x8 fa[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+      const char *p = sm + boff + ya0 + ((32 * a) ^ ys0);
+      const u32x2 lo = lds_tr4(p), hi = lds_tr4(p + 4 * VY);
+      fa[a] = __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+    }
+    if (want_b)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) accb[a] = mfma16(fa[a], ones, accb[a]);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        // (the half of a voxel's channels alternates with the 8-voxel block
+        // and the line, so that two runs' reads fall on distinct banks)
+        const int h = NB == 2 ? 32 * ((b + d) & 1) : 0;
+        const char *p = sm + xa + d * lstep;
+        const int here = h ^ xs1, next = NB == 2 ? here ^ 32 : 0;
+        const u32x2 v0 = lds_tr4(p + here), v1 = lds_tr4(p + here + 4 * VX);
+        const u32x2 v2 = lds_tr4(p + (in ? next : 0) + 8 * VX);
+        u32x4 m = {v0[0], v0[1], v1[0], v1[1]};
+        const u32x4 c = {__builtin_amdgcn_alignbit(v0[1], v0[0], 16), __builtin_amdgcn_alignbit(v1[0], v0[1], 16),
+                         __builtin_amdgcn_alignbit(v1[1], v1[0], 16), __builtin_amdgcn_alignbit(v2[0], v1[1], 16)};
+        const u32x4 n = {v0[1], v1[0], v1[1], v2[0]};
+        if (tails) m &= tm;
+        const bf16x8 fm = __builtin_bit_cast(bf16x8, m), fc = __builtin_bit_cast(bf16x8, c),
+                     fn = __builtin_bit_cast(bf16x8, n);
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+          acc[3 * d][a][b] = mfma16(fa[a], fm, acc[3 * d][a][b]);
+          acc[3 * d + 1][a][b] = mfma16(fa[a], fc, acc[3 * d + 1][a][b]);
+          acc[3 * d + 2][a][b] = mfma16(fa[a], fn, acc[3 * d + 2][a][b]);
+        }
+      }
+    }
+    if (more) put(sm + (buf ^ 1) * buf_bytes);
+    __syncthreads();
+    buf ^= 1;
+  }
+  // the four waves' sums, one dy at a time, added in wave order; partials
+  // fragment by fragment: lane holds (co = co0 + 16 a + 4 kq + r, ci = ci0 +
+  // 16 b + (lane & 15))
+  constexpr int NF = 3 * NA * NB;
+  f32x4 *red = (f32x4 *)sm;
+  f32x4 *dst = (f32x4 *)part + (((long)split * tiles + tile) * 3 + dzi) * (3 * NF * 64);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) red[(wave * NF + (t * NA + a) * NB + b) * 64 + lane] = acc[3 * d + t][a][b];
+    __syncthreads();
+    for (int e = tid; e < NF * 64; e += 256)
+      dst[d * NF * 64 + e] = (red[e] + red[NF * 64 + e]) + (red[2 * NF * 64 + e] + red[3 * NF * 64 + e]);
+    __syncthreads();
+  }
+  if (want_b) {  // every column of the product with ones is the sum
+    if ((lane & 15) == 0)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) red[(wave * NA + a) * 4 + kq] = accb[a];
+    __syncthreads();
+    const float *rf = (const float *)red;
+    if (tid < 16 * NA && co0 + tid < Cout)
+      bpart[(long)split * Cout + co0 + tid] = (rf[tid] + rf[16 * NA + tid]) + (rf[32 * NA + tid] + rf[48 * NA + tid]);
+  }
+}
+
+// dw from the splits' partials (fragment order, see k_conv_wgrad) and db from
+// theirs, in a fixed order.  A block covers 16 fragment quads (256 contiguous
+// bytes per split); its 16 thread groups take every 16th split, four loads
+// in flight at a time, and add up through LDS in group order.  The blocks
+// past the weights' take 16 channels of the bias each.  (19 MB: 5.7 us for both
+// gradients; one thread walking a quarter of the splits with two loads in
+// flight took 23 us for 28 MB, and the bias 34 us in two launches of its own.)
+template <int NA, int NB>
+__global__ void __launch_bounds__(256) k_wgrad_sum(const float *__restrict__ part, const float *__restrict__ bpart,
+                                                   float *__restrict__ dw, float *__restrict__ db, int splits, int Cin,
+                                                   int Cout, int ci_tiles, long n4) {
+  __shared__ f32x4 red[16][17];
+  const int tid = threadIdx.x, el = tid & 15, g = tid >> 4;
+  const long e = (long)blockIdx.x * 16 + el;
+  const bool is_w = e < n4;  // uniform: n4 is a multiple of 16
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  if (is_w) {
+    const f32x4 *p = (const f32x4 *)part + e;
+    int k = g;
+    for (; k + 48 < splits; k += 64) {
+      const f32x4 a = p[k * n4], b = p[(k + 16) * n4], c = p[(k + 32) * n4], d = p[(k + 48) * n4];
+      s += (a + b) + (c + d);
+    }
+    for (; k < splits; k += 16) s += p[k * n4];
+  } else if (e - n4 < Cout) {
+    for (int k = g; k < splits; k += 16) s[0] += bpart[(long)k * Cout + (e - n4)];
+  }
+  red[g][el] = s;
+  __syncthreads();
+  if (g) return;
+  for (int k = 1; k < 16; ++k) s += red[k][el];
+  if (!is_w) {
+    if (e - n4 < Cout) db[e - n4] = s[0];
+    return;
+  }
+  const int lane = (int)(e & 63), f = (int)(e >> 6), b = f % NB, a = f / NB % NA, t = f / (NB * NA) % 27;
+  const int tile = f / (27 * NA * NB);
+  const int ci = (tile % ci_tiles) * 32 + 16 * b + (lane & 15);
+  const int co = (tile / ci_tiles) * 32 + 16 * a + 4 * (lane >> 4);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (co + r < Cout) dw[((long)(co + r) * 27 + t) * Cin + ci] = s[r];
+}
+
+// Units and split of the voxel reduction, from the shape only (so every entry
+// point that shares it gives the same bits), capped so that the partials fit
+// in `cap_bytes`.
+struct WgradPlan {
+  WgGeo q;
+  int ci_tiles, tiles, splits, na, nb;
+  long ups, n4;  // units per split; fragment quads of one split's partials
+  size_t lds, part_bytes;
+};
+
+WgradPlan wgrad_plan(int B, int D, int H, int W, int Cin, int Cout, size_t cap_bytes) {
   WgradPlan p;
+  WgGeo &q = p.q;
+  // whole lines up to 64 voxels (an LDS line of at most 68), else 32-voxel
+  // segments: 64-voxel ones with their two neighbours need a fifth round of
+  // loads for 8 pieces
+  q.halo = W > 64;
+  q.TX = W > 64 ? 32 : (W + 7) / 8 * 8;
+  q.nr = q.TX / 8;
+  q.R = H < kWgRuns / q.nr ? H : kWgRuns / q.nr;
+  q.nseg = (W + q.TX - 1) / q.TX;
+  q.nyb = (H + q.R - 1) / q.R;
+  q.planes = (long)B * D;
+  q.P = 1;
+  if (q.R == H && q.nseg == 1) {  // whole planes: as many as the runs hold
+    const long fit = kWgRuns / (q.nr * q.R);
+    q.P = (int)(fit < q.planes ? fit : q.planes);
+    while (q.P > 1 && q.P * (q.R + 2) * (q.TX + 4) > 360) --q.P;  // two buffers within 64 KB of LDS
+  }
+  q.nlx = q.R == H ? H : q.R + 2;
+  q.l0 = q.R == H ? 1 : 0;
+  q.LP = q.TX + 4;
+  q.nunits = (q.planes + q.P - 1) / q.P * q.nyb * q.nseg;
+  p.na = Cout >= 32 ? 2 : 1;
+  p.nb = Cin >= 32 ? 2 : 1;
+  q.xbytes = q.P * (q.R + 2) * q.LP * 32 * p.nb;
+  q.ybytes = kWgRuns * 8 * 32 * p.na;
+  p.lds = 2 * (size_t)(q.xbytes + q.ybytes) + 12 * 32 * p.nb;
+  const size_t red = (size_t)4 * 3 * p.na * p.nb * 64 * sizeof(f32x4);
+  if (p.lds < red) p.lds = red;
   p.ci_tiles = (Cin + 31) / 32;
-  p.co_tiles = (Cout + 31) / 32;
-  p.nchunks = (M + kWgChunk - 1) / kWgChunk;
-  const int tiles = p.ci_tiles * p.co_tiles;
-  const size_t per_split = (size_t)Cout * 27 * Cin * sizeof(float);
-  long want = (512 + tiles - 1) / tiles;  // about 512 blocks: one round at 2 per CU
-  if (want > p.nchunks) want = p.nchunks;
-  long cap = (long)(cap_bytes / per_split);
+  p.tiles = p.ci_tiles * ((Cout + 31) / 32);
+  p.n4 = (long)p.tiles * 27 * p.na * p.nb * 64;
+  const size_t per_split = (size_t)p.n4 * 16 + (size_t)Cout * 4;
+  // about 512 blocks, one round at 2 per CU
+  long want = 512 / (3 * p.tiles);
+  if (want < 1) want = 1;
+  if (want > q.nunits) want = q.nunits;
+  const long cap = (long)(cap_bytes / per_split);
   if (want > cap) want = cap;
   if (want < 1) want = 1;
-  p.cps = (int)((p.nchunks + want - 1) / want);
-  p.splits = (int)((p.nchunks + p.cps - 1) / p.cps);
+  p.ups = (q.nunits + want - 1) / want;
+  p.splits = (int)((q.nunits + p.ups - 1) / p.ups);
   p.part_bytes = per_split * p.splits;
   return p;
 }
 
-constexpr int kColsumBlocks = 1024;
+template <int NA, int NB>
+int launch_wgrad(const WgradPlan &p, const void *x, const void *dy, float *dw, float *db, int D, int H, int W, int Cin,
+                 int Cout, float *part, hipStream_t s) {
+  float *bpart = db ? part + (size_t)p.n4 * 4 * p.splits : nullptr;
+  const int jobs = p.tiles * 3 * p.splits;
+  auto go = [&](auto kern) {
+    kern<<<(jobs + 7) / 8 * 8, 256, p.lds, s>>>((const uint16_t *)x, (const uint16_t *)dy, part, bpart, p.q, D, H, W, Cin,
+                                                Cout, p.ci_tiles, p.tiles, p.splits, p.ups);
+  };
+  // byte offsets within a unit take 32 bits unless its lines are enormous
+  const long span = (long)p.q.P * p.q.nlx * W * (Cin > Cout ? Cin : Cout) * 2;
+  if (span < (1L << 31)) go(k_conv_wgrad<NA, NB, false>);
+  else go(k_conv_wgrad<NA, NB, true>);
+  HIPCHK(hipGetLastError());
+  const unsigned nb = (unsigned)(p.n4 / 16 + (db ? (Cout + 15) / 16 : 0));
+  k_wgrad_sum<NA, NB><<<nb, 256, 0, s>>>(part, bpart, dw, db, p.splits, Cin, Cout, p.ci_tiles, p.n4);
+  HIPCHK(hipGetLastError());
+  return LBMIB_OK;
+}
 
 int wgrad_with(const void *x, const void *dy, float *dw, float *db, int B, int D, int H, int W, int Cin, int Cout,
                void *ws, size_t ws_bytes, hipStream_t s) {
-  const long M = (long)B * D * H * W;
-  const WgradPlan p = wgrad_plan(M, Cin, Cout, ws_bytes);
-  if (p.part_bytes > ws_bytes || p.nchunks < 1) return LBMIB_ERR_ARG;
+  const WgradPlan p = wgrad_plan(B, D, H, W, Cin, Cout, ws_bytes);
+  if (p.part_bytes > ws_bytes || p.q.nunits < 1) return LBMIB_ERR_ARG;
   float *part = (float *)ws;
-  k_conv_wgrad<<<dim3(p.ci_tiles * p.co_tiles, p.splits), 256, 0, s>>>(
-      (const uint16_t *)x, (const uint16_t *)dy, part, D, H, W, M, Cin, Cout, p.ci_tiles, p.cps, p.nchunks);
-  HIPCHK(hipGetLastError());
-  const long n = (long)Cout * 27 * Cin;
-  k_sum_parts<<<(unsigned)((n + 63) / 64), kSumBlock, 0, s>>>(part, dw, n, p.splits);
-  HIPCHK(hipGetLastError());
-  if (db) {
-    if ((size_t)kColsumBlocks * Cout * sizeof(float) > ws_bytes) return LBMIB_ERR_ARG;
-    const long per = (M + kColsumBlocks - 1) / kColsumBlocks;
-    const int nb = (int)((M + per - 1) / per);
-    k_colsum<<<nb, 256, 0, s>>>((const uint16_t *)dy, part, M, Cout, per);
-    HIPCHK(hipGetLastError());
-    k_sum_parts<<<(unsigned)((Cout + 63) / 64), kSumBlock, 0, s>>>(part, db, Cout, nb);
-    HIPCHK(hipGetLastError());
-  }
-  return LBMIB_OK;
+  if (p.na == 2 && p.nb == 2) return launch_wgrad<2, 2>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
+  if (p.na == 2) return launch_wgrad<2, 1>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
+  if (p.nb == 2) return launch_wgrad<1, 2>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
+  return launch_wgrad<1, 1>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
 }
 
 // The library's workspace: one buffer per device, allocated on first use.
