@@ -214,6 +214,313 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const uint16_t *__restrict__ x
   }
 }
 
+// Forward convolution of few input channels (CI = 16 or 32) on lines of at
+// most 64 voxels.  A block owns 16 WN output channels of 4 G lines (G of them
+// a wave: G W <= 16 WM positions) and marches along z two planes at a time,
+// four of its eight waves on each: the weights of all 27 taps stay in LDS in
+// fragment order, and a ring of four z-planes holds the lines around the
+// block's (the next two planes are loaded into registers while these
+// multiply).  Each input voxel is thus staged once per (4 G + 2) / 4 G lines
+// and the weights once per block, where the box form below fetches 132 KB for
+// every 256 voxels.
+//
+// A line's fragment of 16 voxels is read from LDS once for its three dx: the
+// products with the weights of each dx go to accumulators of their own, acc[dx][u]
+// = sum W[dx] x[u], and out[v] = sum over dx of acc[dx][v + dx] is formed by
+// lane shifts at the end.  A whole line is in one wave, so nothing crosses
+// waves, and beyond a line's ends there is nothing to add.  Per (dz, dy) a
+// wave reads WM + 3 WN fragments for 3 WM WN MFMAs.
+//
+// Reduction slots 8 kq + e (kq = lane >> 4): CI = 32: channel 8 kq + e of one
+// (dz, dy); CI = 16: channel 8 (kq & 1) + e of (dz, dy) number 2 c + (kq >> 1)
+// in chunk c (the tenth is zero).
+//
+// The LDS holds one block, so two waves a SIMD: one's LDS reads and epilogue
+// run beside the other's products (with four waves and one plane at a time
+// they did not: 67 us where this takes 53).  Measured, with the box form's
+// times: 64^3 32 -> 32 at batch 4 53 us, 1089 TFLOP/s (92 us), at batch 1 18
+// us (31); 48^3 32 -> 32 12.5 us (27); 32^3 32 -> 64 at batch 4 16 us (27).
+// Matrix units are busy 43% of the time; the rest is the epilogue and, twice a
+// step, the barriers around the exchange of planes.
+struct MarchGeo {
+  int G, nyb, zc, zs, cot;  // lines per wave; line groups, planes per block, z ranges, channel tiles
+  int plane_bytes;          // of one ring slot
+  long jobs;
+};
+
+// v of another lane of the row of 16, zero where there is none: the next
+// lane's, the previous one's; lane 0's at lane 15 alone, lane 15's at lane 0
+// alone.  Added to a sum, each is one v_add_f32 with a DPP operand.
+template <int CTRL>
+__device__ __forceinline__ float row_shift(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kFromNext = 0x101, kFromPrev = 0x111, kFirstToLast = 0x11f, kLastToFirst = 0x10f;
+
+// BF16 bits of two floats, round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const bf16x2 v = {(__bf16)a, (__bf16)b};
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+template <int WM, int WN, int CI, bool WHOLE>
+__global__ void __launch_bounds__(512, 2)
+    k_conv_march(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
+                 const uint16_t *__restrict__ mask, uint16_t *__restrict__ y, MarchGeo q, int D, int H, int W, int Cout,
+                 int relu) {
+  constexpr int VX = 2 * CI, kChunks = CI == 32 ? 9 : 5, kWFrags = kChunks * 3 * WN;
+  constexpr int kRounds = 3;  // 16-byte pieces of a plane per thread at most (CI = 16: two)
+  constexpr uint32_t kNone = 0x80000000u;
+  extern __shared__ __attribute__((aligned(16))) char sm[];  // weights, then the ring of planes
+  const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4, col = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wl4 = wave & 3;
+  const long per = (q.jobs + 7) / 8;
+  long job = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((long)(blockIdx.x >> 3) >= per || job >= q.jobs) return;
+  const int ct = (int)(job % q.cot);
+  job /= q.cot;
+  const int zi = (int)(job % q.zs);
+  job /= q.zs;
+  const int yb = (int)(job % q.nyb);
+  const long b = job / q.nyb;
+  const int n0 = ct * (16 * WN), y0 = yb * 4 * q.G, z0 = zi * q.zc, z1 = min(z0 + q.zc, D);
+  const int HW = H * W;
+  char *ring = sm + kWFrags * 1024;
+
+  // A plane's lines are contiguous, and those outside it lie outside the
+  // resource, which reads zeros: a plane outside the volume has size zero.
+  auto fetch = [&](int z, u32x4(&px)[kRounds]) {
+    const bool in = z >= 0 && z < D;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(x + (b * D + (in ? z : 0)) * HW * CI), (short)0, in ? HW * VX : 0, 0x00020000);
+    const int first = (y0 - 1) * W * VX + tid * 16;
+#pragma unroll
+    for (int k = 0; k < kRounds * CI / 32 + (CI == 16); ++k)
+      px[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (uint32_t)(first + k * 8192), 0, 0));
+  };
+  auto put = [&](int z, const u32x4(&px)[kRounds]) {  // (a slot is whole waves of pieces)
+    char *d = ring + (z & 3) * q.plane_bytes + tid * 16;
+#pragma unroll
+    for (int k = 0; k < kRounds * CI / 32 + (CI == 16); ++k)
+      if (tid * 16 + k * 8192 < q.plane_bytes) *(u32x4 *)(d + k * 8192) = px[k];
+  };
+  u32x4 pa[kRounds], pb[kRounds];
+  {
+    // all of the first loads in flight together
+    u32x4 pc[kRounds], pd[kRounds];
+    fetch(z0 - 1, pa);
+    fetch(z0, pb);
+    fetch(z0 + 1, pc);
+    fetch(z0 + 2, pd);
+    // weights: fragment (chunk, dx, j), lane (row col, slots 8 kq ..)
+    constexpr int kWRounds = (kWFrags + 7) / 8;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(w), (short)0,
+                                                                      Cout * 27 * VX, 0x00020000);
+    u32x4 pw[kWRounds];
+#pragma unroll
+    for (int k = 0; k < kWRounds; ++k) {
+      const int f = 8 * k + wave, j = f % WN, dx = f / WN % 3, c = f / (3 * WN);
+      const int line = CI == 32 ? c : 2 * c + (kq >> 1), n = n0 + 16 * j + col;
+      const uint32_t o = line < 9 && n < Cout ? (uint32_t)((n * 27 + line * 3 + dx) * VX + (CI == 32 ? kq : kq & 1) * 16)
+                                              : kNone;
+      pw[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0));
+    }
+    put(z0 - 1, pa);
+    put(z0, pb);
+    put(z0 + 1, pc);
+    put(z0 + 2, pd);
+#pragma unroll
+    for (int k = 0; k < kWRounds; ++k)
+      if (8 * k + wave < kWFrags) *(u32x4 *)(sm + (8 * k + wave) * 1024 + lane * 16) = pw[k];
+  }
+  __syncthreads();
+
+  float bs[WN][4];
+#pragma unroll
+  for (int j = 0; j < WN; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = n0 + 16 * j + 4 * kq + r;
+      bs[j][r] = bias && n < Cout ? bias[n] : 0.f;
+    }
+  // this lane's positions: byte offset of channels n0 + 4 kq in the plane of y
+  uint32_t yo[WM];
+  bool nxt[WM], prv[WM];
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    const int pos = 16 * i + col, xx = pos % W, lin = (y0 + wl4 * q.G) * W + pos;
+    yo[i] = pos < q.G * W && lin < HW ? (uint32_t)((lin * Cout + n0 + 4 * kq) * 2) : kNone;
+    nxt[i] = WHOLE ? (16 * i + 16) % W != 0 : xx < W - 1;
+    prv[i] = WHOLE ? 16 * i % W != 0 : xx > 0;
+  }
+  const int bl = (wl4 * q.G * W + col) * VX + (CI == 32 ? kq : kq & 1) * 16;
+  const char *wl = sm + lane * 16;
+  for (int zp = z0; zp < z1; zp += 2) {
+    const bool more = zp + 2 < z1;
+    if (more) {
+      fetch(zp + 3, pa);
+      fetch(zp + 4, pb);
+    }
+    const int z = zp + (wave >> 2);
+    if (z < z1) {
+      const long pl = (b * D + z) * HW * Cout;
+      u32x2 mk[WN][WM];
+      const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(mask + pl), (short)0,
+                                                                         mask ? HW * Cout * 2 : 0, 0x00020000);
+      if (mask)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+          for (int i = 0; i < WM; ++i)
+            mk[j][i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rm, yo[i], j * 32, 0));
+      f32x4 acc[3][WN][WM];
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+          acc[0][j][i] = acc[2][j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+          acc[1][j][i] = f32x4{bs[j][0], bs[j][1], bs[j][2], bs[j][3]};
+        }
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c) {
+        const char *p;
+        if constexpr (CI == 32) {
+          p = ring + ((z - 1 + c / 3) & 3) * q.plane_bytes + (c % 3) * W * VX + bl;
+        } else {
+          const int c1 = min(2 * c + 1, 8);
+          const int o0 = ((z - 1 + 2 * c / 3) & 3) * q.plane_bytes + (2 * c % 3) * W * VX;
+          const int o1 = ((z - 1 + c1 / 3) & 3) * q.plane_bytes + (c1 % 3) * W * VX;
+          p = ring + (kq >> 1 ? o1 : o0) + bl;
+        }
+        bf16x8 bf[WM];
+#pragma unroll
+        for (int i = 0; i < WM; ++i) bf[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(p + i * 16 * VX));
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+          for (int j = 0; j < WN; ++j) {
+            const bf16x8 af = __builtin_bit_cast(bf16x8, *(const u32x4 *)(wl + ((c * 3 + dx) * WN + j) * 1024));
+#pragma unroll
+            for (int i = 0; i < WM; ++i) acc[dx][j][i] = mfma16(af, bf[i], acc[dx][j][i]);
+          }
+      }
+      // a chunk's LDS reads between the products of the one before
+      constexpr int kReads = WM + 3 * WN, kProds = 3 * WM * WN, kPer = kProds / kReads;
+      __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+#pragma unroll
+      for (int c = 1; c < kChunks; ++c) {
+#pragma unroll
+        for (int r = 0; r < kReads; ++r) {
+          __builtin_amdgcn_sched_group_barrier(0x008, kPer, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, kProds - kPer * kReads, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, kProds, 0);
+      const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y + pl, (short)0, HW * Cout * 2, 0x00020000);
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+          float v[4];
+          if constexpr (WHOLE) {  // lines are whole fragments: a fragment's neighbours are its line's or add nothing
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              v[r] = acc[1][j][i][r] + row_shift<kFromNext>(acc[2][j][i][r]) + row_shift<kFromPrev>(acc[0][j][i][r]);
+            if (i + 1 < WM && nxt[i])
+#pragma unroll
+              for (int r = 0; r < 4; ++r) v[r] += row_shift<kFirstToLast>(acc[2][j][i + 1 < WM ? i + 1 : i][r]);
+            if (i > 0 && prv[i])
+#pragma unroll
+              for (int r = 0; r < 4; ++r) v[r] += row_shift<kLastToFirst>(acc[0][j][i > 0 ? i - 1 : 0][r]);
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              float up = row_shift<kFromNext>(acc[2][j][i][r]), dn = row_shift<kFromPrev>(acc[0][j][i][r]);
+              if (i + 1 < WM) up += row_shift<kFirstToLast>(acc[2][j][i + 1 < WM ? i + 1 : i][r]);
+              if (i > 0) dn += row_shift<kLastToFirst>(acc[0][j][i > 0 ? i - 1 : 0][r]);
+              v[r] = acc[1][j][i][r] + (nxt[i] ? up : 0.f) + (prv[i] ? dn : 0.f);
+            }
+          }
+          if (relu)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
+          if (mask) {
+            const uint16_t mb[4] = {(uint16_t)(mk[j][i][0] & 0xffff), (uint16_t)(mk[j][i][0] >> 16),
+                                    (uint16_t)(mk[j][i][1] & 0xffff), (uint16_t)(mk[j][i][1] >> 16)};
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (!(bf2f(mb[r]) > 0.f)) v[r] = 0.f;
+          }
+          const u32x2 o = {pack2(v[0], v[1]), pack2(v[2], v[3])};
+          __builtin_amdgcn_raw_buffer_store_b64(o, ry, n0 + 16 * j < Cout ? yo[i] : kNone, j * 32, 0);
+        }
+    }
+    if (more) {
+      __syncthreads();  // the readers of the two oldest planes are done
+      put(zp + 3, pa);
+      put(zp + 4, pb);
+      __syncthreads();
+    }
+  }
+}
+
+// Where the march applies, and its shape.
+bool march_geo(int B, int D, int H, int W, int Cin, int Cout, int *wm, MarchGeo *q) {
+  if ((Cin != 16 && Cin != 32) || W < 8 || W > 64) return false;
+  const long HW = (long)H * W;
+  if (HW * (Cin > Cout ? Cin : Cout) * 2 >= (1L << 31)) return false;
+  // positions per wave: the multiple of 16 that whole lines fill best
+  const int g4 = 64 / W, g3 = 48 / W;
+  *wm = g3 && g3 * W * 4 > g4 * W * 3 ? 3 : 4;
+  q->G = *wm == 3 ? g3 : g4;
+  q->nyb = (H + 4 * q->G - 1) / (4 * q->G);
+  q->plane_bytes = ((4 * q->G + 2) * W * 2 * Cin + 1023) / 1024 * 1024;
+  q->cot = (Cout + 31) / 32;
+  // z ranges: one block a CU (256), so the rounds of blocks times the plane
+  // pairs each takes (and about two for its weights and first planes) are least
+  const long cols = (long)B * q->nyb * q->cot;
+  long best = -1;
+  for (int zs = 1; zs <= D; ++zs) {
+    const int zc = (D + zs - 1) / zs, used = (D + zc - 1) / zc;
+    const long cost = (cols * used + 255) / 256 * ((zc + 1) / 2 + 2);
+    if (best < 0 || cost < best) {
+      best = cost;
+      q->zc = zc;
+      q->zs = used;
+    }
+  }
+  q->jobs = cols * q->zs;
+  return q->jobs < (1L << 30);
+}
+
+template <int WM, int WN, int CI>
+int launch_march(const MarchGeo &q, const void *x, const void *w, const float *bias, const void *mask, void *y, int D,
+                 int H, int W, int Cout, int relu, hipStream_t s) {
+  const size_t shm = (CI == 32 ? 9 : 5) * 3 * WN * 1024 + 4 * (size_t)q.plane_bytes + 1024;
+  auto go = [&](auto kern) {
+    kern<<<(unsigned)((q.jobs + 7) / 8 * 8), 512, shm, s>>>((const uint16_t *)x, (const uint16_t *)w, bias,
+                                                            (const uint16_t *)mask, (uint16_t *)y, q, D, H, W, Cout,
+                                                            relu);
+  };
+  if (W % 16 == 0) go(k_conv_march<WM, WN, CI, true>);
+  else go(k_conv_march<WM, WN, CI, false>);
+  HIPCHK(hipGetLastError());
+  return LBMIB_OK;
+}
+
+template <int CI>
+int launch_march_any(int wm, const MarchGeo &q, const void *x, const void *w, const float *bias, const void *mask,
+                     void *y, int D, int H, int W, int Cout, int relu, hipStream_t s) {
+  if (Cout >= 32) {
+    if (wm == 4) return launch_march<4, 2, CI>(q, x, w, bias, mask, y, D, H, W, Cout, relu, s);
+    return launch_march<3, 2, CI>(q, x, w, bias, mask, y, D, H, W, Cout, relu, s);
+  }
+  if (wm == 4) return launch_march<4, 1, CI>(q, x, w, bias, mask, y, D, H, W, Cout, relu, s);
+  return launch_march<3, 1, CI>(q, x, w, bias, mask, y, D, H, W, Cout, relu, s);
+}
+
 // Large-grid forward convolution with the input staged in LDS.  A block owns
 // 256 consecutive voxels in linear order -- R = 256 / W whole x-rows of one
 // z-plane of one sample (W divides 256, R divides H, W <= 64) -- and WN x 16
@@ -719,6 +1026,14 @@ int conv_fwd(const void *x, const void *w, const float *bias, const void *mask, 
              int Cin, int Cout, int relu, hipStream_t s) {
   if (!x || !w || !y || !shape_ok(B, D, H, W, Cin, Cout)) return LBMIB_ERR_ARG;
   const long M = (long)B * D * H * W;
+  MarchGeo mg;
+  int wm = 4;
+  // few input channels: the march, from where its ~9 us of first loads and
+  // launch are no more than the small-grid forms take (16^3 at batch 4, 32 ->
+  // 64: 9.2 against 10.6 us; 32 -> 32: 9.0 against 8.5)
+  if ((M >= 24576 || (M >= 16384 && M * Cout >= 1L << 20)) && march_geo(B, D, H, W, Cin, Cout, &wm, &mg))
+    return Cin == 32 ? launch_march_any<32>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s)
+                     : launch_march_any<16>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s);
   // wave tiles: 4 x 16 voxels when the grid is large, fewer when the
   // voxel count alone cannot fill the device; 64 channels per block
   // (32 / 16 for the narrow layers)
