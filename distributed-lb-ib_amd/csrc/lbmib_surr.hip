@@ -521,169 +521,356 @@ int launch_march_any(int wm, const MarchGeo &q, const void *x, const void *w, co
   return launch_march<3, 1, CI>(q, x, w, bias, mask, y, D, H, W, Cout, relu, s);
 }
 
-// Large-grid forward convolution with the input staged in LDS.  A block owns
-// 256 consecutive voxels in linear order -- R = 256 / W whole x-rows of one
-// z-plane of one sample (W divides 256, R divides H, W <= 64) -- and WN x 16
-// output channels; its 4 waves own 64 voxels each (4 fragments of 16).  Per
-// block of 8 input channels it stages in LDS the input box around the tile,
-// (W + 2) x (R + 2) x 3 voxels with zeros outside the volume (16 bytes a
-// voxel), and the weights of its output channels for all 27 taps, so each
-// input voxel is fetched from memory once per block and channel block
-// instead of once per tap, and the 7 chunks of the channel block (four taps
-// x 8 channels each: slot 8 kq + e of chunk p, kq = lane >> 4, is tap
-// 4p + kq, channel c0 + e, in both operands; a 28th tap is zero) read both
-// operands from LDS without a barrier.  The next channel block's box and
-// weights are loaded into registers while the current one multiplies
-// (buffer loads: a piece with nothing to load points past the end of its
-// tensor and reads zeros, so the loads carry no branch and no early wait).
-constexpr int kBoxPieces = 5;  // ceil(box voxels / 256) for W = 16, 32, 64
-constexpr int kWRow = 28 * 8 + 8;  // weight row pitch: 8 rows' 16-byte reads on distinct banks
-__host__ __device__ inline int box_voxels(int W) { return (W + 2) * (256 / W + 2) * 3; }
-inline bool box_conv_ok(int H, int W, long M, int Cin, int Cout) {
-  return W >= 16 && W <= 64 && 256 % W == 0 && H % (256 / W) == 0 && M % 256 == 0 &&
-         M * Cin * 2 < (1L << 31) && (long)Cout * 27 * Cin * 2 < (1L << 30);
-}
+// Forward convolution of 32 or more input channels on lines of at most 64
+// voxels.  A block owns a tile of LP lines x PZ planes (VG groups of G whole
+// lines, 16 WM positions each) and 16 NC output channels.  It stages the box
+// around the tile, (LP + 2) x (PZ + 2) lines with zeros outside the volume,
+// for all input channels at once (or a slice at a time where that exceeds the
+// LDS), and then multiplies without a barrier: its eight waves are NC channel
+// groups x VG voxel groups x KW parts of the reduction.  The reduction goes by
+// items, one (dz, dy) and 32 channels with its three dx: a wave reads the WM
+// input fragments of an item from LDS once for the three dx (as in the march
+// above: an accumulator per dx, joined by lane shifts at the end), and each of
+// its three weight fragments, straight from L2 three items ahead, serves WM
+// products.  The KW partial sums meet in LDS in a fixed order.
+//
+// Neighbouring lanes load pieces of one weight row, four to its 64 bytes, and
+// pass them through 3 KB of LDS of the wave's own into fragment order: loaded
+// in that order, with neighbouring lanes on different rows, every load took
+// four times the cache lookups and they were the bound (120 us where this takes
+// 105, at 24^3, 256 -> 256, batch 2).  LDS voxels are padded by 16 bytes, so
+// that a fragment's 16 lanes read distinct banks.
+//
+// Measured, against the forms it replaced (boxes of 8 channels at a time,
+// reductions split over blocks with partial sums in memory): 16^3, 128 -> 128
+// at batch 4 20.2 us, 716 TFLOP/s (51.7 us), 64 -> 128 at batch 1 8.8 (13.8);
+// 32^3, 64 -> 64 at batch 4 38 (59), at batch 1 14 (27); 8^3, 256 -> 256 at
+// batch 1 8.8 (17.9), at batch 4 14.5 (31.5); 24^3, 256 -> 256 at batch 2 105
+// (230).  The small ones are launch, first loads and the sum over KW; in the
+// large ones the loads of a block's box, which nothing overlaps (one block a
+// CU), and LDS reads beside the products.
+struct TileGeo {
+  int G, LP, PZ, nty, ntz, cot;  // lines per group; tile lines and planes; tiles in y and z; channel tiles
+  int cs, lgp;                   // channels staged at a time; log2 of their 16-byte pieces per voxel
+  int box, lds;                  // LDS bytes of the box, and of all
+  int mW, mLP;                   // 65536 / W + 1, 65536 / LP + 1: quotients of small numbers
+  long jobs;
+};
 
-template <int WN>
-__global__ void __launch_bounds__(256) k_conv_fwd_box(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-                                                      const float *__restrict__ bias,
-                                                      const uint16_t *__restrict__ mask, uint16_t *__restrict__ y,
-                                                      int D, int H, int W, long M, int Cin, int Cout, int relu) {
-  constexpr int WM = 4, kWPieces = (WN * 16 * 28 + 255) / 256;
-  // [box voxel][8 channels], then the weights [WN x 16 rows][kWRow]
-  extern __shared__ __attribute__((aligned(16))) uint16_t xs[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 15, kq = lane >> 4;
-  const long m0 = (long)blockIdx.x * 256;
-  const int n0 = blockIdx.y * (WN * 16);
-  const int R = 256 / W, BX = W + 2, BY = R + 2, NB = BX * BY * 3;
-  const long HW = (long)H * W, plane = m0 / HW;  // the tile's (sample, z) plane
-  const int zt = (int)(plane % D), y0 = (int)((m0 % HW) / W);
-  const int K = 27 * Cin;
-  uint16_t *ws = xs + NB * 8;
-  int vb[WM];  // box index of each fragment's voxel (box coordinates x + 1, row + 1, 1)
+template <int WM, int NC, int KW, int VG, bool WHOLE>
+__global__ void __launch_bounds__(512, 2)
+    k_conv_tile(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
+                const uint16_t *__restrict__ mask, uint16_t *__restrict__ y, TileGeo q, int D, int H, int W, int Cin,
+                int Cout, int relu) {
+  static_assert(NC * KW * VG == 8, "eight waves");
+  constexpr uint32_t kNone = 0x80000000u;
+  extern __shared__ __attribute__((aligned(16))) char sm[];  // the box, then 3 KB of weights per wave
+  const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4, col = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cg = wave % NC, vg = wave / NC % VG, kg = wave / (NC * VG);
+  const long per = (q.jobs + 7) / 8;
+  long job = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((long)(blockIdx.x >> 3) >= per || job >= q.jobs) return;
+  const int ct = (int)(job % q.cot);
+  job /= q.cot;
+  const int ty = (int)(job % q.nty);
+  job /= q.nty;
+  const int tz = (int)(job % q.ntz);
+  const long b = job / q.ntz;
+  const int y0 = ty * q.LP, z0 = tz * q.PZ, n0 = (ct * NC + cg) * 16;
+  const int BL = q.LP + 2, nlines = BL * (q.PZ + 2), pitch = q.cs * 2 + 16;
+  const long S = (long)D * H * W;
+
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(x + b * S * Cin), (short)0,
+                                                                      (int)(S * Cin * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(w), (short)0,
+                                                                      Cout * 27 * Cin * 2, 0x00020000);
+  // items of a slice: (dz, dy) times 32-channel blocks; this wave's are kg, kg
+  // + KW, ..., rounded up to pairs (weights past the end are zero)
+  const int lgc = q.lgp - 2, nitems = 9 << lgc;
+  const int nrounds = ((nitems + KW - 1) / KW + 1) / 2;
+  const uint32_t wb = n0 < Cout ? (uint32_t)((n0 + (lane >> 2)) * 27 * Cin * 2 + (lane & 3) * 16) : kNone;
+  u32x4 wf[2][3];
+  auto load_w = [&](int s, int n, int c0) {
+    const int t = kg + KW * n, row = t >> lgc;
+    const int o = (row * 3 * Cin + c0 + ((t & ((1 << lgc) - 1)) << 5)) * 2;
+    const uint32_t at = t < nitems ? wb : kNone;
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+      wf[s][dx] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, at, o + dx * Cin * 2, 0));
+  };
+  // row r's four pieces lie in an order that spreads 8 or 16 rows' reads over all banks
+  auto turn = [](int r) { return ((r >> 2) + (r & 2)) & 3; };
+  char *wst = sm + q.box + wave * 3072;
+  const int wput = (lane >> 2) * 64 + (((lane & 3) ^ turn(lane >> 2)) << 4), wget = col * 64 + ((kq ^ turn(col)) << 4);
+  bf16x8 wa[2][3];
+  auto swap_w = [&](int s) {  // from the order of the loads into the fragments'
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) *(u32x4 *)(wst + dx * 1024 + wput) = wf[s][dx];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) wa[s][dx] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(wst + dx * 1024 + wget));
+    __builtin_amdgcn_wave_barrier();
+  };
+  // LDS offset of item n's lines and channels relative to the voxel's own
+  auto item_off = [&](int n) {
+    const int t = min(kg + KW * n, nitems - 1), row = t >> lgc;
+    return (row / 3 * BL + row % 3) * W * pitch + ((t & ((1 << lgc) - 1)) << 6);
+  };
+
+  // positions
+  int at[WM];
+  uint32_t yo[WM];
+  bool nxt[WM], prv[WM];
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
-    const int lm = wave * 64 + i * 16 + col;
-    vb[i] = (BY + lm / W + 1) * BX + lm % W + 1;
+    const int pos = 16 * i + col, l = (pos * q.mW) >> 16, xx = pos - l * W, lt = vg * q.G + l;
+    const int pz = (lt * q.mLP) >> 16, ly = lt - pz * q.LP;
+    const bool in = l < q.G && pz < q.PZ, out = in && z0 + pz < D && y0 + ly < H;
+    at[i] = (in ? ((pz * BL + ly) * W + xx) * pitch : 0) + kq * 16;
+    yo[i] = out ? (uint32_t)(((((z0 + pz) * H + y0 + ly) * W + xx) * Cout + n0 + 4 * kq) * 2) : kNone;
+    nxt[i] = WHOLE ? (16 * i + 16) % W != 0 : xx < W - 1;
+    prv[i] = WHOLE ? 16 * i % W != 0 : xx > 0;
   }
-  f32x4 acc[WN][WM];
+  f32x4 acc[3][WM];
 #pragma unroll
-  for (int j = 0; j < WN; ++j)
+  for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-    for (int i = 0; i < WM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(x), (short)0,
-                                                                      (int)(M * Cin * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(w), (short)0,
-                                                                      Cout * K * 2, 0x00020000);
-  constexpr uint32_t kNone = 0x80000000u;  // past the end of both resources: loads zeros
-  // this thread's pieces: byte offsets relative to the channel block (or kNone)
-  uint32_t xo[kBoxPieces], wo[kWPieces];
+    for (int i = 0; i < WM; ++i) acc[dx][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  for (int c0 = 0; c0 < Cin; c0 += q.cs) {
+    load_w(0, 0, c0);
+    load_w(1, 1, c0);
+    if (c0) __syncthreads();  // the readers of the previous slice are done
+    {
+      // lines wave, wave + 8, ... of the box, 64 pieces at a time
+      constexpr int kBatch = 8;
+      const int np = W << q.lgp, rounds = (np + 63) >> 6;
+      int ln = wave, bp = 0, ly = wave, r = 0;
+      while (ly >= BL) ly -= BL, ++bp;
+      while (ln < nlines) {
+        u32x4 px[kBatch];
+        int dst[kBatch];
 #pragma unroll
-  for (int r = 0; r < kBoxPieces; ++r) {
-    const int vi = tid + 256 * r;
-    const int bx = vi % BX, by = (vi / BX) % BY, bz = vi / (BX * BY);
-    const int gx = bx - 1, gy = y0 + by - 1, gz = zt + bz - 1;
-    const bool in = vi < NB && (unsigned)gx < (unsigned)W && (unsigned)gy < (unsigned)H && (unsigned)gz < (unsigned)D;
-    xo[r] = in ? (uint32_t)((((plane - zt + gz) * HW + (long)gy * W + gx) * Cin) * 2) : kNone;
-  }
+        for (int k = 0; k < kBatch; ++k) {
+          const int e = (r << 6) + lane, v = e >> q.lgp, pc = e & ((1 << q.lgp) - 1);
+          const int yy = y0 - 1 + ly, zz = z0 - 1 + bp;
+          const bool have = ln < nlines && e < np;
+          const bool in = have && (unsigned)yy < (unsigned)H && (unsigned)zz < (unsigned)D;
+          const uint32_t src = in ? (uint32_t)((((zz * H + yy) * W + v) * Cin + c0) * 2 + pc * 16) : kNone;
+          px[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, src, 0, 0));
+          dst[k] = have ? (ln * W + v) * pitch + pc * 16 : -1;
+          if (++r == rounds) {
+            r = 0;
+            ln += 8;
+            ly += 8;
+            while (ly >= BL) ly -= BL, ++bp;
+          }
+        }
 #pragma unroll
-  for (int r = 0; r < kWPieces; ++r) {
-    const int e = tid + 256 * r, row = e / 28, tap = e % 28, n = n0 + row;
-    wo[r] = (row < WN * 16 && tap < 27 && n < Cout) ? (uint32_t)((n * K + tap * Cin) * 2) : kNone;
-  }
-  u32x4 px[kBoxPieces], pw[kWPieces];
-  auto fetch = [&](int c0) {  // the channel block's pieces into registers
-    const uint32_t cb = (uint32_t)(c0 * 2);
-#pragma unroll
-    for (int r = 0; r < kBoxPieces; ++r)
-      px[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xo[r] | 0u, cb, 0));
-#pragma unroll
-    for (int r = 0; r < kWPieces; ++r)
-      pw[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo[r], cb, 0));
-  };
-  auto put = [&]() {  // registers into LDS
-#pragma unroll
-    for (int r = 0; r < kBoxPieces; ++r) {
-      const int vi = tid + 256 * r;
-      if (vi < NB) *(u32x4 *)(xs + vi * 8) = px[r];
+        for (int k = 0; k < kBatch; ++k)
+          if (dst[k] >= 0) *(u32x4 *)(sm + dst[k]) = px[k];
+      }
     }
-#pragma unroll
-    for (int r = 0; r < kWPieces; ++r) {
-      const int e = tid + 256 * r;
-      if (e < WN * 16 * 28) *(u32x4 *)(ws + (e / 28) * kWRow + (e % 28) * 8) = pw[r];
-    }
-  };
-  fetch(0);
-  for (int c0 = 0; c0 < Cin; c0 += 8) {
-    __syncthreads();  // the previous channel block's readers are done
-    put();
     __syncthreads();
-    if (c0 + 8 < Cin) fetch(c0 + 8);  // in flight while this block multiplies
-#pragma unroll 2
-    for (int p = 0; p < 7; ++p) {
-      const int tap = 4 * p + kq;
-      bf16x8 b[WM];
-      if (tap < 27) {
-        const int off = ((tap / 9 - 1) * BY + (tap / 3) % 3 - 1) * BX + tap % 3 - 1;
+    bf16x8 bf[WM];
+    {
+      const int o = item_off(0);
 #pragma unroll
-        for (int i = 0; i < WM; ++i) b[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(xs + (vb[i] + off) * 8));
-      } else {
+      for (int i = 0; i < WM; ++i) bf[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(sm + at[i] + o));
+    }
+    swap_w(0);
+    load_w(0, 2, c0);
+    for (int rd = 0; rd < nrounds; ++rd) {
 #pragma unroll
-        for (int i = 0; i < WM; ++i) b[i] = zero8();
-      }
+      for (int s = 0; s < 2; ++s) {
+        const int o = item_off(rd * 2 + s + 1);
+        swap_w(s ^ 1);
+        load_w(s ^ 1, rd * 2 + s + 3, c0);
 #pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        const bf16x8 a = __builtin_bit_cast(bf16x8, *(const u32x4 *)(ws + (j * 16 + col) * kWRow + 32 * p + 8 * kq));
+        for (int i = 0; i < WM; ++i) {
 #pragma unroll
-        for (int i = 0; i < WM; ++i) acc[j][i] = mfma16(a, b[i], acc[j][i]);
+          for (int dx = 0; dx < 3; ++dx) acc[dx][i] = mfma16(wa[s][dx], bf[i], acc[dx][i]);
+          bf[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(sm + at[i] + o));
+        }
+        __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int i = 1; i < WM; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
       }
     }
   }
-  // epilogue: lane holds channels n0 + 16 j + 4 kq + r of voxel m0 + 64 wave + 16 i + col
-  const long mw = m0 + wave * 64;
+
+  // out[v] = sum over dx of acc[dx][v + dx - 1] within v's line
+  f32x4 sum[WM];
 #pragma unroll
-  for (int j = 0; j < WN; ++j) {
-    const int n = n0 + j * 16 + 4 * kq;
-    if (n >= Cout) continue;
-    float bs[4] = {0.f, 0.f, 0.f, 0.f};
-    if (bias)
+  for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bs[r] = bias[n + r];
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      const long m = mw + i * 16 + col;
-      float v[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        v[r] = acc[j][i][r] + bs[r];
-        if (relu) v[r] = fmaxf(v[r], 0.f);
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (WHOLE) {
+        float v = acc[1][i][r] + row_shift<kFromNext>(acc[2][i][r]) + row_shift<kFromPrev>(acc[0][i][r]);
+        if (i + 1 < WM && nxt[i]) v += row_shift<kFirstToLast>(acc[2][i + 1 < WM ? i + 1 : i][r]);
+        if (i > 0 && prv[i]) v += row_shift<kLastToFirst>(acc[0][i > 0 ? i - 1 : 0][r]);
+        sum[i][r] = v;
+      } else {
+        float up = row_shift<kFromNext>(acc[2][i][r]), dn = row_shift<kFromPrev>(acc[0][i][r]);
+        if (i + 1 < WM) up += row_shift<kFirstToLast>(acc[2][i + 1 < WM ? i + 1 : i][r]);
+        if (i > 0) dn += row_shift<kLastToFirst>(acc[0][i > 0 ? i - 1 : 0][r]);
+        sum[i][r] = acc[1][i][r] + (nxt[i] ? up : 0.f) + (prv[i] ? dn : 0.f);
       }
-      if (mask) {
-        const u32x2 mk = *(const u32x2 *)(mask + m * Cout + n);
-        const uint16_t mb[4] = {(uint16_t)(mk[0] & 0xffff), (uint16_t)(mk[0] >> 16), (uint16_t)(mk[1] & 0xffff),
-                                (uint16_t)(mk[1] >> 16)};
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (!(bf2f(mb[r]) > 0.f)) v[r] = 0.f;
-      }
-      u32x2 o;
-      o[0] = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-      o[1] = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-      *(u32x2 *)(y + m * Cout + n) = o;
     }
+  f32x4 *red = (f32x4 *)sm;  // [kg][fragment of the (cg, vg) group][lane]
+  if constexpr (KW > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WM; ++i) red[((kg * NC * VG + wave % (NC * VG)) * WM + i) * 64 + lane] = sum[i];
+    __syncthreads();
+  }
+  if (n0 >= Cout) return;
+  float bs[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bs[r] = bias ? bias[n0 + 4 * kq + r] : 0.f;
+  const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y + b * S * Cout, (short)0, (int)(S * Cout * 2),
+                                                                      0x00020000);
+  const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(mask + b * S * Cout),
+                                                                      (short)0, mask ? (int)(S * Cout * 2) : 0,
+                                                                      0x00020000);
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    if (KW > 1 && i % KW != kg) continue;  // each of the KW waves finishes its share of the fragments
+    u32x2 mk = {0u, 0u};
+    if (mask) mk = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rm, yo[i], 0, 0));
+    f32x4 t = sum[i];
+    if constexpr (KW > 1) {
+      t = red[((wave % (NC * VG)) * WM + i) * 64 + lane];
+#pragma unroll
+      for (int k = 1; k < KW; ++k) t += red[((k * NC * VG + wave % (NC * VG)) * WM + i) * 64 + lane];
+    }
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      v[r] = t[r] + bs[r];
+      if (relu) v[r] = fmaxf(v[r], 0.f);
+    }
+    if (mask) {
+      const uint16_t mb[4] = {(uint16_t)(mk[0] & 0xffff), (uint16_t)(mk[0] >> 16), (uint16_t)(mk[1] & 0xffff),
+                              (uint16_t)(mk[1] >> 16)};
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (!(bf2f(mb[r]) > 0.f)) v[r] = 0.f;
+    }
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])}, ry, yo[i], 0, 0);
   }
 }
 
-template <int WN>
-int launch_fwd_box(const void *x, const void *w, const float *bias, const void *mask, void *y, int D, int H, int W,
-                   long M, int Cin, int Cout, int relu, hipStream_t s) {
-  const dim3 grid((unsigned)(M / 256), (unsigned)((Cout + WN * 16 - 1) / (WN * 16)));
-  const size_t shm = sizeof(uint16_t) * (8 * box_voxels(W) + WN * 16 * kWRow);
-  k_conv_fwd_box<WN><<<grid, 256, shm, s>>>((const uint16_t *)x, (const uint16_t *)w, bias, (const uint16_t *)mask,
-                                            (uint16_t *)y, D, H, W, M, Cin, Cout, relu);
+// Shape of the tile form for 16 WM positions, NC channel groups, KW parts and
+// VG voxel groups; false where it does not apply.
+bool tile_geo(int B, int D, int H, int W, int Cin, int Cout, int wm, int nc, int kw, int vg, TileGeo *q) {
+  if (Cin < 32 || W > 16 * wm || W > 64) return false;
+  const long S = (long)D * H * W;
+  if (S * (Cin > Cout ? Cin : Cout) * 2 >= (1L << 31) || (long)Cout * 27 * Cin * 2 >= (1L << 31)) return false;
+  q->G = 16 * wm / W;
+  const int nl = q->G * vg;
+  // lines x planes: the fewest tiles, then the fewest lines in a tile's box
+  long best = -1;
+  for (int pz = 1; pz <= nl && pz <= D && pz <= 16; ++pz) {
+    const int lp = nl / pz < H ? nl / pz : H;
+    const long tiles = (long)((H + lp - 1) / lp) * ((D + pz - 1) / pz);
+    const long cost = tiles * 100000 + (long)(lp + 2) * (pz + 2);
+    if (best < 0 || cost < best) {
+      best = cost;
+      q->LP = lp;
+      q->PZ = pz;
+    }
+  }
+  q->nty = (H + q->LP - 1) / q->LP;
+  q->ntz = (D + q->PZ - 1) / q->PZ;
+  q->cot = (Cout + 16 * nc - 1) / (16 * nc);
+  q->mW = 65536 / W + 1;
+  q->mLP = 65536 / q->LP + 1;
+  const long vox = (long)(q->LP + 2) * (q->PZ + 2) * W;
+  q->cs = Cin;
+  const long most = 160 * 1024 - 8 * 3072;
+  while (q->cs > 32 && vox * (q->cs * 2 + 16) > most) q->cs /= 2;
+  const long box = vox * (q->cs * 2 + 16), red = kw > 1 ? 8L * wm * 1024 : 0;
+  if (box > most) return false;
+  q->box = (int)box;
+  q->lds = (int)(box + 8 * 3072 > red ? box + 8 * 3072 : red);
+  q->lgp = ilog2(q->cs / 8);
+  q->jobs = (long)B * q->nty * q->ntz * q->cot;
+  return q->jobs < (1L << 30);
+}
+
+template <int WM, int NC, int KW, int VG>
+int launch_tile(const TileGeo &q, const void *x, const void *w, const float *bias, const void *mask, void *y, int D,
+                int H, int W, int Cin, int Cout, int relu, hipStream_t s) {
+  auto go = [&](auto kern) {
+    kern<<<(unsigned)((q.jobs + 7) / 8 * 8), 512, q.lds, s>>>((const uint16_t *)x, (const uint16_t *)w, bias,
+                                                              (const uint16_t *)mask, (uint16_t *)y, q, D, H, W, Cin,
+                                                              Cout, relu);
+  };
+  if (W % 16 == 0) go(k_conv_tile<WM, NC, KW, VG, true>);
+  else go(k_conv_tile<WM, NC, KW, VG, false>);
   HIPCHK(hipGetLastError());
   return LBMIB_OK;
+}
+
+// The shape of least estimated time, in us: a block's first loads and box,
+// which take longer the more of the 256 CUs fetch at once, its items, and the
+// sum over KW.  The constants are a fit to 13 shapes on 70 layers (Cin 64 to
+// 256, and 32 below 4096 voxels; 4 to 64 voxels a side, Cout 16 to 256): 6.6%
+// rms, and the shape it picks takes 2% longer than the fastest on average.
+// The narrowest shape leaves room for two blocks a CU where its box is small.
+struct TileShape {
+  int wm, nc, kw, vg;
+};
+constexpr TileShape kTileShapes[] = {{8, 8, 1, 1}, {8, 4, 1, 2}, {8, 2, 1, 4}, {8, 4, 2, 1}, {8, 2, 4, 1}, {8, 1, 8, 1},
+                                     {4, 4, 2, 1}, {4, 2, 2, 2}, {4, 2, 4, 1}, {4, 1, 8, 1}, {2, 1, 8, 1}};
+
+bool tile_plan(int B, int D, int H, int W, int Cin, int Cout, int *shape, TileGeo *q) {
+  double best = 0;
+  bool any = false;
+  for (int k = 0; k < (int)(sizeof(kTileShapes) / sizeof(kTileShapes[0])); ++k) {
+    const TileShape &c = kTileShapes[k];
+    TileGeo g;
+    if (!tile_geo(B, D, H, W, Cin, Cout, c.wm, c.nc, c.kw, c.vg, &g)) continue;
+    const int per = c.wm == 2 && g.lds <= 80 * 1024 ? 2 : 1;
+    const long rounds = (g.jobs + 256 * per - 1) / (256 * per);
+    const double busy = g.jobs < 256 * per ? (double)g.jobs / (256 * per) : 1.0;
+    const int slices = Cin / g.cs, items = ((9 * g.cs / 32 + c.kw - 1) / c.kw + 1) / 2 * 2 * slices;
+    const double mb = (double)(g.LP + 2) * (g.PZ + 2) * W * (2 * Cin + 16) * 1e-6;
+    const double t = rounds * (2.0 * slices + 10.3 * mb * (0.28 + busy) +
+                               items * (0.073 * c.wm + 0.1) * (per == 2 ? 1.7 : 1.0) + (c.kw > 1 ? 2.1 : 0.0));
+    if (!any || t < best) {
+      any = true;
+      best = t;
+      *shape = k;
+      *q = g;
+    }
+  }
+  return any;
+}
+
+int launch_tile_any(int shape, const TileGeo &q, const void *x, const void *w, const float *bias, const void *mask,
+                    void *y, int D, int H, int W, int Cin, int Cout, int relu, hipStream_t s) {
+  switch (shape) {
+    case 0: return launch_tile<8, 8, 1, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 1: return launch_tile<8, 4, 1, 2>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 2: return launch_tile<8, 2, 1, 4>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 3: return launch_tile<8, 4, 2, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 4: return launch_tile<8, 2, 4, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 5: return launch_tile<8, 1, 8, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 6: return launch_tile<4, 4, 2, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 7: return launch_tile<4, 2, 2, 2>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 8: return launch_tile<4, 2, 4, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case 9: return launch_tile<4, 1, 8, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    default: return launch_tile<2, 1, 8, 1>(q, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+  }
 }
 
 // Small-grid forward convolution: the KW waves of a block all own the same
@@ -823,87 +1010,6 @@ int launch_fwd_kw(const void *x, const void *w, const float *bias, const void *m
   return LBMIB_OK;
 }
 
-// Small samples (8^3, 16^3: the z-planes a block of 256 voxels spans, one
-// more on each side, padded by one cell in x and y, hold at most kVolMax
-// voxels): a block owns up to 256 voxels of one sample (4 waves x 4
-// fragments of 16), 16 output channels, and one slice of 16 input channels
-// of the reduction (gridDim.z slices).  It stages that padded slab of the
-// slice in LDS (zeros outside the volume; rows of 24 elements, so that 8
-// lanes' 16-byte reads fall on distinct banks) and the slice's weights for
-// all 27 taps (rows of 28 x 16 + 8 elements), then multiplies its 14 chunks from LDS with no
-// barrier: slot 8 kq + e of chunk p is tap 2p + (kq >> 1), channel
-// c0 + 8 (kq & 1) + e, in both operands (a 28th tap is zero).  The FP32
-// partial of the slice goes to part[slice][v][n]; k_conv_reduce adds the
-// slices in order with bias, activation and mask.  Each input and weight
-// element is then read once per block, where the split over chunks reads
-// the weights once per 64 voxels and the inputs once per tap.
-constexpr int kVolMax = 1024, kVolPitch = 24, kVolWRow = 28 * 16 + 8;
-
-__global__ void __launch_bounds__(256) k_conv_fwd_vol(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-                                                      float *__restrict__ part, int D, int H, int W, long M, int Cin,
-                                                      int Cout) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t ws[];  // [16 rows][kVolWRow], then [slab voxel][24]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 15, kq = lane >> 4;
-  const int S = D * H * W, parts = (S + 255) / 256;
-  const int smp = blockIdx.x / parts, v0 = (blockIdx.x % parts) * 256;
-  const int n0 = blockIdx.y * 16, c0 = blockIdx.z * 16, K = 27 * Cin;
-  // the z-planes of the block's voxels, and one more on each side
-  const int zlo = v0 / (H * W), zhi = min(v0 + 255, S - 1) / (H * W);
-  const int PX = W + 2, PY = H + 2, NP = PX * PY * (zhi - zlo + 3);
-  uint16_t *xs = ws + 16 * kVolWRow;
-  const long base = (long)smp * S;
-  for (int e = tid; e < 2 * NP; e += 256) {
-    const int vi = e >> 1, half = e & 1;
-    const int gx = vi % PX - 1, gy = (vi / PX) % PY - 1, gz = zlo - 1 + vi / (PX * PY);
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if ((unsigned)gx < (unsigned)W && (unsigned)gy < (unsigned)H && (unsigned)gz < (unsigned)D)
-      v = *(const u32x4 *)(x + (base + ((long)gz * H + gy) * W + gx) * Cin + c0 + 8 * half);
-    *(u32x4 *)(xs + vi * kVolPitch + 8 * half) = v;
-  }
-  for (int e = tid; e < 16 * 56; e += 256) {
-    const int row = e / 56, pc = e % 56, tap = pc >> 1, half = pc & 1, n = n0 + row;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (tap < 27 && n < Cout) v = *(const u32x4 *)(w + (long)n * K + tap * Cin + c0 + 8 * half);
-    *(u32x4 *)(ws + row * kVolWRow + tap * 16 + 8 * half) = v;
-  }
-  __syncthreads();
-  int vb[4], lv[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    lv[i] = v0 + wave * 64 + i * 16 + col;
-    const int l = lv[i] < S ? lv[i] : v0;  // past the end: any voxel of the slab
-    const int vx = l % W, vy = (l / W) % H, vz = l / (W * H);
-    vb[i] = ((vz - zlo + 1) * PY + vy + 1) * PX + vx + 1;
-  }
-  f32x4 acc[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-  for (int p = 0; p < 14; ++p) {
-    const int tap = 2 * p + (kq >> 1);
-    bf16x8 b[4];
-    if (tap < 27) {
-      const int off = ((tap / 9 - 1) * PY + (tap / 3) % 3 - 1) * PX + tap % 3 - 1;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        b[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(xs + (vb[i] + off) * kVolPitch + 8 * (kq & 1)));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) b[i] = zero8();
-    }
-    const bf16x8 a = __builtin_bit_cast(bf16x8, *(const u32x4 *)(ws + col * kVolWRow + 32 * p + 8 * kq));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = mfma16(a, b[i], acc[i]);
-  }
-  // lane holds channels n0 + 4 kq + r of voxel lv[i]
-  float *dst = part + (long)blockIdx.z * M * Cout;
-  const int n = n0 + 4 * kq;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (lv[i] < S && n < Cout) *(f32x4 *)(dst + (base + lv[i]) * Cout + n) = acc[i];
-}
-
 // y[v][n] = act(sum over z < ns of part[z][v][n] + bias[n]) [* (mask > 0)]:
 // one thread per (voxel, 4 channels)
 __global__ void k_conv_reduce(const float *__restrict__ part, int ns, const float *__restrict__ bias,
@@ -969,51 +1075,6 @@ int launch_fwd(const void *x, const void *w, const float *bias, const void *mask
   return LBMIB_OK;
 }
 
-// the largest padded slab over a sample's blocks of 256 voxels
-long vol_slab_voxels(int D, int H, int W) {
-  const long S = (long)D * H * W, HW = (long)H * W;
-  long span = 0;
-  for (long v0 = 0; v0 < S; v0 += 256) {
-    const long v1 = v0 + 255 < S - 1 ? v0 + 255 : S - 1;
-    const long sp = v1 / HW - v0 / HW + 1;
-    if (sp > span) span = sp;
-  }
-  return (long)(W + 2) * (H + 2) * (span + 2);
-}
-
-// Taken where it measured faster than the other small-grid forms: samples
-// of at most 512 voxels, or larger ones with at least 128 input channels
-// (16^3, 128 -> 64: 17.7 against 22.2 us; with 64 input channels the
-// two-wave form is faster: 13.9 against 16.6 us at 64 -> 128), and the
-// slices' partials at most 8 MB (beyond, the reduction's pass over them
-// cost more than the form saves: 16 MB at batch 4 on 8^3, 128 -> 256,
-// 25.5 against 23.6 us split over chunks; 32 MB at 256 -> 256, 49.5 against
-// 32.5 us).
-bool vol_conv_ok(int D, int H, int W, long M, int Cin, int Cout) {
-  const long S = (long)D * H * W;
-  return (S <= 512 || (S <= (1L << 20) && Cin >= 128)) && vol_slab_voxels(D, H, W) <= kVolMax && Cin % 16 == 0 &&
-         (size_t)(Cin / 16) * M * Cout * sizeof(float) <= (8u << 20);
-}
-
-int launch_fwd_vol(const void *x, const void *w, const float *bias, const void *mask, void *y, int D, int H, int W,
-                   long M, int Cin, int Cout, int relu, hipStream_t s) {
-  void *ws = nullptr;
-  const int rc = workspace(&ws);
-  if (rc) return rc;
-  const int S = D * H * W;
-  const dim3 grid((unsigned)(M / S * ((S + 255) / 256)), (unsigned)(Cout / 16), (unsigned)(Cin / 16));
-  const size_t shm = sizeof(uint16_t) * ((size_t)vol_slab_voxels(D, H, W) * kVolPitch + 16 * kVolWRow);
-  k_conv_fwd_vol<<<grid, 256, shm, s>>>((const uint16_t *)x, (const uint16_t *)w, (float *)ws, D, H, W, M, Cin, Cout);
-  HIPCHK(hipGetLastError());
-  const long nq = M * (Cout / 4);
-  long nb = (nq + 255) / 256;
-  if (nb > 4096) nb = 4096;
-  k_conv_reduce<<<(unsigned)nb, 256, 0, s>>>((const float *)ws, (int)grid.z, bias, (const uint16_t *)mask,
-                                              (uint16_t *)y, M, Cout, relu);
-  HIPCHK(hipGetLastError());
-  return LBMIB_OK;
-}
-
 bool shape_ok(int B, int D, int H, int W, int Cin, int Cout) {
   if (B < 1 || D < 1 || H < 1 || W < 1) return false;
   if (Cin < 16 || Cin > 256 || (Cin & (Cin - 1))) return false;
@@ -1034,33 +1095,29 @@ int conv_fwd(const void *x, const void *w, const float *bias, const void *mask, 
   if ((M >= 24576 || (M >= 16384 && M * Cout >= 1L << 20)) && march_geo(B, D, H, W, Cin, Cout, &wm, &mg))
     return Cin == 32 ? launch_march_any<32>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s)
                      : launch_march_any<16>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s);
-  // wave tiles: 4 x 16 voxels when the grid is large, fewer when the
-  // voxel count alone cannot fill the device; 64 channels per block
-  // (32 / 16 for the narrow layers)
+  // more channels, and few-channel grids too small for the forms below (8^3
+  // at batch 4, 32 -> 64: 6.7 us; from 4096 voxels on those are faster, 7.4
+  // against 7.6 us at 16^3)
+  TileGeo tg;
+  int shape = 0;
+  if ((Cin >= 64 || (Cin == 32 && M < 4096)) && tile_plan(B, D, H, W, Cin, Cout, &shape, &tg))
+    return launch_tile_any(shape, tg, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+  // lines longer than 64 voxels, and few channels on small grids.  Wave
+  // tiles: 4 x 16 voxels when the grid is large, fewer when the voxel count
+  // alone cannot fill the device; 64 channels per block (32 / 16 for the
+  // narrow layers)
   const int wn = Cout % 64 == 0 ? 4 : (Cout % 32 == 0 ? 2 : 1);
   const long blocks64 = (M + 255) / 256 * (Cout / (16 * wn));
   if (blocks64 >= 512) {
-    if (box_conv_ok(H, W, M, Cin, Cout)) {  // the input box staged in LDS
-      if (wn == 4) return launch_fwd_box<4>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
-      if (wn == 2) return launch_fwd_box<2>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
-      return launch_fwd_box<1>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
-    }
     if (wn == 4) return launch_fwd<4, 4>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, 1, s);
     if (wn == 2) return launch_fwd<4, 2>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, 1, s);
     return launch_fwd<4, 1>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, 1, s);
   }
-  // mid-size grids with wide inputs: the input box with 16-channel tiles
-  // (32^3 at batch 1, 64 -> 64 channels: 29.1 against 35.4 us split)
-  if (M >= 32768 && Cin >= 64 && box_conv_ok(H, W, M, Cin, Cout))
-    return launch_fwd_box<1>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
-  // tiny grids: the whole padded sample in LDS, the reduction split by input slices
-  if (vol_conv_ok(D, H, W, M, Cin, Cout))
-    return launch_fwd_vol(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
   // small grids whose weights stay modest: the two waves of a block split
   // the reduction of one 32-voxel tile, one launch and no partial sums in
   // memory; the weights are read once per tile, at most 128 MB in all
   const double kw_bytes = (double)((M + 31) / 32) * Cout * 27 * Cin * 2;
-  if (M >= 4096 && kw_bytes <= 128e6 && M * Cin * 2 < (1L << 31)) {
+  if ((M >= 4096 || Cin == 16) && kw_bytes <= 128e6 && M * Cin * 2 < (1L << 31)) {
     if (wn == 4) return launch_fwd_kw<2, 4, 2, 2>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
     if (wn == 2) return launch_fwd_kw<2, 2, 2, 2>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
     return launch_fwd_kw<2, 1, 2, 2>(x, w, bias, mask, y, D, H, W, M, Cin, Cout, relu, s);
