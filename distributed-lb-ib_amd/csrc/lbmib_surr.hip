@@ -1166,24 +1166,53 @@ __global__ void k_flip(const uint16_t *__restrict__ w, uint16_t *__restrict__ wt
 // Three such reads hold the 12 voxels from one before the run on: taps dx =
 // -1 and +1 are registers of them as they are, dx = 0 four v_alignbit.
 //
-// 36 MFMAs per wave and unit against 22 LDS reads; the next unit's loads are
-// in flight meanwhile and go into the other LDS buffer (one barrier per
-// unit), and what bounds it is their latency.  Measured, this kernel against
-// the form that gathered its operands with 2-byte LDS reads: 154 against 539
-// us at batch 4 x 64^3, 32 -> 32 channels (376 TFLOP/s), 43 against 150 us at
-// batch 4 x 16^3, 128 -> 128.
+// 36 MFMAs per wave and unit against 22 LDS reads, each group of 6 products
+// behind the next group's 3 reads.  The units come by direct loads from memory
+// to LDS, two ahead of the one that multiplies, with no register and no store
+// on the way (through registers only one unit ahead fitted, with 36 bytes of
+// spills).  Alone, the loads take 67 us and the products 70 at batch 4 x 64^3,
+// 32 -> 32 channels: each dz fetches its own x and dy, 600 MB from L2.
+//
+// Measured, against the form with one unit ahead through registers: 98 us
+// (593 TFLOP/s) for 139 at batch 4 x 64^3, 32 -> 32; 53 for 74 at 32^3, 64 ->
+// 64; 38 for 46 at 16^3, 128 -> 128; 203 for 275 at batch 2 x 24^3, 256 -> 256.
 constexpr int kWgRuns = 16;
-constexpr int kWgXP = 4, kWgYP = 2;  // 16-byte pieces per thread of a unit's x and dy at most
+constexpr int kWgBufs = 3;      // units in LDS: one multiplies, two arrive
+constexpr int kWgMaxVox = 288;  // LDS voxels of a unit's x: three units and two blocks a CU in 160 KB
 
 struct WgGeo {
   int TX, nr, R, P;  // voxels of a line segment, its runs of 8, lines per plane, planes
   int halo;          // 1: segments of a longer line, loaded with their x neighbours
-  int nlx, l0;       // x lines loaded per plane, and the LDS line of the first: R + 2, 0, or R, 1 where R = H
   int LP;            // LDS voxels per line: index i is x = xs + i - 1
   int nseg, nyb;     // segments per line, line groups per plane
-  long planes, nunits;
-  int xbytes, ybytes;  // of one LDS buffer
+  int npg, nunits;     // plane groups, units
+  long planes;
+  int xbytes, ybytes;  // of one LDS buffer, multiples of 1024
 };
+
+// 16 bytes per lane from r + off to LDS at + 16 lane, without registers in
+// between; zeros where off lies past the resource.  Nothing waits: dma_wait.
+// (The builtin makes the compiler wait for every such load before the next LDS
+// read, whichever buffer it reads.  The compiler keeps nothing in m0.)
+__device__ __forceinline__ void dma16(u32x4 r, uint32_t off, uint32_t at) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %2, 0 offen lds"
+      :
+      : "s"(at), "v"(off), "s"(r)
+      : "memory");
+}
+// all but the last N loads have arrived, and this wave's LDS reads are done
+template <int N>
+__device__ __forceinline__ void dma_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
+}
+__device__ __forceinline__ u32x4 rsrc_words(const void *p) {
+  const uint64_t a = (uint64_t)p;
+  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)((a >> 32) & 0xffff)), 0x7fffffffu, 0x00020000u};
+}
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -1199,11 +1228,14 @@ template <int NA, int NB, bool BIG>
 __global__ void __launch_bounds__(256, 2)
     k_conv_wgrad(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part,
                  float *__restrict__ bpart, WgGeo q, int D, int H, int W, int Cin, int Cout, int ci_tiles, int tiles,
-                 int splits, long units_per_split) {
+                 int splits, int units_per_split) {
   constexpr int VX = 32 * NB, VY = 32 * NA;  // bytes per voxel in LDS
   constexpr uint32_t kNone = 0x80000000u;    // past the end of the resources: loads zeros
-  extern __shared__ __attribute__((aligned(16))) char sm[];  // two buffers of x and dy, then 12 voxels of zeros
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kq = lane >> 4;
+  constexpr int KX = (kWgMaxVox * VX / 1024 + 3) / 4, KY = kWgRuns * 8 * VY / 4096;  // DMA instructions per wave and unit
+  // three buffers of x and dy, 12 voxels of zeros, 1 KB that nothing reads
+  extern __shared__ __attribute__((aligned(1024))) char sm[];
+  const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Workgroup b runs on XCD b % 8: the three dz of a split and tile, which
   // read the same dy and neighbouring planes of x, follow each other there.
   const int jobs = tiles * 3 * splits, per = (jobs + 7) / 8;
@@ -1211,36 +1243,34 @@ __global__ void __launch_bounds__(256, 2)
   if ((int)(blockIdx.x >> 3) >= per || job >= jobs) return;
   const int dzi = job % 3, tile = (job / 3) % tiles, split = job / (3 * tiles);
   const int ci0 = (tile % ci_tiles) * 32, co0 = (tile / ci_tiles) * 32;
-  const int buf_bytes = q.xbytes + q.ybytes;
+  const int buf_bytes = q.xbytes + q.ybytes, zeros_at = kWgBufs * buf_bytes;
+  const uint32_t unread_at = (uint32_t)(zeros_at + 12 * VX + 1023) / 1024 * 1024;
 
-  // this thread's pieces: where they lie in memory relative to the unit, and
-  // (in one register each) line, plane and x within it, which decide whether
-  // they exist, and the LDS piece they go to
-  uint32_t xo[kWgXP], yo[kWgYP], xl[kWgXP], yl[kWgYP];
+  // Instruction k of a wave fills the 1024 bytes number wave + 4 k of a
+  // buffer's x (and of its dy): this lane's piece of it, where it lies in
+  // memory relative to the unit, and (in one register) line, plane and x,
+  // which decide whether it exists
+  uint32_t xo[KX], yo[KY], xl[KX], yl[KY];
   constexpr uint32_t kNoPiece = 0x80000000u;
-  auto pack = [](int l, int p, int ix, int at) { return (uint32_t)(l | p << 5 | ix << 10 | (at >> 4) << 17); };
+  auto pack = [](int l, int p, int ix) { return (uint32_t)(l | p << 5 | ix << 10); };
   auto line_of = [](uint32_t v) { return (int)(v & 31); };
   auto plane_of = [](uint32_t v) { return (int)(v >> 5 & 31); };
   auto x_of = [](uint32_t v) { return (int)(v >> 10 & 127); };
-  auto at_of = [](uint32_t v) { return (int)(v >> 17 << 4); };
-  const int SX = min(W, q.TX) + 2 * q.halo, TXs = min(W, q.TX);
 #pragma unroll
-  for (int r = 0; r < kWgXP; ++r) {
-    const int e = tid + 256 * r, pc = e & (2 * NB - 1), v = e / (2 * NB);
-    const int ix = v % SX, ln = v / SX, l = ln % q.nlx, p = ln / q.nlx;
-    const int L = p * (q.R + 2) + l + q.l0, i = ix + 1 - q.halo;
-    const int s = NB == 2 ? ((i >> 3) + L) & 1 : 0;
-    xo[r] = (uint32_t)((((long)p * H + l) * W + ix) * Cin * 2 + pc * 16);
-    xl[r] = p < q.P ? pack(l, p, ix, (L * q.LP + i) * VX + (((pc >> 1) ^ s) * 32) + (pc & 1) * 16) : kNoPiece;
+  for (int k = 0; k < KX; ++k) {
+    const int e = (wave + 4 * k) * 64 + lane, pc = e & (2 * NB - 1), v = e / (2 * NB);
+    const int i = v % q.LP, L = v / q.LP, l = L % (q.R + 2), p = L / (q.R + 2);
+    const int h = NB == 2 ? (pc >> 1) ^ (((i >> 3) + L) & 1) : 0;
+    xo[k] = (uint32_t)((((long)p * H + l) * W + i) * Cin * 2 + h * 32 + (pc & 1) * 16);
+    xl[k] = p < q.P ? pack(l, p, i) : kNoPiece;
   }
 #pragma unroll
-  for (int r = 0; r < kWgYP; ++r) {
-    const int e = tid + 256 * r, pc = e & (2 * NA - 1), v = e / (2 * NA);
-    const int ix = v % TXs, ln = v / TXs, l = ln % q.R, p = ln / q.R;
-    const int run = (p * q.R + l) * q.nr + (ix >> 3);
-    yo[r] = co0 + pc * 8 < Cout ? (uint32_t)((((long)p * H + l) * W + ix) * Cout * 2 + pc * 16) : kNone;
-    const int h = NA == 2 ? (pc >> 1) ^ (run & 1) : 0;
-    yl[r] = p < q.P ? pack(l, p, ix, q.xbytes + (run * 8 + (ix & 7)) * VY + h * 32 + (pc & 1) * 16) : kNoPiece;
+  for (int k = 0; k < KY; ++k) {
+    const int e = (wave + 4 * k) * 64 + lane, pc = e & (2 * NA - 1), v = e / (2 * NA);
+    const int run = v >> 3, ix = (run % q.nr) * 8 + (v & 7), l = (run / q.nr) % q.R, p = run / (q.nr * q.R);
+    const int h = NA == 2 ? (pc >> 1) ^ (run & 1) : 0, ch = h * 16 + (pc & 1) * 8;
+    yo[k] = (uint32_t)((((long)p * H + l) * W + ix) * Cout * 2 + ch * 2);
+    yl[k] = p < q.P && co0 + ch < Cout ? pack(l, p, ix) : kNoPiece;
   }
   // this lane's run: LDS addresses of its x (line dy = -1) and dy operands
   const int run = 4 * wave + kq, rx = run % q.nr, rl = (run / q.nr) % q.R, rp = run / (q.nr * q.R);
@@ -1249,74 +1279,77 @@ __global__ void __launch_bounds__(256, 2)
   const int L0 = rp * (q.R + 2) + rl;
   const int xa0 = (L0 * q.LP + 8 * rx + rowb) * VX + colb, xs0 = NB == 2 ? ((rx + L0) & 1) * 32 : 0;
   const int ya0 = q.xbytes + (run * 8 + rowb) * VY + colb, ys0 = NA == 2 ? (run & 1) * 32 : 0;
-  const int zero_at = 2 * buf_bytes + rowb * VX + colb;
+  const int zero_at = zeros_at + rowb * VX + colb;
   const bool tails = q.halo || (W & 7);  // lines whose last run is not full
 
-  // the unit sequence: plane group, line group, segment
-  long u = (long)split * units_per_split;
-  const long u_end = min(u + units_per_split, q.nunits);
-  int sg = (int)(u % q.nseg), yb = (int)(u / q.nseg % q.nyb);
-  long pg = u / q.nseg / q.nyb;
-  int z0 = (int)(pg * q.P % D);  // the first plane's z
-  auto step = [&]() {
-    ++u;
-    if (++sg == q.nseg) {
-      sg = 0;
-      if (++yb == q.nyb) {
-        yb = 0;
-        ++pg;
-        for (z0 += q.P; z0 >= D;) z0 -= D;
+  // The unit sequence: plane groups first, so that a plane of x that one dz
+  // reads is still in L2 when the next two do; then line groups, segments.  (A
+  // single plane whose z + dz lies outside the volume adds nothing and is
+  // passed by.)
+  const int u_begin = split * units_per_split, u_end = min(u_begin + units_per_split, q.nunits);
+  struct Unit {
+    int u, pg, sg, yb, z0;  // z0: the first plane's z
+  };
+  auto step = [&](Unit &t) {
+    ++t.u;
+    t.z0 += q.P;
+    if (++t.pg == q.npg) {
+      t.pg = t.z0 = 0;
+      if (++t.yb == q.nyb) {
+        t.yb = 0;
+        ++t.sg;
       }
     }
+    while (t.z0 >= D) t.z0 -= D;
   };
-  // (a single plane whose z + dz lies outside the volume adds nothing)
-  auto skip = [&]() {
-    while (u < u_end && q.P == 1 && (unsigned)(z0 + dzi - 1) >= (unsigned)D) step();
+  auto skip = [&](Unit &t) {
+    if (q.P == 1)
+      while (t.u < u_end && (unsigned)(t.z0 + dzi - 1) >= (unsigned)D) step(t);
   };
-  u32x4 px[kWgXP], py[kWgYP];
-  auto fetch = [&]() {
-    const long pl = pg * q.P;
-    const int y0 = yb * q.R, xs = sg * q.TX, yx = y0 - (1 - q.l0);
-    const uint16_t *bx = x + (((pl + dzi - 1) * H + yx) * W + xs - q.halo) * Cin + ci0;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)sm;
+  auto issue = [&](const Unit &t, int buf) {
+    const long pl = (long)t.pg * q.P;
+    // the planes that exist at z + dz, by their number in the unit
+    uint32_t zin = 1, yin = 1;
+    if (q.P > 1) {
+      zin = yin = 0;
+      for (int p = 0, z = t.z0; p < q.P && pl + p < q.planes; ++p) {
+        yin |= 1u << p;
+        if ((unsigned)(z + dzi - 1) < (unsigned)D) zin |= 1u << p;
+        if (++z == D) z = 0;
+      }
+    }
+    const int y0 = t.yb * q.R, xs = t.sg * q.TX;
+    const uint16_t *bx = x + (((pl + dzi - 1) * H + y0 - 1) * W + xs - 1) * Cin + ci0;
     const uint16_t *by = dy + ((pl * H + y0) * W + xs) * Cout + co0;
-    const __amdgpu_buffer_rsrc_t rx_ = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(bx), (short)0, 0x7fffffff,
-                                                                        0x00020000);
-    const __amdgpu_buffer_rsrc_t ry_ = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(by), (short)0, 0x7fffffff,
-                                                                        0x00020000);
+    const u32x4 rx_ = rsrc_words(bx), ry_ = rsrc_words(by);
+    const uint32_t at0 = lds0 + buf * buf_bytes;
 #pragma unroll
-    for (int r = 0; r < kWgXP; ++r) {
-      const int l = line_of(xl[r]), p = plane_of(xl[r]), ix = x_of(xl[r]);
-      bool ok = xl[r] != kNoPiece && (unsigned)(yx + l) < (unsigned)H && (unsigned)(xs + ix - q.halo) < (unsigned)W;
-      if (q.P > 1) ok = ok && pl + p < q.planes && (unsigned)((z0 + p) % D + dzi - 1) < (unsigned)D;
+    for (int k = 0; k < KX; ++k) {
+      const int l = line_of(xl[k]), p = plane_of(xl[k]), ix = x_of(xl[k]), at = (wave + 4 * k) * 1024;
+      const bool ok = (xl[k] != kNoPiece) & ((unsigned)(y0 - 1 + l) < (unsigned)H) &
+                      ((unsigned)(xs - 1 + ix) < (unsigned)W) & (bool)(zin >> p & 1);
       if constexpr (BIG) {
-        const int pc = (tid + 256 * r) & (2 * NB - 1);
-        const uint16_t *src = ok ? bx + (((long)p * H + l) * W + ix) * Cin + pc * 8 : x;
-        px[r] = ok ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
+        const int pc = lane & (2 * NB - 1), h = NB == 2 ? (xo[k] >> 5) & 1 : 0;
+        const uint16_t *src = ok ? bx + (((long)p * H + l) * W + ix) * Cin + h * 16 + (pc & 1) * 8 : x;
+        const u32x4 v = ok ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
+        if (at < q.xbytes) *(u32x4 *)(sm + buf * buf_bytes + at + lane * 16) = v;
       } else {
-        px[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx_, ok ? xo[r] : kNone, 0, 0));
+        dma16(rx_, ok ? xo[k] : kNone, at < q.xbytes ? at0 + at : lds0 + unread_at);
       }
     }
 #pragma unroll
-    for (int r = 0; r < kWgYP; ++r) {
-      const int l = line_of(yl[r]), p = plane_of(yl[r]), ix = x_of(yl[r]);
-      const bool ok = yl[r] != kNoPiece && y0 + l < H && xs + ix < W && pl + p < q.planes;
+    for (int k = 0; k < KY; ++k) {
+      const int l = line_of(yl[k]), p = plane_of(yl[k]), ix = x_of(yl[k]), at = q.xbytes + (wave + 4 * k) * 1024;
+      const bool ok = (yl[k] != kNoPiece) & (y0 + l < H) & (xs + ix < W) & (bool)(yin >> p & 1);
       if constexpr (BIG) {
-        const int pc = (tid + 256 * r) & (2 * NA - 1);
-        const bool in = ok && yo[r] != kNone;
-        const uint16_t *src = in ? by + (((long)p * H + l) * W + ix) * Cout + pc * 8 : dy;
-        py[r] = in ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
+        const int pc = lane & (2 * NA - 1), h = NA == 2 ? (yo[k] >> 5) & 1 : 0;
+        const uint16_t *src = ok ? by + (((long)p * H + l) * W + ix) * Cout + h * 16 + (pc & 1) * 8 : dy;
+        *(u32x4 *)(sm + buf * buf_bytes + at + lane * 16) = ok ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
       } else {
-        py[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ry_, ok ? yo[r] : kNone, 0, 0));
+        dma16(ry_, ok ? yo[k] : kNone, at0 + at);
       }
     }
-  };
-  auto put = [&](char *b) {
-#pragma unroll
-    for (int r = 0; r < kWgXP; ++r)
-      if (xl[r] != kNoPiece) *(u32x4 *)(b + at_of(xl[r])) = px[r];
-#pragma unroll
-    for (int r = 0; r < kWgYP; ++r)
-      if (yl[r] != kNoPiece) *(u32x4 *)(b + at_of(yl[r])) = py[r];
   };
 
   f32x4 acc[9][NA][NB], accb[NA];
@@ -1331,31 +1364,44 @@ __global__ void __launch_bounds__(256, 2)
   const bool want_b = bpart && dzi == 1 && ci0 == 0;  // this block also sums dy over the voxels
   const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
 
-  // what no piece fills stays zero: the neighbours outside a line, lines
-  // outside the plane, slots past the unit's runs
-  for (int k = tid * 16; k < 2 * buf_bytes + 12 * VX; k += 256 * 16) *(u32x4 *)(sm + k) = u32x4{0u, 0u, 0u, 0u};
-  skip();
-  if (u < u_end) fetch();
-  __syncthreads();
-  if (u < u_end) put(sm);
-  __syncthreads();
-  int buf = 0;
-  while (u < u_end) {
+  if (tid * 16 < 12 * VX) *(u32x4 *)(sm + zeros_at + tid * 16) = u32x4{0u, 0u, 0u, 0u};
+  Unit cur = {u_begin, u_begin % q.npg, u_begin / q.npg / q.nyb, u_begin / q.npg % q.nyb, 0};
+  cur.z0 = (int)((long)cur.pg * q.P % D);
+  skip(cur);
+  Unit ahead = cur;  // the next unit to fetch
+  int left = 0, buf = 0;
+  for (; left < kWgBufs - 1 && ahead.u < u_end; ++left) {
+    issue(ahead, left);
+    step(ahead);
+    skip(ahead);
+  }
+  while (left > 0) {
+    // this unit's pieces are here (those of the one after may be on their
+    // way), and every wave is done with the buffer that is filled next
+    if (left > 1) dma_wait<KX + KY>();
+    else dma_wait<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    --left;
+    if (ahead.u < u_end) {
+      issue(ahead, buf == 0 ? kWgBufs - 1 : buf - 1);
+      step(ahead);
+      skip(ahead);
+      ++left;
+    }
     // the lanes whose run lies past the unit or the plane multiply zeros by zeros
-    const bool in = has_run && yb * q.R + rl < H;
+    const bool in = has_run && cur.yb * q.R + rl < H;
     const int boff = buf * buf_bytes;
     const int xa = in ? boff + xa0 : zero_at, lstep = in ? q.LP * VX : 0, xs1 = in ? xs0 : 0;
     u32x4 tm = {~0u, ~0u, ~0u, ~0u};  // clears x[last voxel] where dx = -1 pairs it with a voxel past the line
     if (tails) {
-      const int e0 = W - sg * q.TX - 8 * rx;
+      const int e0 = W - cur.sg * q.TX - 8 * rx;
 #pragma unroll
       for (int k = 0; k < 8; ++k)
         if (e0 == k) tm[k >> 1] = k & 1 ? 0x0000ffffu : 0xffff0000u;
     }
-    step();
-    skip();
-    const bool more = u < u_end;
-    if (more) fetch();
+    step(cur);
+    skip(cur);
     bf16x8 fa[NA];
 #pragma unroll
     for (int a = 0; a < NA; ++a) {
@@ -1363,39 +1409,52 @@ __global__ void __launch_bounds__(256, 2)
       const u32x2 lo = lds_tr4(p), hi = lds_tr4(p + 4 * VY);
       fa[a] = __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
     }
+    // groups of 3 reads and 3 NA products, a group's reads before the products
+    // of the one before
+    u32x2 v[2][3];
+    auto read = [&](int g) {
+      // (the half of a voxel's channels alternates with the 8-voxel block and
+      // the line, so that two runs' reads fall on distinct banks)
+      const int d = g / NB, h = NB == 2 ? 32 * ((g % NB + d) & 1) : 0;
+      const char *p = sm + xa + d * lstep;
+      const int here = h ^ xs1, next = NB == 2 ? here ^ 32 : 0;
+      v[g & 1][0] = lds_tr4(p + here);
+      v[g & 1][1] = lds_tr4(p + here + 4 * VX);
+      v[g & 1][2] = lds_tr4(p + (in ? next : 0) + 8 * VX);
+    };
+    read(0);
+#pragma unroll
+    for (int g = 0; g < 3 * NB; ++g) {
+      if (g + 1 < 3 * NB) read(g + 1);
+      const int d = g / NB, b = g % NB;
+      const u32x2 v0 = v[g & 1][0], v1 = v[g & 1][1], v2 = v[g & 1][2];
+      u32x4 m = {v0[0], v0[1], v1[0], v1[1]};
+      const u32x4 c = {__builtin_amdgcn_alignbit(v0[1], v0[0], 16), __builtin_amdgcn_alignbit(v1[0], v0[1], 16),
+                       __builtin_amdgcn_alignbit(v1[1], v1[0], 16), __builtin_amdgcn_alignbit(v2[0], v1[1], 16)};
+      const u32x4 n = {v0[1], v1[0], v1[1], v2[0]};
+      if (tails) m &= tm;
+      const bf16x8 fm = __builtin_bit_cast(bf16x8, m), fc = __builtin_bit_cast(bf16x8, c),
+                   fn = __builtin_bit_cast(bf16x8, n);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        acc[3 * d][a][b] = mfma16(fa[a], fm, acc[3 * d][a][b]);
+        acc[3 * d + 1][a][b] = mfma16(fa[a], fc, acc[3 * d + 1][a][b]);
+        acc[3 * d + 2][a][b] = mfma16(fa[a], fn, acc[3 * d + 2][a][b]);
+      }
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * NA + 6, 0);
+#pragma unroll
+    for (int g = 0; g + 2 < 3 * NB; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 3 * NA, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 6 * NA, 0);
     if (want_b)
 #pragma unroll
       for (int a = 0; a < NA; ++a) accb[a] = mfma16(fa[a], ones, accb[a]);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        // (the half of a voxel's channels alternates with the 8-voxel block
-        // and the line, so that two runs' reads fall on distinct banks)
-        const int h = NB == 2 ? 32 * ((b + d) & 1) : 0;
-        const char *p = sm + xa + d * lstep;
-        const int here = h ^ xs1, next = NB == 2 ? here ^ 32 : 0;
-        const u32x2 v0 = lds_tr4(p + here), v1 = lds_tr4(p + here + 4 * VX);
-        const u32x2 v2 = lds_tr4(p + (in ? next : 0) + 8 * VX);
-        u32x4 m = {v0[0], v0[1], v1[0], v1[1]};
-        const u32x4 c = {__builtin_amdgcn_alignbit(v0[1], v0[0], 16), __builtin_amdgcn_alignbit(v1[0], v0[1], 16),
-                         __builtin_amdgcn_alignbit(v1[1], v1[0], 16), __builtin_amdgcn_alignbit(v2[0], v1[1], 16)};
-        const u32x4 n = {v0[1], v1[0], v1[1], v2[0]};
-        if (tails) m &= tm;
-        const bf16x8 fm = __builtin_bit_cast(bf16x8, m), fc = __builtin_bit_cast(bf16x8, c),
-                     fn = __builtin_bit_cast(bf16x8, n);
-#pragma unroll
-        for (int a = 0; a < NA; ++a) {
-          acc[3 * d][a][b] = mfma16(fa[a], fm, acc[3 * d][a][b]);
-          acc[3 * d + 1][a][b] = mfma16(fa[a], fc, acc[3 * d + 1][a][b]);
-          acc[3 * d + 2][a][b] = mfma16(fa[a], fn, acc[3 * d + 2][a][b]);
-        }
-      }
-    }
-    if (more) put(sm + (buf ^ 1) * buf_bytes);
-    __syncthreads();
-    buf ^= 1;
+    buf = buf == kWgBufs - 1 ? 0 : buf + 1;
   }
+  __syncthreads();
   // the four waves' sums, one dy at a time, added in wave order; partials
   // fragment by fragment: lane holds (co = co0 + 16 a + 4 kq + r, ci = ci0 +
   // 16 b + (lane & 15))
@@ -1475,8 +1534,8 @@ __global__ void __launch_bounds__(256) k_wgrad_sum(const float *__restrict__ par
 // in `cap_bytes`.
 struct WgradPlan {
   WgGeo q;
-  int ci_tiles, tiles, splits, na, nb;
-  long ups, n4;  // units per split; fragment quads of one split's partials
+  int ci_tiles, tiles, splits, na, nb, ups;  // ups: units per split
+  long n4;  // fragment quads of one split's partials
   size_t lds, part_bytes;
 };
 
@@ -1497,17 +1556,16 @@ WgradPlan wgrad_plan(int B, int D, int H, int W, int Cin, int Cout, size_t cap_b
   if (q.R == H && q.nseg == 1) {  // whole planes: as many as the runs hold
     const long fit = kWgRuns / (q.nr * q.R);
     q.P = (int)(fit < q.planes ? fit : q.planes);
-    while (q.P > 1 && q.P * (q.R + 2) * (q.TX + 4) > 360) --q.P;  // two buffers within 64 KB of LDS
+    while (q.P > 1 && q.P * (q.R + 2) * (q.TX + 4) > kWgMaxVox) --q.P;
   }
-  q.nlx = q.R == H ? H : q.R + 2;
-  q.l0 = q.R == H ? 1 : 0;
   q.LP = q.TX + 4;
-  q.nunits = (q.planes + q.P - 1) / q.P * q.nyb * q.nseg;
+  q.npg = (int)((q.planes + q.P - 1) / q.P);
+  q.nunits = q.npg * q.nyb * q.nseg;
   p.na = Cout >= 32 ? 2 : 1;
   p.nb = Cin >= 32 ? 2 : 1;
-  q.xbytes = q.P * (q.R + 2) * q.LP * 32 * p.nb;
+  q.xbytes = (q.P * (q.R + 2) * q.LP * 32 * p.nb + 1023) / 1024 * 1024;
   q.ybytes = kWgRuns * 8 * 32 * p.na;
-  p.lds = 2 * (size_t)(q.xbytes + q.ybytes) + 12 * 32 * p.nb;
+  p.lds = ((size_t)kWgBufs * (q.xbytes + q.ybytes) + 12 * 32 * p.nb + 1023) / 1024 * 1024 + 1024;
   const size_t red = (size_t)4 * 3 * p.na * p.nb * 64 * sizeof(f32x4);
   if (p.lds < red) p.lds = red;
   p.ci_tiles = (Cin + 31) / 32;
@@ -1521,8 +1579,8 @@ WgradPlan wgrad_plan(int B, int D, int H, int W, int Cin, int Cout, size_t cap_b
   const long cap = (long)(cap_bytes / per_split);
   if (want > cap) want = cap;
   if (want < 1) want = 1;
-  p.ups = (q.nunits + want - 1) / want;
-  p.splits = (int)((q.nunits + p.ups - 1) / p.ups);
+  p.ups = (int)((q.nunits + want - 1) / want);
+  p.splits = (q.nunits + p.ups - 1) / p.ups;
   p.part_bytes = per_split * p.splits;
   return p;
 }
@@ -1537,7 +1595,7 @@ int launch_wgrad(const WgradPlan &p, const void *x, const void *dy, float *dw, f
                                                 Cout, p.ci_tiles, p.tiles, p.splits, p.ups);
   };
   // byte offsets within a unit take 32 bits unless its lines are enormous
-  const long span = (long)p.q.P * p.q.nlx * W * (Cin > Cout ? Cin : Cout) * 2;
+  const long span = (long)p.q.P * (p.q.R + 2) * W * (Cin > Cout ? Cin : Cout) * 2;
   if (span < (1L << 31)) go(k_conv_wgrad<NA, NB, false>);
   else go(k_conv_wgrad<NA, NB, true>);
   HIPCHK(hipGetLastError());
