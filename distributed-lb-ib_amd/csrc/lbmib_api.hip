@@ -72,7 +72,7 @@ extern "C" int lbmib_destroy(lbmib_ctx *ctx) {
   if (ctx->stream_b) (void)hipStreamDestroy(ctx->stream_b);
   void *ptrs[] = {ctx->f[0], ctx->f[1], ctx->F[0], ctx->F[1], ctx->ib.pos, ctx->ib.frc, ctx->ib.start,
                   ctx->ib.wgt, ctx->ib.bin_count, ctx->ib.bin_list, ctx->ib.box, ctx->ib.done, ctx->ib.ub, ctx->d_sheets,
-                  ctx->d_err, ctx->d_partials, ctx->d_tot, ctx->d_mat, ctx->d_tab, ctx->d_rowtab, ctx->d_rect, ctx->d_ref,
+                  ctx->d_err, ctx->d_partials, ctx->d_tot, ctx->d_mat, ctx->d_tab, ctx->d_rowtab, ctx->d_rowtab_elems, ctx->d_rect, ctx->d_ref,
                   ctx->f_spare, ctx->pos_save, ctx->F_save, ctx->box_save, ctx->d_raster, ctx->d_cpart};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -225,15 +225,17 @@ extern "C" int lbmib_create(const lbmib_fluid_params *fluid, int nsheets, const 
     c.dtab = ctx->d_tab;
     c.dref = ctx->d_ref;
   }
-  if (!rc && row_path_buffered(g, ctx->esz)) {
+  const bool buffered = row_path_buffered(g, ctx->esz);
+  if (!rc && (buffered || row_path_elems(g))) {
     std::vector<uint32_t> tab;
-    if (row_source_table(g, ctx->esz, tab) == LBMIB_OK) {
-      alloc((void **)&ctx->d_rowtab, sizeof(uint32_t) * tab.size());
-      if (!rc && hipMemcpy(ctx->d_rowtab, tab.data(), sizeof(uint32_t) * tab.size(), hipMemcpyHostToDevice) !=
-                     hipSuccess)
+    uint32_t **dst = buffered ? &ctx->d_rowtab : &ctx->d_rowtab_elems;
+    if (row_source_table(g, buffered ? ctx->esz : 1, tab) == LBMIB_OK) {
+      alloc((void **)dst, sizeof(uint32_t) * tab.size());
+      if (!rc && hipMemcpy(*dst, tab.data(), sizeof(uint32_t) * tab.size(), hipMemcpyHostToDevice) != hipSuccess)
         rc = LBMIB_ERR_HIP;
     }
   }
+  ctx->kv.rowtab_elems = ctx->d_rowtab_elems;
 
   IBState &ib = ctx->ib;
   ib.nsheets = nsheets;

@@ -275,6 +275,7 @@ __device__ __forceinline__ void update_cell(const Geometry &g, const typename Tr
 constexpr int kRowTabStride = 20;
 
 int row_source_table(const Geometry &g, size_t es, std::vector<uint32_t> &tab) {
+  // es: bytes of an element (offsets in bytes), or 1 (offsets in elements)
   const long nrows = (long)g.ny * g.nz;
   tab.assign((size_t)nrows * kRowTabStride, 0u);
   const uint64_t pitch_b = (uint64_t)g.pq * es, sy_b = (uint64_t)g.prow * es;
@@ -369,15 +370,79 @@ struct NoSink {
   __device__ __forceinline__ void operator()(const V *) const {}
 };
 
-// One lane of the buffer-addressed row path: the update of cell (x, row) by
-// a wave whose lanes hold consecutive x of the same row (SGPR row offsets).
-// Dead lanes of an active row store zeros (whole cache lines); x edges of a
-// wall or periodic x axis are left to k_collide_xedges.  sink(v) sees the
+// How a row kernel reaches the two population arrays: a lane's byte offset vo
+// and a wave-uniform offset so in units of `unit` per element.  Arrays under
+// 4 GiB: buffer instructions, so in bytes.  Larger ones: so in elements (the
+// table holds 32 bits: up to 2^32 elements), one 64-bit scalar address per
+// population; the cell-by-cell general path, which larger arrays took before,
+// ran the fused kernel at 4.7 TB/s at 512 x 256 x 256 in FP64 (2163 us; this form
+// 1948 us, 5.2 TB/s).
+template <int P>
+struct BufRows {
+  static constexpr uint32_t unit = sizeof(typename Traits<P>::S);
+  __amdgpu_buffer_rsrc_t rin, rout;
+  template <bool NTL>
+  __device__ __forceinline__ typename Traits<P>::T ld(uint32_t vo, uint32_t so) const {
+    return bld_h<P, NTL>(rin, vo, so);
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(uint32_t vo, uint32_t so, typename Traits<P>::T v) const {
+    bst_h<P, NT>(rout, vo, so, v);
+  }
+};
+template <int P>
+struct PtrRows {
+  using S = typename Traits<P>::S;
+  static constexpr uint32_t unit = 1;
+  const S *fin;
+  S *fout;
+  template <bool NTL>
+  __device__ __forceinline__ typename Traits<P>::T ld(uint32_t vo, uint32_t so) const {
+    return ld_h<P, NTL>((const S *)((const char *)(fin + so) + vo));
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(uint32_t vo, uint32_t so, typename Traits<P>::T v) const {
+    st_h<P, NT>((S *)((char *)(fout + so) + vo), v);
+  }
+};
+
+// The two x-edge cells of an active row on a wall or periodic x axis: the directions
+// whose source lies beyond the edge come from the cell's own opposite
+// population (half-way bounce-back) or from the row's other end.  Directions
+// reflected at a y/z wall (mask) stay as they are.  (A launch of its own for
+// these cells took 24 us at 151 x 102 x 77, where the fused kernel takes 42; the steps of
+// 256^3 grids went from 655 to 494 us in FP32, from 422 to 315 in FP16.)
+template <int P, bool NTL, class A>
+__device__ __forceinline__ void x_edge_sources(const Geometry &g, const A &acc, int x, const uint32_t so[19],
+                                               uint32_t mask, uint32_t row_u, typename Traits<P>::T b1,
+                                               typename Traits<P>::T b2, typename Traits<P>::T v[19]) {
+  constexpr uint32_t es = sizeof(typename Traits<P>::S);
+  if (g.bc[0] == LBMIB_BC_INOUT) return;
+  const uint32_t pitch_u = (uint32_t)g.pq * A::unit;
+#pragma unroll
+  for (int side = -1; side <= 1; side += 2) {
+    if (x != (side > 0 ? g.lo[0] : g.hi[0])) continue;
+#pragma unroll
+    for (int q = 0; q < 19; ++q) {
+      if (kCX[q] != side || ((mask >> q) & 1u)) continue;
+      if (g.bc[0] == LBMIB_BC_PERIODIC) {
+        // so holds the x shift: x = -1 is the last cell of the row, x = nx the first
+        v[q] = side > 0 ? acc.template ld<NTL>((uint32_t)g.nx * es, so[q]) : acc.template ld<NTL>(0, so[q] - A::unit);
+      } else {
+        v[q] = acc.template ld<NTL>((uint32_t)x * es, row_u + kOPP[q] * pitch_u);
+        if constexpr (Traits<P>::dev) v[q] -= kCX[q] * (kCLS[q] == 1 ? b1 : b2);
+      }
+    }
+  }
+}
+
+// One lane of the row path: the update of cell (x, row) by a wave whose lanes
+// hold consecutive x of the same row (SGPR row offsets).  Dead lanes of an
+// active row store zeros (whole cache lines).  sink(v) sees the
 // post-collision values (kernel units, before the stores round them) of an
-// updated cell: not on dead rows or lanes, x edges or frozen planes.
-template <int P, bool NT, bool NTL, class Sink = NoSink>
-__device__ __forceinline__ void row_cell(const Geometry &g, __amdgpu_buffer_rsrc_t rin, __amdgpu_buffer_rsrc_t rout,
-                                         int own, const KConsts<typename Traits<P>::T> &c, int nsheets,
+// updated cell: not on dead rows or lanes or frozen planes.
+template <int P, bool NT, bool NTL, class A, class Sink = NoSink>
+__device__ __forceinline__ void row_cell(const Geometry &g, const A &acc, int own, const KConsts<typename Traits<P>::T> &c, int nsheets,
                                          const int *__restrict__ box_cur, const int *__restrict__ box_prev,
                                          const typename Traits<P>::FT *__restrict__ Fcur,
                                          const typename Traits<P>::FT *__restrict__ Fprev,
@@ -387,22 +452,21 @@ __device__ __forceinline__ void row_cell(const Geometry &g, __amdgpu_buffer_rsrc
   using T = typename Traits<P>::T;
   using S = typename Traits<P>::S;
   constexpr uint32_t es = sizeof(S);
-  const uint32_t pitch_b = (uint32_t)g.pq * es;   // between the populations of a cell
-  const uint32_t sy_b = (uint32_t)g.prow * es;    // between rows (y, z) and (y + 1, z)
+  const uint32_t pitch_b = (uint32_t)g.pq * A::unit;   // between the populations of a cell
+  const uint32_t sy_b = (uint32_t)g.prow * A::unit;    // between rows (y, z) and (y + 1, z)
   // bulk of a split step: the band launch has stored the band's cells
   if (band && row_meets_band(band, row % g.ny, row / g.ny) && in_band_boxes(band, x, row % g.ny, row / g.ny)) return;
   const bool edge = x == g.lo[0] || x == g.hi[0];
-  // frozen inlet/outlet planes; x edges of wall/periodic x go to k_collide_xedges
+  // frozen inlet/outlet planes
   const bool frozen = edge && g.bc[0] == LBMIB_BC_INOUT;
-  // Filler lanes (dead x, and the x edges left to k_collide_xedges) store
-  // zeros, so that every store instruction writes whole cache lines of the
-  // row: partially written lines cost HBM write bandwidth.  Nothing reads
-  // a dead cell; k_collide_xedges rewrites its edge cells afterwards.
-  const bool filler = x < g.lo[0] || x > g.hi[0] || (edge && !frozen);
+  // Filler lanes (dead x) store zeros, so that every store instruction writes
+  // whole cache lines of the row: partially written lines cost HBM write
+  // bandwidth.  Nothing reads a dead cell.
+  const bool filler = x < g.lo[0] || x > g.hi[0];
   const uint32_t vo = (uint32_t)x * es;
   const int y = row % g.ny, z = row / g.ny;
   if (y < g.lo[1] || y > g.hi[1] || z < g.lo[2] || z > g.hi[2]) return;  // dead row
-  const uint32_t row_b = (uint32_t)row * sy_b;  // byte offset of (0, y, z) in a plane
+  const uint32_t row_b = (uint32_t)row * sy_b;  // of (0, y, z) in a plane
   const long c0 = (long)x + (long)g.nx * row;
   T v[19];
   if (filler) {
@@ -421,7 +485,7 @@ __device__ __forceinline__ void row_cell(const Geometry &g, __amdgpu_buffer_rsrc
         uint32_t qb = row_b;  // first step: the cell's own populations
 #pragma unroll
         for (int q = 0; q < 19; ++q) {
-          v[q] = bld_h<P, NTL>(rin, vo, qb);
+          v[q] = acc.template ld<NTL>(vo, qb);
           qb += pitch_b;
         }
       } else {
@@ -430,8 +494,10 @@ __device__ __forceinline__ void row_cell(const Geometry &g, __amdgpu_buffer_rsrc
 #pragma unroll
         for (int q = 0; q < 19; ++q) so[q] = ldc(rt + q);
 #pragma unroll
-        for (int q = 0; q < 19; ++q) v[q] = bld_h<P, NTL>(rin, vo, so[q]);
-        bounce_fix<P>(ldc(rt + 19), c.br[1], c.br[2], v);
+        for (int q = 0; q < 19; ++q) v[q] = acc.template ld<NTL>(vo, so[q]);
+        const uint32_t bbm = ldc(rt + 19);
+        x_edge_sources<P, NTL>(g, acc, x, so, bbm, row_b, c.br[1], c.br[2], v);
+        bounce_fix<P>(bbm, c.br[1], c.br[2], v);
       }
       if (own) {
         rho = c.rho0; d = c.d0; ux = c.u0x; uy = c.u0y; uz = c.u0z;  // lbm_ib.c:837-849
@@ -456,14 +522,14 @@ __device__ __forceinline__ void row_cell(const Geometry &g, __amdgpu_buffer_rsrc
     // k_collide_stream_pairs)
 #pragma unroll
     for (int q = 0; q < 19; ++q) {
-      bst_h<P, false>(rout, vo, sb, v[q]);
+      acc.template st<false>(vo, sb, v[q]);
       sb += pitch_b;
     }
     return;
   }
 #pragma unroll
   for (int q = 0; q < 19; ++q) {
-    bst_h<P, NT>(rout, vo, sb, v[q]);
+    acc.template st<NT>(vo, sb, v[q]);
     sb += pitch_b;
   }
 }
@@ -471,16 +537,17 @@ __device__ __forceinline__ void row_cell(const Geometry &g, __amdgpu_buffer_rsrc
 // Row form: blocks walk whole (y, z) rows with a stride (one block per row
 // when the grid has as many blocks as rows).
 //
-// BUF (buffer addressing, needs a population array under 2^32 bytes): for each
+// ADDR kRowsBuf and kRowsPtr (BufRows, PtrRows): for each
 // population the source row -- wrapped on periodic axes, or the own row's
 // opposite population where the source lies beyond a y/z wall (half-way
-// bounce-back) -- is the same for the whole row, so its byte offset is a
+// bounce-back) -- is the same for the whole row, so its offset is a
 // wave-uniform (SGPR) value and the 19 loads and 19 stores of a lane share one
 // VGPR offset, x * sizeof(S) (one cell per thread, blockDim.x >= nx).  Lanes
 // on the frozen inlet/outlet planes take the table; the two x-edge cells of a
-// row on a wall or periodic x axis are left to k_collide_xedges.  Without BUF
-// every cell takes update_cell.
-template <int P, bool NT, bool NTL, bool BUF>
+// row on a wall or periodic x axis take x_edge_sources.  kRowsGeneral: every
+// cell takes update_cell.
+enum { kRowsGeneral = 0, kRowsBuf = 1, kRowsPtr = 2 };
+template <int P, bool NT, bool NTL, int ADDR>
 __global__ void __launch_bounds__(1024)
     k_collide_stream_rows(Geometry g, const typename Traits<P>::S *__restrict__ fin,
                           typename Traits<P>::S *__restrict__ fout, int own, KConsts<typename Traits<P>::T> c,
@@ -488,7 +555,7 @@ __global__ void __launch_bounds__(1024)
                           const typename Traits<P>::FT *__restrict__ Fcur,
                           const typename Traits<P>::FT *__restrict__ Fprev, const uint32_t *__restrict__ rowtab,
                           const int *__restrict__ band, int box_rows_cached) {
-  if constexpr (!BUF) {
+  if constexpr (ADDR == kRowsGeneral) {
     int row;
     for (long it = blockIdx.x; next_row(g, it, row); it += gridDim.x) {
       const int y = row % g.ny, z = row / g.ny;
@@ -498,12 +565,15 @@ __global__ void __launch_bounds__(1024)
     }
   } else {
     // one cell per thread: blockDim.x >= nx (checked by the launcher)
-    const __amdgpu_buffer_rsrc_t rin = make_rsrc(fin), rout = make_rsrc(fout);
     const int x = threadIdx.x;
     if (x >= g.nx) return;
+    const auto acc = [&] {
+      if constexpr (ADDR == kRowsBuf) return BufRows<P>{make_rsrc(fin), make_rsrc(fout)};
+      else return PtrRows<P>{fin, fout};
+    }();
     int row;
     for (long it = blockIdx.x; next_row(g, it, row); it += gridDim.x)
-      row_cell<P, NT, NTL>(g, rin, rout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, row, x, band,
+      row_cell<P, NT, NTL>(g, acc, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, row, x, band,
                            box_rows_cached);
   }
 }
@@ -514,9 +584,8 @@ __global__ void __launch_bounds__(1024)
 // adjacent; for c_x != 0 it is one element off the pair alignment, which the
 // memory system handles as an unaligned access.  Requires nx even, the
 // active x range [lo, hi] with lo even and hi odd (so no pair straddles it),
-// and blockDim.x >= nx / 2 (nx <= 1024).  Edge pairs of a wall or periodic x axis compute
-// their edge cell with the in-row neighbour, and k_collide_xedges, launched
-// after this kernel on the same stream, rewrites that cell.
+// and blockDim.x >= nx / 2 (nx <= 1024).  The edge cells of a wall or periodic x
+// axis take x_edge_sources.
 template <int P>
 struct PairBits;
 template <>
@@ -612,6 +681,9 @@ __global__ void __launch_bounds__(512)
         for (int q = 0; q < 19; ++q) bld_pair<P, NTL>(rin, vo, so[q], v[0][q], v[1][q]);
         const uint32_t bbm = ldc(rt + 19);
 #pragma unroll
+        for (int k = 0; k < 2; ++k)
+          x_edge_sources<P, NTL>(g, BufRows<P>{rin, rout}, x0 + k, so, bbm, row_b, c.br[1], c.br[2], v[k]);
+#pragma unroll
         for (int k = 0; k < 2; ++k) {
           bounce_fix<P>(bbm, c.br[1], c.br[2], v[k]);
           T fpx = 0, fpy = 0, fpz = 0;
@@ -659,9 +731,8 @@ __global__ void __launch_bounds__(512)
 // One lane of the two-row path: cells (x, row0) and (x, row0 + 1), rows
 // (y0, z) and (y0 + 1, z) of one z plane (row0 even, ny even), with two
 // independent sets of aligned buffer loads, which doubles the bytes each wave
-// keeps in flight.  Filler lanes (dead x, and the x edges of a wall or
-// periodic x axis, left to k_collide_xedges) store zeros so that the rows'
-// cache lines are written whole.
+// keeps in flight.  Filler lanes (dead x) store zeros so that the rows' cache
+// lines are written whole.
 template <int P, bool NT, bool NTL>
 __device__ __forceinline__ void row_pair_cell(const Geometry &g, __amdgpu_buffer_rsrc_t rin,
                                               __amdgpu_buffer_rsrc_t rout, int own,
@@ -678,7 +749,7 @@ __device__ __forceinline__ void row_pair_cell(const Geometry &g, __amdgpu_buffer
   const uint32_t sy_b = (uint32_t)g.prow * es;    // between rows (y, z) and (y + 1, z)
   const bool edge = x == g.lo[0] || x == g.hi[0];
   const bool frozen = edge && g.bc[0] == LBMIB_BC_INOUT;
-  const bool filler = x < g.lo[0] || x > g.hi[0] || (edge && !frozen);
+  const bool filler = x < g.lo[0] || x > g.hi[0];
   const uint32_t vo = (uint32_t)x * es;
   const int y0 = row0 % g.ny, z = row0 / g.ny;  // rows row0, row0 + 1 = (y0, z), (y0 + 1, z)
   if (z < g.lo[2] || z > g.hi[2]) return;  // dead rows
@@ -718,7 +789,11 @@ __device__ __forceinline__ void row_pair_cell(const Geometry &g, __amdgpu_buffer
         for (int q = 0; q < 19; ++q) v[k][q] = bld_h<P, NTL>(rin, vo, so[k][q]);
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        bounce_fix<P>(ldc(rt + k * kRowTabStride + 19), c.br[1], c.br[2], v[k]);
+        const uint32_t bbm = ldc(rt + k * kRowTabStride + 19);
+        if (live[k])  // (a dead row has no sources in the table)
+          x_edge_sources<P, NTL>(g, BufRows<P>{rin, rout}, x, so[k], bbm, (uint32_t)(row0 + k) * sy_b, c.br[1],
+                                 c.br[2], v[k]);
+        bounce_fix<P>(bbm, c.br[1], c.br[2], v[k]);
         const long ck = (long)x + (long)g.nx * (row0 + k);
         T fpx = 0, fpy = 0, fpz = 0;
         if (in_any_box(box_prev, nsheets, x, y0 + k, z)) {
@@ -768,8 +843,7 @@ __device__ __forceinline__ void row_pair_cell(const Geometry &g, __amdgpu_buffer
 // Two rows per block (y and y + 1 of one z plane): lane x updates (x, y, z)
 // and (x, y + 1, z) (row_pair_cell), which doubles the bytes each wave keeps
 // in flight without the unaligned pair loads of k_collide_stream_pairs.
-// Requires ny even and blockDim.x >= nx; x-edge cells of a wall or periodic x
-// axis are left to k_collide_xedges.
+// Requires ny even and blockDim.x >= nx.
 template <int P, bool NT, bool NTL>
 __global__ void __launch_bounds__(512)
     k_collide_stream_rows2(Geometry g, const typename Traits<P>::S *__restrict__ fin,
@@ -814,7 +888,8 @@ __global__ void __launch_bounds__(512)
   if (row >= nrows || x >= g.nx) return;
   const KConsts<T> c = ldc_obj(reinterpret_cast<const KConsts<T> *>(dp->kc));
   const int *box = ldc(&dp->ib.box);
-  row_cell<P, NT, NTL>(g, make_rsrc(ldc(&dp->f[cur])), make_rsrc(ldc(&dp->f[1 - cur])), own, c, ldc(&dp->nsheets),
+  row_cell<P, NT, NTL>(g, BufRows<P>{make_rsrc(ldc(&dp->f[cur])), make_rsrc(ldc(&dp->f[1 - cur]))}, own, c,
+                       ldc(&dp->nsheets),
                        box + slot * kMaxSheets * 6, box + (1 - slot) * kMaxSheets * 6,
                        (const FT *)ldc(&dp->F[slot]), (const FT *)ldc(&dp->F[1 - slot]), ldc(&dp->rowtab), row, x,
                        nullptr, box_rows_cached);
@@ -887,25 +962,6 @@ __global__ void __launch_bounds__(256)
     }
     if (!dup) update_cell<P, NT, NTL>(g, fin, fout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, x, y, z);
   }
-}
-
-// The x-edge cells (x = lo, hi) of every active row when x is a wall or a
-// periodic axis, by the general rules; completes the buffer-addressed rows.
-template <int P, bool NT, bool NTL>
-__global__ void __launch_bounds__(256)
-    k_collide_xedges(Geometry g, const typename Traits<P>::S *__restrict__ fin,
-                     typename Traits<P>::S *__restrict__ fout, int own, KConsts<typename Traits<P>::T> c,
-                     int nsheets, const int *__restrict__ box_cur, const int *__restrict__ box_prev,
-                     const typename Traits<P>::FT *__restrict__ Fcur,
-                     const typename Traits<P>::FT *__restrict__ Fprev, const int *__restrict__ band) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= 2L * g.ny * g.nz) return;
-  const long row = e >> 1;
-  const int x = (e & 1) ? g.hi[0] : g.lo[0];
-  if ((e & 1) && g.lo[0] == g.hi[0]) return;  // one-cell-wide axis: done by the even item
-  if (band && in_band_boxes(band, x, (int)(row % g.ny), (int)(row / g.ny))) return;  // stored by the band launch
-  update_cell<P, NT, NTL>(g, fin, fout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, x, (int)(row % g.ny),
-                          (int)(row / g.ny));
 }
 
 // V consecutive cells of one x-row per thread: the 9 populations with
@@ -1202,6 +1258,10 @@ static void launch_vec(const Geometry &g, const void *fin, void *fout, int own, 
 bool row_path_buffered(const Geometry &g, size_t es) {
   return (unsigned long long)g.pelems * es <= 0xFFFFFFFFull && (int)row_block(g).x >= g.nx;
 }
+// The same by scalar addresses (PtrRows): offsets in elements.
+bool row_path_elems(const Geometry &g) {
+  return (unsigned long long)g.pelems <= 0xFFFFFFFFull && (int)row_block(g).x >= g.nx;
+}
 
 template <int P, bool NT, bool NTL>
 static void launch_rows2(int nblocks, const Geometry &g, const void *fin, void *fout, int own,
@@ -1216,12 +1276,6 @@ static void launch_rows2(int nblocks, const Geometry &g, const void *fin, void *
   k_collide_stream_rows2<P, NT, NTL><<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets,
                                                       box_cur, box_prev, (const FT *)Fcur, (const FT *)Fprev, rowtab,
                                                       box_rows_cached);
-  if (g.bc[0] != LBMIB_BC_INOUT) {  // whole-grid steps only
-    const long items = 2L * g.ny * g.nz;
-    k_collide_xedges<P, NT, NTL><<<(unsigned)((items + 255) / 256), 256, 0, s>>>(
-        g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets, box_cur, box_prev, (const FT *)Fcur,
-        (const FT *)Fprev, nullptr);
-  }
 }
 
 // Whether the two-rows-per-block path applies (see k_collide_stream_rows2).
@@ -1245,38 +1299,25 @@ static void launch_pairs(int nblocks, const Geometry &g, const void *fin, void *
   k_collide_stream_pairs<P, NT, NTL><<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets,
                                                       box_cur, box_prev, (const FT *)Fcur, (const FT *)Fprev, rowtab,
                                                       band, box_rows_cached);
-  if (g.bc[0] != LBMIB_BC_INOUT) {
-    const long items = 2L * g.ny * g.nz;
-    k_collide_xedges<P, NT, NTL><<<(unsigned)((items + 255) / 256), 256, 0, s>>>(
-        g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets, box_cur, box_prev, (const FT *)Fcur,
-        (const FT *)Fprev, band);
-  }
 }
 
 template <int P, bool NT, bool NTL>
 static void launch_rows(int nblocks, const Geometry &g, const void *fin, void *fout, int own,
                         const FluidConsts<double> &c, int nsheets, const int *box_cur, const int *box_prev,
-                        const void *Fcur, const void *Fprev, const uint32_t *rowtab, const int *band,
-                        int box_rows_cached, hipStream_t s) {
+                        const void *Fcur, const void *Fprev, const uint32_t *rowtab, const uint32_t *rowtab_elems,
+                        const int *band, int box_rows_cached, hipStream_t s) {
   using FT = typename Traits<P>::FT;
   using S = typename Traits<P>::S;
   const dim3 b = row_block(g);
   const int nrows = g.ny * g.nz;
   const dim3 gr(nblocks < nrows ? nblocks : nrows);
-  if (rowtab && row_path_buffered(g, sizeof(S))) {
-    k_collide_stream_rows<P, NT, NTL, true><<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets,
-                                                             box_cur, box_prev, (const FT *)Fcur, (const FT *)Fprev,
-                                                             rowtab, band, box_rows_cached);
-    if (g.bc[0] != LBMIB_BC_INOUT) {
-      const long items = 2L * g.ny * g.nz;
-      k_collide_xedges<P, NT, NTL><<<(unsigned)((items + 255) / 256), 256, 0, s>>>(
-          g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets, box_cur, box_prev, (const FT *)Fcur,
-          (const FT *)Fprev, band);
-    }
-  } else
-    k_collide_stream_rows<P, NT, NTL, false><<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c),
-                                                              nsheets, box_cur, box_prev, (const FT *)Fcur,
-                                                              (const FT *)Fprev, nullptr, band, box_rows_cached);
+  auto go = [&](auto kern, const uint32_t *tab) {
+    kern<<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets, box_cur, box_prev,
+                          (const FT *)Fcur, (const FT *)Fprev, tab, band, box_rows_cached);
+  };
+  if (rowtab && row_path_buffered(g, sizeof(S))) go(k_collide_stream_rows<P, NT, NTL, kRowsBuf>, rowtab);
+  else if (rowtab_elems) go(k_collide_stream_rows<P, NT, NTL, kRowsPtr>, rowtab_elems);
+  else go(k_collide_stream_rows<P, NT, NTL, kRowsGeneral>, nullptr);
 }
 
 template <int P, bool NT>
@@ -1293,7 +1334,7 @@ static void launch_any(int v, const Geometry &g, const void *fin, void *fout, in
     if (v == 8) return launch_vec<P, 8, NT>(g, fin, fout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, s);
   }
   launch_rows<P, NT, false>(g.ny * g.nz, g, fin, fout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, nullptr,
-                            nullptr, 0, s);
+                            nullptr, nullptr, 0, s);
 }
 
 int launch_collide_stream(int prec, const Geometry &g, const void *fin, void *fout, int own_mode,
@@ -1349,10 +1390,10 @@ int launch_collide_stream(int prec, const Geometry &g, const void *fin, void *fo
   if (v == 1) {
     const int nb = kv.blocks > 0 ? kv.blocks : g.ny * g.nz;
     LBMIB_DISPATCH(prec, ({
-      if (nt && ntl) launch_rows<P, true, true>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, band, kv.box_rows_cached, s);
-      else if (nt) launch_rows<P, true, false>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, band, kv.box_rows_cached, s);
-      else if (ntl) launch_rows<P, false, true>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, band, kv.box_rows_cached, s);
-      else launch_rows<P, false, false>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, band, kv.box_rows_cached, s);
+      if (nt && ntl) launch_rows<P, true, true>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, kv.rowtab_elems, band, kv.box_rows_cached, s);
+      else if (nt) launch_rows<P, true, false>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, kv.rowtab_elems, band, kv.box_rows_cached, s);
+      else if (ntl) launch_rows<P, false, true>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, kv.rowtab_elems, band, kv.box_rows_cached, s);
+      else launch_rows<P, false, false>(nb, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, kv.rowtab_elems, band, kv.box_rows_cached, s);
     }));
     return hipGetLastError() == hipSuccess ? LBMIB_OK : LBMIB_ERR_HIP;
   }
@@ -1392,8 +1433,8 @@ __global__ void __launch_bounds__(1024)
   int row;
   for (long it = blockIdx.x; next_row(g, it, row); it += gridDim.x) {
     A sr = (A)rho0, sx = (A)u0x, sy = (A)u0y, sz = (A)u0z;
-    row_cell<P, NT, NTL>(g, rin, rout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, row, x, nullptr,
-                         box_rows_cached, [&](const T *v) {
+    row_cell<P, NT, NTL>(g, BufRows<P>{rin, rout}, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, row, x,
+                         nullptr, box_rows_cached, [&](const T *v) {
                            S h[19];
 #pragma unroll
                            for (int q = 0; q < 19; ++q) h[q] = to_bits<P>(v[q]);

@@ -219,6 +219,7 @@ struct KernelVariant {
   int blocks;            // > 0: persistent grid of this many blocks walking rows (one cell per thread)
   int box_rows_cached;   // with nontemporal stores: rows meeting a support box stored with the default policy
                          // (1), or not (0); -1 automatic (box_rows_auto)
+  const uint32_t *rowtab_elems;  // arrays of 2^32 bytes and more: the row source table in elements, or null
 };
 
 // rowtab: the row source table (row_source_table) on the device, or null for
@@ -232,6 +233,7 @@ int launch_collide_stream(int prec, const Geometry &g, const void *fin, void *fo
                           hipStream_t s, int sel = 0, int *rect_buf = nullptr, int band_blocks = 0);
 constexpr int kRectBufInts = 1 + 6 * kMaxSheets;
 bool row_path_buffered(const Geometry &g, size_t es);
+bool row_path_elems(const Geometry &g);
 // A fused step that also writes the coarse stored-moment planes of the state
 // it writes (lbmib_step_coarse): whether it applies, and its launch
 // (LBMIB_ERR_ARG where it does not apply).
