@@ -1337,17 +1337,67 @@ static void launch_any(int v, const Geometry &g, const void *fin, void *fout, in
                             nullptr, nullptr, 0, s);
 }
 
+// Shape of the fused launch where the caller leaves it open (cpt 0, nt -1): x
+// pairs or one cell per lane, and which accesses are nontemporal.  Each side
+// was measured in the rows layout; times are the fused kernel's, in us.
+//  - Rows that are no whole number of 64-byte pieces: each row's first and
+//    last pieces are written by two waves, and nontemporal stores send them to
+//    memory in parts.  Default policy: 500 x 256 x 256 FP32 1314 -> 932, 250 x
+//    100 x 100 FP16 52 -> 36, 151 x 100 x 100 FP64 106 -> 90.  Rows of one wave
+//    in 32 or 64 bits keep nontemporal stores (60 x 280 x 280 FP32 130, 139
+//    with the default policy).
+//  - An array that the 256 MB Infinity Cache holds next to part of the other:
+//    default policy (192 x 100 x 100 FP32 54.1 -> 51.8, 128 x 100 x 100 FP32
+//    38.1 -> 35.2), except rows of one 128-byte line or less (64 x 100 x 100
+//    FP16 16.3, nontemporal 15.2).  Beyond it nontemporal loads and stores
+//    (256^3 FP32 446 -> 435).
+//  - Wall or periodic x: the edge lanes read lines that other lanes read too,
+//    so loads use the default policy (256^3 FP32 448 -> 434, 64 x 288 x 288 212 ->
+//    193); so does the path by scalar addresses (512 x 256 x 256 FP64 1944 ->
+//    1782).
+//  - Pairs: FP32 from 96 cells a row (256^3 435 -> 417, 192 x 256 x 256 325 ->
+//    315; 64 cells fill half a wave: 137 -> 177), FP64 where they fill their
+//    waves (128 x 288 x 288 568 -> 551; 192 x 256 x 256 672 -> 684), in 16 bits
+//    where they fill their waves or beyond 256 cells (288^3 426 -> 355; 192 x
+//    256 x 256 161, pairs 180; 64 x 100 x 100 15.2, pairs 21.8).  Not on small
+//    arrays, and on wall or periodic x only in 16 bits beyond 256 cells
+//    (256^3 FP32 448 -> 520; 288^3 FP16 613 -> 446).
+FusedShape fused_shape(int prec, const Geometry &g, bool buffered, int cpt_req, int nt_req) {
+  const size_t es = prec == LBMIB_F64 ? 8 : (prec == LBMIB_F32 ? 4 : 2);
+  const bool half = es == 2, rows = g.prow != g.nx;
+  const bool edges = g.bc[0] != LBMIB_BC_INOUT;
+  FusedShape sh;
+  if (!rows) {
+    // planes: nontemporal, pairs in 16 bits
+    sh.nt = 3;
+    sh.cpt = half && buffered && pair_path_ok(g) ? 2 : 1;
+  } else {
+    const size_t row_bytes = g.nx * es;
+    const bool aligned = row_bytes % 64 == 0;
+    const bool small = 19.0 * g.n * es <= 160.0 * (1 << 20);
+    bool nts;
+    if (small) nts = row_bytes <= 128;
+    else nts = aligned || (g.nx <= 64 && !half);
+    const bool ntl = nts && (aligned || small) && !edges && buffered;
+    sh.nt = (nts ? 1 : 0) | (ntl ? 2 : 0);
+    const bool full = g.nx % 128 == 0;  // pairs fill their waves
+    bool pairs;
+    if (half) pairs = g.nx > 256 || (!edges && !small && full);
+    else pairs = !edges && !small && aligned && (prec == LBMIB_F32 ? g.nx >= 96 : full);
+    sh.cpt = pairs && buffered && pair_path_ok(g) ? 2 : 1;
+  }
+  if (nt_req >= 0) sh.nt = nt_req;
+  if (cpt_req > 0) sh.cpt = cpt_req;
+  return sh;
+}
+
 int launch_collide_stream(int prec, const Geometry &g, const void *fin, void *fout, int own_mode,
                           const FluidConsts<double> &c, int nsheets, const int *box_cur, const int *box_prev,
                           const void *Fcur, const void *Fprev, const uint32_t *rowtab, const KernelVariant &kv,
                           hipStream_t s, int sel, int *rect_buf, int band_blocks) {
   if (sel != kRowsAll && (!rowtab || !rect_buf)) return LBMIB_ERR_ARG;
-  // nontemporal stores and loads by default: the populations are touched
-  // once per step, and keeping them out of the caches was fastest measured
-  const int nt = kv.nt_mask < 0 ? 1 : (kv.nt_mask & 1);
-  const int ntl = kv.nt_mask < 0 ? 1 : ((kv.nt_mask >> 1) & 1);
-  // automatic shape: x pairs for the 16-bit forms (4-byte lanes), one cell
-  // per lane otherwise -- the fastest measured at 256^3
+  const FusedShape shape = fused_shape(prec, g, rowtab != nullptr, kv.cells_per_thread, kv.nt_mask);
+  const int nt = shape.nt & 1, ntl = shape.nt >> 1;
   if (sel == kRowsBand) {
     // the band of a split step, cell by cell (band_blocks blocks of 256)
     LBMIB_DISPATCH(prec, ({
@@ -1363,8 +1413,7 @@ int launch_collide_stream(int prec, const Geometry &g, const void *fin, void *fo
   }
   // the bulk of a split step skips the band's cells
   const int *band = sel == kRowsBulk ? rect_buf : nullptr;
-  int cpt = kv.cells_per_thread;
-  if (cpt <= 0) cpt = ((prec == LBMIB_F16 || prec == LBMIB_BF16) && rowtab && pair_path_ok(g)) ? 2 : 1;
+  int cpt = shape.cpt;
   if (cpt == 3 && sel != kRowsAll) cpt = 1;  // split steps use the row and pair kernels
   if (cpt == 3 && rowtab && rows2_path_ok(g)) {
     const int nb = kv.blocks > 0 ? kv.blocks : g.ny * g.nz / 2;
@@ -1455,8 +1504,7 @@ int launch_collide_coarse(int prec, const Geometry &g, const void *fin, void *fo
                           const void *Fcur, const void *Fprev, const uint32_t *rowtab, const KernelVariant &kv,
                           int F, float *part, float *stored, hipStream_t s) {
   if (!part || !stored) return LBMIB_ERR_ARG;
-  const int nt = kv.nt_mask < 0 ? 1 : (kv.nt_mask & 1);
-  const int ntl = kv.nt_mask < 0 ? 1 : ((kv.nt_mask >> 1) & 1);
+  const int mask = fused_shape(prec, g, true, 1, kv.nt_mask).nt, nt = mask & 1, ntl = mask >> 1;
   const int nrows = g.ny * g.nz;
   const int nb = kv.blocks > 0 && kv.blocks < nrows ? kv.blocks : nrows;
   const double mrx = c.rhor * c.urx;
@@ -1539,8 +1587,7 @@ int launch_collide_batch(int prec, const BatchDesc *d, const int *map, int nbloc
                          int slot, int nt_mask, int rows, int box_rows_cached, hipStream_t s) {
   if (nblocks <= 0) return LBMIB_OK;
   if (wpb < 1 || wpb > 8 || (rows != 1 && rows != 2)) return LBMIB_ERR_ARG;
-  const int nt = nt_mask < 0 ? 1 : (nt_mask & 1);
-  const int ntl = nt_mask < 0 ? 1 : ((nt_mask >> 1) & 1);
+  const int nt = nt_mask & 1, ntl = (nt_mask >> 1) & 1;
   const dim3 b(64 * wpb);
   if (rows == 2) {
     LBMIB_DISPATCH(prec, ({

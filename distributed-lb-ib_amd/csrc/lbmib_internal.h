@@ -222,6 +222,14 @@ struct KernelVariant {
   const uint32_t *rowtab_elems;  // arrays of 2^32 bytes and more: the row source table in elements, or null
 };
 
+// The fused launch's shape: cells per thread and nontemporal mask as in
+// KernelVariant, chosen by grid and storage where the request leaves them
+// open (0, -1).  buffered: the buffer-addressed row path applies.
+struct FusedShape {
+  int cpt, nt;
+};
+FusedShape fused_shape(int prec, const Geometry &g, bool buffered, int cpt_req, int nt_req);
+
 // rowtab: the row source table (row_source_table) on the device, or null for
 // the general path.  sel: which cells to update -- 0 all, 1 the band of a
 // split step (the cells of the band boxes in rect_buf, which the step's

@@ -167,20 +167,20 @@ int lbmib_get_band_box(lbmib_ctx *ctx, int sheet, int *box6);
  * length with one event pair per launch). */
 int lbmib_time_steps(lbmib_ctx *ctx, int nwarm, int nsteps, double *ms_total, double *ms_main_mean);
 /* Launch shape of the fused collide-stream kernel.  cells_per_thread:
- *   0 automatic (2 for the 16-bit forms where it applies, else 1);
+ *   0 automatic (1 or 2, by storage form, row length and array size);
  *   1 one cell per lane, one block per (y, z) row (or a persistent grid);
- *   2 two x-adjacent cells per lane (needs nx even; wall/periodic x edges
- *     then run in a small extra kernel);
+ *   2 two x-adjacent cells per lane (needs nx even);
  *   3 two rows (y, y+1) per block, one cell of each per lane (needs ny even);
  *   4, 8 x-vectors per lane (16 bytes per lane at most; one block per row,
  *     cached loads).
- * nontemporal: bit 0 stores, bit 1 loads; -1 automatic (both).
+ * nontemporal: bit 0 stores, bit 1 loads; -1 automatic (both on large grids
+ *   whose rows are whole 64-byte pieces; see fused_shape in lbmib_fluid.hip).
  * blocks_per_cu > 0: a persistent grid of that many blocks per compute unit
  * walking the rows (0 = one block per row or row pair).  Not in the
  * reference: the knobs bench.py's autotuning sweep sets.  Every variant
  * computes bit-identical results. */
 int lbmib_set_kernel_variant(lbmib_ctx *ctx, int cells_per_thread, int nontemporal, int blocks_per_cu);
-/* With nontemporal stores (the default), the fused kernel can store the rows
+/* With nontemporal stores, the fused kernel can store the rows
  * that meet a sheet's support box (widened by one cell in y and z) with the
  * default cache policy (cached = 1) instead (0).  -1, the default at
  * create: 1 when those rows' stores, estimated from the sheets' extents,
