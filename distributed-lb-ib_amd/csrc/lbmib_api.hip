@@ -227,13 +227,9 @@ extern "C" int lbmib_create(const lbmib_fluid_params *fluid, int nsheets, const 
   }
   const bool buffered = row_path_buffered(g, ctx->esz);
   if (!rc && (buffered || row_path_elems(g))) {
-    std::vector<uint32_t> tab;
     uint32_t **dst = buffered ? &ctx->d_rowtab : &ctx->d_rowtab_elems;
-    if (row_source_table(g, buffered ? ctx->esz : 1, tab) == LBMIB_OK) {
-      alloc((void **)dst, sizeof(uint32_t) * tab.size());
-      if (!rc && hipMemcpy(*dst, tab.data(), sizeof(uint32_t) * tab.size(), hipMemcpyHostToDevice) != hipSuccess)
-        rc = LBMIB_ERR_HIP;
-    }
+    alloc((void **)dst, sizeof(uint32_t) * (size_t)row_table_entries(g));
+    if (!rc) rc = launch_row_table(g, buffered ? ctx->esz : 1, *dst, ctx->stream);
   }
   ctx->kv.rowtab_elems = ctx->d_rowtab_elems;
 

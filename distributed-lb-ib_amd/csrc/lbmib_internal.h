@@ -5,8 +5,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <vector>
-
 #include "../../include/lbmib.h"
 
 namespace lbmib {
@@ -166,7 +164,7 @@ struct BatchDesc {
   IBState ib;
   const void *f[2];         // population buffers (ping-pong)
   void *F[2];               // force fields by step parity
-  const uint32_t *rowtab;   // row source table (row_source_table)
+  const uint32_t *rowtab;   // row source table (launch_row_table)
   int nsheets, mcap;        // sheets; gather candidate capacity
   int wpr;                  // waves per row of the fused launch (ceil(nx / 64))
   int nrows;                // ny * nz
@@ -230,7 +228,7 @@ struct FusedShape {
 };
 FusedShape fused_shape(int prec, const Geometry &g, bool buffered, int cpt_req, int nt_req);
 
-// rowtab: the row source table (row_source_table) on the device, or null for
+// rowtab: the row source table (launch_row_table) on the device, or null for
 // the general path.  sel: which cells to update -- 0 all, 1 the band of a
 // split step (the cells of the band boxes in rect_buf, which the step's
 // fiber kernel wrote; a grid of band_blocks blocks of 256), 2 all others;
@@ -252,7 +250,10 @@ int launch_collide_coarse(int prec, const Geometry &g, const void *fin, void *fo
                           int F, float *part, float *stored, hipStream_t s);
 bool pair_path_ok(const Geometry &g);
 bool rows2_path_ok(const Geometry &g);
-int row_source_table(const Geometry &g, size_t es, std::vector<uint32_t> &tab);
+// The row source table: its entries, and the launch that fills it (es: bytes of
+// an element, or 1 for offsets in elements).
+long row_table_entries(const Geometry &g);
+int launch_row_table(const Geometry &g, size_t es, uint32_t *tab, hipStream_t s);
 int collide_vec_width(int prec, int nx, int vec_req);
 int launch_materialize(int prec, const Geometry &g, const void *f, int own_mode, const FluidConsts<double> &c,
                        int nsheets, const int *box, const void *F, double *df, double *rho, double *vel,
