@@ -73,7 +73,7 @@ extern "C" int lbmib_destroy(lbmib_ctx *ctx) {
   void *ptrs[] = {ctx->f[0], ctx->f[1], ctx->F[0], ctx->F[1], ctx->ib.pos, ctx->ib.frc, ctx->ib.start,
                   ctx->ib.wgt, ctx->ib.bin_count, ctx->ib.bin_list, ctx->ib.box, ctx->ib.done, ctx->ib.ub, ctx->d_sheets,
                   ctx->d_err, ctx->d_partials, ctx->d_tot, ctx->d_mat, ctx->d_tab, ctx->d_rowtab, ctx->d_rowtab_elems, ctx->d_rect, ctx->d_ref,
-                  ctx->f_spare, ctx->pos_save, ctx->F_save, ctx->box_save, ctx->d_raster, ctx->d_cpart};
+                  ctx->f_spare, ctx->pos_save, ctx->F_save, ctx->box_save, ctx->d_raster, ctx->d_cpart, ctx->d_io};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -264,6 +264,7 @@ extern "C" int lbmib_create(const lbmib_fluid_params *fluid, int nsheets, const 
     alloc((void **)&ctx->d_sheets, sizeof(SheetDesc) * kMaxSheets);
     alloc((void **)&ib.ub, sizeof(double) * 3 * n);
     alloc((void **)&ib.done, sizeof(unsigned));
+    alloc((void **)&ctx->d_io, sizeof(double) * 12 * M);
   }
   ib.sheets = ctx->d_sheets;
   ib.err = ctx->d_err;
@@ -288,10 +289,7 @@ extern "C" int lbmib_create(const lbmib_fluid_params *fluid, int nsheets, const 
 extern "C" int lbmib_set_fiber_positions(lbmib_ctx *ctx, int sheet, const double *xyz) {
   if (!ctx || !xyz || sheet < 0 || sheet >= ctx->nsheets) return LBMIB_ERR_ARG;
   const SheetDesc &d = ctx->sd[sheet];
-  const int m = d.rows * d.cols, M = ctx->nnodes;
-  std::vector<double> soa((size_t)3 * m);
-  for (int k = 0; k < m; ++k)
-    for (int a = 0; a < 3; ++a) soa[(size_t)a * m + k] = xyz[3 * (size_t)k + a];
+  const int m = d.rows * d.cols;
   double ext[4] = {1e300, -1e300, 1e300, -1e300};
   for (int k = 0; k < m; ++k) {
     ext[0] = fmin(ext[0], xyz[3 * (size_t)k + 1]);
@@ -300,9 +298,9 @@ extern "C" int lbmib_set_fiber_positions(lbmib_ctx *ctx, int sheet, const double
     ext[3] = fmax(ext[3], xyz[3 * (size_t)k + 2]);
   }
   for (int a = 0; a < 4; ++a) ctx->hyz[sheet][a] = ext[a];
-  for (int a = 0; a < 3; ++a)
-    HIPCHK(hipMemcpyAsync(ctx->ib.pos + (size_t)a * M + d.off, soa.data() + (size_t)a * m, sizeof(double) * m,
-                          hipMemcpyHostToDevice, ctx->stream));
+  double *io = ctx->d_io + 12 * (size_t)d.off;
+  HIPCHK(hipMemcpyAsync(io, xyz, sizeof(double) * 3 * m, hipMemcpyHostToDevice, ctx->stream));
+  RCHK(launch_unpack_positions(ctx->ib, d.off, m, io, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   return LBMIB_OK;
 }
@@ -661,21 +659,12 @@ extern "C" int lbmib_get_time(lbmib_ctx *ctx, int *t) {
 
 extern "C" int lbmib_get_fibers(lbmib_ctx *ctx, int sheet, double *out) {
   if (!ctx || !out || sheet < 0 || sheet >= ctx->nsheets) return LBMIB_ERR_ARG;
-  HIPCHK(hipStreamSynchronize(ctx->stream));
   const SheetDesc &d = ctx->sd[sheet];
-  const int m = d.rows * d.cols, M = ctx->nnodes;
-  std::vector<double> pos((size_t)3 * m), frc((size_t)NF_COUNT * m);
-  for (int a = 0; a < 3; ++a)
-    HIPCHK(hipMemcpy(pos.data() + (size_t)a * m, ctx->ib.pos + (size_t)a * M + d.off, sizeof(double) * m,
-                     hipMemcpyDeviceToHost));
-  for (int a = 0; a < NF_COUNT; ++a)
-    HIPCHK(hipMemcpy(frc.data() + (size_t)a * m, ctx->ib.frc + (size_t)a * M + d.off, sizeof(double) * m,
-                     hipMemcpyDeviceToHost));
-  for (int k = 0; k < m; ++k) {
-    double *r = out + (size_t)12 * k;
-    for (int a = 0; a < 3; ++a) r[a] = pos[(size_t)a * m + k];
-    for (int a = 0; a < NF_COUNT; ++a) r[3 + a] = frc[(size_t)a * m + k];
-  }
+  const int m = d.rows * d.cols;
+  double *io = ctx->d_io + 12 * (size_t)d.off;
+  RCHK(launch_pack_fibers(ctx->ib, d.off, m, io, ctx->stream));
+  HIPCHK(hipMemcpyAsync(out, io, sizeof(double) * 12 * m, hipMemcpyDeviceToHost, ctx->stream));
+  HIPCHK(hipStreamSynchronize(ctx->stream));
   return LBMIB_OK;
 }
 

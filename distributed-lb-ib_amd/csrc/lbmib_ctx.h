@@ -39,6 +39,7 @@ struct lbmib_ctx {
   double *d_ref = nullptr;   // reference populations of the deviation forms
   uint32_t *d_rowtab = nullptr;  // row source table of the buffer-addressed fused kernel
   size_t mat_bytes = 0;
+  double *d_io = nullptr;    // [nodes][12]: the sheets' nodes as the caller lays them out
   hipStream_t stream = nullptr;
   int time = 1;
   int init_bits = 0;  // 1: DF0, 2: df1, 4: inout

@@ -268,6 +268,10 @@ int launch_fiber(const IBState &ib, const Geometry &g, int mask, int slot, hipSt
 int launch_gather(int prec, const IBState &ib, const Geometry &g, int slot, void *F, hipStream_t s);
 int launch_move(int prec, const IBState &ib, const Geometry &g, const void *f, const void *F,
                 const FluidConsts<double> &c, int reset_slot, int ntiles, hipStream_t s);
+// A sheet's m nodes from off on, between the node arrays and the caller's
+// order: buf[m][12] position and the three forces; buf[m][3] positions.
+int launch_pack_fibers(const IBState &ib, int off, int m, double *buf, hipStream_t s);
+int launch_unpack_positions(const IBState &ib, int off, int m, const double *buf, hipStream_t s);
 int launch_ib_reset(const IBState &ib, int reset_bins, int reset_slot_mask, hipStream_t s);
 
 }  // namespace lbmib
