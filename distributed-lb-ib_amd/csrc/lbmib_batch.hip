@@ -37,7 +37,6 @@ struct BatchGroup {
   BatchDesc *d_desc = nullptr;
   int *d_map[kMapCount] = {};
   int nblk[kMapCount] = {};
-  int mcap_max = 0;              // largest gather candidate capacity of the group
   hipStream_t stream = nullptr;  // the batch stream for group 0
   hipEvent_t ev_fluid = nullptr; // last fused launch of the group done
 };
@@ -108,7 +107,6 @@ static void free_group(BatchGroup &g) {
   if (g.d_desc) (void)hipFree(g.d_desc);
   g.d_desc = nullptr;
   g.members.clear();
-  g.mcap_max = 0;
 }
 
 // Block tables of every batched launch of group g for the current tile shape.
@@ -158,10 +156,7 @@ static int build_groups(lbmib_batch *b) {
     BatchGroup &g = b->grp[k];
     std::sort(g.members.begin(), g.members.end());
     std::vector<BatchDesc> d;
-    for (int i : g.members) {
-      d.push_back(b->desc[i]);
-      g.mcap_max = std::max(g.mcap_max, b->desc[i].mcap);
-    }
+    for (int i : g.members) d.push_back(b->desc[i]);
     if (hipMalloc((void **)&g.d_desc, sizeof(BatchDesc) * d.size()) != hipSuccess) return LBMIB_ERR_ALLOC;
     HIPCHK(hipMemcpy(g.d_desc, d.data(), sizeof(BatchDesc) * d.size(), hipMemcpyHostToDevice));
     g.stream = k == 0 ? b->stream : b->stream2;
@@ -355,7 +350,7 @@ static int batch_steps(lbmib_batch *b, int nsteps, hipEvent_t e0, hipEvent_t e1,
       BatchGroup &g = b->grp[gi];
       hipStream_t st = g.stream;
       RCHK(launch_fiber_batch(g.d_desc, g.d_map[kMapFiber], g.nblk[kMapFiber], slot, st));
-      RCHK(launch_gather_batch(b->prec, g.d_desc, g.d_map[kMapGather], g.nblk[kMapGather], slot, g.mcap_max, st));
+      RCHK(launch_gather_batch(b->prec, g.d_desc, g.d_map[kMapGather], g.nblk[kMapGather], slot, st));
       // fused launches alternate: A(t) after B(t-1), B(t) after A(t)
       if (G > 1 && (gi > 0 || k > 0)) HIPCHK(hipStreamWaitEvent(st, b->grp[(gi + G - 1) % G].ev_fluid, 0));
       if (kev) HIPCHK(hipEventRecord(kev[2 * (k * G + gi)], st));

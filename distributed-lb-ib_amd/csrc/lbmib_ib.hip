@@ -1,11 +1,11 @@
 // lbmib_ib.hip -- immersed-boundary kernels for gfx950.
 //
 // Per step (the order of do_thread, lbm_ib.c:3124-3412):
-//   k_fiber        four lanes per fiber node: bending, stretching and
-//                  elastic force (FP64) on one, the node's 4-point-delta
-//                  support start floor(X-2)+1 and 1+cos(pi r/2) factors on
-//                  one lane per axis; its (y,z) bin and the sheet's support
-//                  box.  One launch covers every sheet.
+//   k_fiber        five waves per 64 fiber nodes: bending, stretching and
+//                  elastic force (FP64) on two, the nodes' 4-point-delta
+//                  support starts floor(X-2)+1 and 1+cos(pi r/2) factors on
+//                  one wave per axis; their (y,z) bins and the sheets' support
+//                  boxes.  One launch covers every sheet.
 //   k_gather       cell-owned force spreading: each workgroup owns a 4x4
 //                  (y,z) column tile of a sheet's support box, loads the
 //                  candidate node ids of the 2x2 bins that can reach it into
@@ -80,8 +80,6 @@ __device__ __forceinline__ void stretch_w(const double W[3][5], int j, int C, do
   }
 }
 
-// Warp-level min/max so that only one lane per wave touches the shared
-// support box (same-address atomics from every node serialise in L2).
 __device__ __forceinline__ int wave_min(int v) {
   for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
   return v;
@@ -91,52 +89,135 @@ __device__ __forceinline__ int wave_max(int v) {
   return v;
 }
 
-// Four lanes per node (a quad of consecutive lanes): lane 0 of the quad
-// computes the node forces, lane 1 + d the support start and the four delta
-// factors along axis d, so that the FP64 force and cosine chains run side
-// by side.  The quad exchanges the starts by lane shuffles for the node's
-// validity, bin entry and support box.  Every value is the same expression
-// as for one lane per node.
+// The bending and stretching force of one line through node n, from the
+// line's neighbourhood of the node: element j of C, neighbours step apart.
+__device__ __forceinline__ void line_force(const double *__restrict__ line, long M, int j, int C, long step, double bc,
+                                           bool slip, double ds, double sc, bool quirk, double bend[3],
+                                           double str[3]) {
+  double W[3][5];
+  for (int d = 0; d < 3; ++d)
+    for (int o = -2; o <= 2; ++o) W[d][o + 2] = j + o >= 0 && j + o < C ? line[d * M + o * step] : 0.0;
+  for (int d = 0; d < 3; ++d) bend[d] = bend_w(W[d], j, C, bc, slip && d == 0);
+  stretch_w(W, j, C, ds, sc, quirk, str);
+}
+
+// Support start floor(X - 2) + 1 of a node along each axis (lbm_ib.c:1424-1429)
+// and whether it lies on the grid, tested in FP64 before the conversion: a NaN
+// or a value beyond the int range (which the conversion would turn into 0 or
+// INT_MAX) fails.
+__device__ __forceinline__ bool support_start(const Geometry &g, const double *__restrict__ p, long M, int st[3]) {
+  const int dim[3] = {g.nx, g.ny, g.nz};
+  bool ok = true;
+  for (int a = 0; a < 3; ++a) {
+    const double sa = floor(p[a * M] / 1.0 - 2) + 1;
+    const bool in = sa >= 0.0 && sa + 3.0 < (double)dim[a];
+    st[a] = in ? (int)sa : INT_MAX;
+    ok = ok && in;
+  }
+  return ok;
+}
+
+// Five waves per 64 nodes, lane = node: wave 0 the row line's forces, wave 1
+// the column line's, wave 2 + d the support start and the four delta factors
+// along axis d.  The kernel is a chain of latencies (a sheet of 26 x 26 nodes
+// is 11 blocks), so its parts -- two FP64 square-root and divide chains, three
+// of cosines, the bin's atomic -- run side by side on waves of their own
+// instead of one after the other on masked lanes of one wave: 26 x 26 nodes 9.3
+// -> 6.6 us, two sheets of 128 x 128 20.6 -> 11.1.
+// Every value is the same expression as for one lane per node.
 __device__ __forceinline__ void fiber_body(const IBState &ib, const Geometry &g, int mask, int slot, int bid,
                                            int nblk) {
-  const int t = bid * blockDim.x + threadIdx.x;
-  const int n = t >> 2, role = t & 3;
+  __shared__ double s_col[6][64];  // the column line's forces
+  const int lane = threadIdx.x & 63, role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = bid * 64 + lane;
   const bool live = n < ib.nnodes;
   const int M = ib.nnodes;
   const double *__restrict__ pos = ib.pos;
   double *__restrict__ frc = ib.frc;
-  int s = 0;
-  bool ok = false;
-  int st[3] = {INT_MAX, INT_MAX, INT_MAX};
-  if (live) s = find_sheet(ib, n);
-  if (live && role == 0 && (mask & (FK_BEND | FK_STRETCH | FK_ELASTIC))) {
-    const SheetDesc sd = ib.sheets[s];
-    const int k = n - sd.off, i = k / sd.cols, j = k % sd.cols;
-    const bool quirk = ib.quirks != 0;
-    // the node's row (along cols) and column (along rows) neighbourhoods,
-    // loaded once
-    double Wr[3][5], Wc[3][5];
-    for (int d = 0; d < 3; ++d) {
-      const double *line = pos + (long)d * M + sd.off;
-      for (int o = -2; o <= 2; ++o) {
-        const int jj = j + o, ii = i + o;
-        Wr[d][o + 2] = (jj >= 0 && jj < sd.cols) ? line[(long)i * sd.cols + jj] : 0.0;
-        Wc[d][o + 2] = (ii >= 0 && ii < sd.rows) ? line[(long)ii * sd.cols + j] : 0.0;
-      }
+  int *box = ib.box + slot * kMaxSheets * 6;
+  const int s = live ? find_sheet(ib, n) : 0;
+  double bend[3] = {0, 0, 0}, str[3] = {0, 0, 0};
+  if (role < 2) {
+    if (live && (mask & (FK_BEND | FK_STRETCH | FK_ELASTIC))) {
+      const SheetDesc sd = ib.sheets[s];
+      const int k = n - sd.off, i = k / sd.cols, j = k % sd.cols;
+      const bool quirk = ib.quirks != 0;
+      if (role == 0) line_force(pos + n, M, j, sd.cols, 1, sd.bend_c, quirk, sd.ds1, sd.str_row_c, quirk, bend, str);
+      else line_force(pos + n, M, i, sd.rows, sd.cols, sd.bend_c, false, sd.ds2, sd.str_col_c, quirk, bend, str);
     }
-    double bend[3] = {0, 0, 0}, str[3] = {0, 0, 0};
-    if (mask & (FK_BEND | FK_ELASTIC)) {
+    if (role == 1)
       for (int d = 0; d < 3; ++d) {
-        const double r = bend_w(Wr[d], j, sd.cols, sd.bend_c, quirk && d == 0);
-        const double c = bend_w(Wc[d], i, sd.rows, sd.bend_c, false);
-        bend[d] = r + c;  // row pass '=', column pass '+=' (lbm_ib.c:1070)
+        s_col[d][lane] = bend[d];
+        s_col[3 + d][lane] = str[d];
+      }
+  } else if (mask & FK_PREP) {
+    const int d = role - 2;
+    int st[3] = {INT_MAX, INT_MAX, INT_MAX};
+    const bool ok = live && support_start(g, pos + n, M, st);
+    const double Xd = live ? pos[(long)d * M + n] : 0.0;
+    if (live && !ok && d == 0) {
+      // the reference exits here (lbm_ib.c:1458-1466); latch the error and
+      // leave the node out of spreading and moving.
+      atomicOr(ib.err, DERR_FIBER_OOB);
+      ib.start[n] = -1;
+    }
+    const int std_ = d == 0 ? st[0] : (d == 1 ? st[1] : st[2]);
+    // the bin's slot is asked for before the cosines and used after them
+    int bin = 0, slot_in_bin = 0;
+    if (ok && d == 0) {
+      bin = (st[1] >> 2) * ib.nbz + (st[2] >> 2);
+      slot_in_bin = atomicAdd(&ib.bin_count[bin], 1);
+    }
+    // The sheets' support boxes along axis d: wave min/max of each sheet in the
+    // wave (nodes are in sheet order), then one lane's atomic min/max into the
+    // slot, which the previous move reset to empty; both are order-independent,
+    // so the box is deterministic.  The six values share a cache line, which
+    // takes the atomics of all blocks in turn (7 ns each: 20 us for 512
+    // blocks), so a wave first takes the box of 8 x 8 sample nodes of the sheet,
+    // the same for every block: block 0 adds that one, and a wave its own only
+    // where it reaches beyond.
+    const int s_hi = wave_max(s);
+    for (int k = __builtin_amdgcn_readfirstlane(s); k <= s_hi; ++k) {
+      const SheetDesc &sd = ib.sheets[k];
+      int t[3];
+      const bool tok = support_start(
+          g, pos + sd.off + (lane / 8 * (sd.rows - 1) / 7) * sd.cols + lane % 8 * (sd.cols - 1) / 7, M, t);
+      const int td = d == 0 ? t[0] : (d == 1 ? t[1] : t[2]);
+      int lo = wave_min(ok && s == k ? std_ : INT_MAX), hi = wave_max(ok && s == k ? std_ : INT_MIN);
+      const int tlo = wave_min(tok ? td : INT_MAX), thi = wave_max(tok ? td : INT_MIN);
+      int *b = box + k * 6 + 2 * d;
+      // sd.off lies in the sheet's first block
+      const bool first = bid == sd.off / 64;
+      if (first) {
+        lo = min(lo, tlo);
+        hi = max(hi, thi);
+      }
+      if (lane == 0 && lo <= hi) {
+        if (first || lo < tlo) atomicMin(b, lo);
+        if (first || hi > thi) atomicMax(b + 1, hi + 3);
       }
     }
-    if (mask & (FK_STRETCH | FK_ELASTIC)) {
-      double r[3], c[3];
-      stretch_w(Wr, j, sd.cols, sd.ds1, sd.str_row_c, quirk, r);
-      stretch_w(Wc, i, sd.rows, sd.ds2, sd.str_col_c, quirk, c);
-      for (int d = 0; d < 3; ++d) str[d] = r[d] + c[d];
+    if (ok) {
+      // 1 + cos(pi r / 2) at r = (start + a) - X, a = 0..3, each cosine
+      // evaluated as the reference does (lbm_ib.c:1456, :2670-2673)
+      const double cpi = kRefPi / (2.0 * 1.0);
+      ib.start[d * (long)M + n] = std_;
+      for (int a = 0; a < 4; ++a) {
+        const double r = 1.0 * (std_ + a) - Xd;
+        ib.wgt[(4 * d + a) * (long)M + n] = 1.0e0 + cos(cpi * r);
+      }
+      if (d == 0) {
+        if (slot_in_bin < ib.cap) ib.bin_list[(long)bin * ib.cap + slot_in_bin] = make_int4(n, st[0], st[1], st[2]);
+        else atomicOr(ib.err, DERR_BIN_OVERFLOW);
+      }
+    }
+  }
+  __syncthreads();
+  if (role == 0 && live) {
+    // row pass '=', column pass '+=' (lbm_ib.c:1070)
+    for (int d = 0; d < 3; ++d) {
+      bend[d] = bend[d] + s_col[d][lane];
+      str[d] = str[d] + s_col[3 + d][lane];
     }
     if (mask & FK_BEND)
       for (int d = 0; d < 3; ++d) frc[(NF_BX + d) * (long)M + n] = bend[d];
@@ -151,89 +232,12 @@ __device__ __forceinline__ void fiber_body(const IBState &ib, const Geometry &g,
       }
     }
   }
-  if (mask & FK_PREP) {
-    // lane 1 + d: support start floor(X - 2) + 1 along axis d
-    // (lbm_ib.c:1424-1429) and whether it lies on the grid
-    const int d = role - 1;
-    int sdv = INT_MAX, okd = 1;
-    double Xd = 0.0;
-    if (live && role > 0) {
-      Xd = pos[(long)d * M + n];
-      const int dim = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
-      // tested in FP64 before the conversion: a NaN or a value beyond the
-      // int range (which the conversion would turn into 0 or INT_MAX) fails
-      const double sdd = floor(Xd / 1.0 - 2) + 1;
-      okd = sdd >= 0.0 && sdd + 3.0 < (double)dim;
-      if (okd) sdv = (int)sdd;
-    }
-    const int q0 = (threadIdx.x & 63) & ~3;  // the quad's lane 0 in the wave
-    for (int a = 0; a < 3; ++a) st[a] = __shfl(sdv, q0 + 1 + a, 64);
-    const int okq = __shfl(okd, q0 + 1, 64) & __shfl(okd, q0 + 2, 64) & __shfl(okd, q0 + 3, 64);
-    ok = live && okq;
-    if (live && !ok) {
-      // the reference exits here (lbm_ib.c:1458-1466); latch the error and
-      // leave the node out of spreading and moving.
-      if (role == 0) {
-        atomicOr(ib.err, DERR_FIBER_OOB);
-        ib.start[n] = -1;
-      }
-    } else if (live && role > 0) {
-      // 1 + cos(pi r / 2) at r = (start + a) - X, a = 0..3, each cosine
-      // evaluated as the reference does (lbm_ib.c:1456, :2670-2673)
-      const double cpi = kRefPi / (2.0 * 1.0);
-      ib.start[d * (long)M + n] = sdv;
-      for (int a = 0; a < 4; ++a) {
-        const double r = 1.0 * (sdv + a) - Xd;
-        ib.wgt[(4 * d + a) * (long)M + n] = 1.0e0 + cos(cpi * r);
-      }
-    } else if (live) {
-      const int b = (st[1] >> 2) * ib.nbz + (st[2] >> 2);
-      const int slot_in_bin = atomicAdd(&ib.bin_count[b], 1);
-      if (slot_in_bin < ib.cap) ib.bin_list[(long)b * ib.cap + slot_in_bin] = make_int4(n, st[0], st[1], st[2]);
-      else atomicOr(ib.err, DERR_BIN_OVERFLOW);
-    }
-  }
   if (!(mask & FK_PREP)) return;  // uniform over the grid
-  // Support box of each sheet: wave min/max, LDS combine per block, then one
-  // global atomic min/max per block and coordinate into the box slot (reset
-  // to empty by the previous move); min/max are order-independent, so the
-  // box is deterministic.  The last block to finish derives the band boxes.
+  const int nk = ib.nsheets * 6;
+  if (!ib.band) return;  // no band boxes wanted (unsplit steps)
+  // the last block to finish derives the band boxes
   __shared__ int sbox[kMaxSheets * 6];
   __shared__ int s_last;
-  for (int t = threadIdx.x; t < kMaxSheets * 6; t += blockDim.x) sbox[t] = (t & 1) ? INT_MIN : INT_MAX;
-  __syncthreads();
-  const int s_lo = __shfl(s, 0, 64);
-  const bool uniform = __all(!live || s == s_lo);
-  const int lo[3] = {ok ? st[0] : INT_MAX, ok ? st[1] : INT_MAX, ok ? st[2] : INT_MAX};
-  const int hi[3] = {ok ? st[0] + 3 : INT_MIN, ok ? st[1] + 3 : INT_MIN, ok ? st[2] + 3 : INT_MIN};
-  if (uniform) {
-    int rlo[3], rhi[3];
-    for (int d = 0; d < 3; ++d) {
-      rlo[d] = wave_min(lo[d]);
-      rhi[d] = wave_max(hi[d]);
-    }
-    if ((threadIdx.x & 63) == 0 && rlo[0] != INT_MAX)
-      for (int d = 0; d < 3; ++d) {
-        atomicMin(&sbox[s_lo * 6 + 2 * d], rlo[d]);
-        atomicMax(&sbox[s_lo * 6 + 2 * d + 1], rhi[d]);
-      }
-  } else if (ok) {
-    for (int d = 0; d < 3; ++d) {  // a wave across a sheet seam
-      atomicMin(&sbox[s * 6 + 2 * d], lo[d]);
-      atomicMax(&sbox[s * 6 + 2 * d + 1], hi[d]);
-    }
-  }
-  __syncthreads();
-  int *box = ib.box + slot * kMaxSheets * 6;
-  const int nk = ib.nsheets * 6;
-  for (int t = threadIdx.x; t < nk; t += blockDim.x) {
-    if (t & 1) {
-      if (sbox[t] != INT_MIN) atomicMax(box + t, sbox[t]);
-    } else if (sbox[t] != INT_MAX) {
-      atomicMin(box + t, sbox[t]);
-    }
-  }
-  if (!ib.band) return;  // no band boxes wanted (unsplit steps)
   __threadfence();
   __syncthreads();
   if (threadIdx.x == 0) s_last = atomicAdd(ib.done, 1u) == (unsigned)(nblk - 1);
@@ -290,27 +294,32 @@ __device__ __forceinline__ bool tile_of(const IBState &ib, int slot, int w, int 
   return false;
 }
 
-constexpr int kGatherMaxCand = 384;    // candidates whose support meets the tile: 13.5 KB of LDS
-constexpr int kGatherStage = 128;      // candidates whose delta factors / forces are staged: 15 KB
+constexpr int kGatherMaxCand = 384;         // candidates whose support meets the tile: 13.8 KB of LDS
+constexpr int kGatherEntries = 2 * kGatherThreads;  // bin entries taken at once: two per thread
+constexpr int kGatherStage = 96;            // candidates whose delta factors / forces are staged
 
-// LDS of a gather block for mcap candidates (the layout of gather_body).
-static size_t gather_shm_bytes(int mcap) {
-  return sizeof(double) * 15 * (size_t)kGatherStage + sizeof(int) * (9 * (size_t)mcap + 4);
-}
+// LDS of a gather block: the staged candidates' factors, forces, starts and
+// ids and a zero entry, and the entries' ids (18.6 KB, so that 8 blocks share a CU), or in their place the starts and
+// ids of up to kGatherMaxCand candidates, raw and sorted (the layout of
+// gather_body).
+constexpr size_t kGatherShm =
+    sizeof(double) * (15 * (kGatherStage + 1) + 1) + sizeof(int) * (4 * (kGatherStage + 1) + kGatherEntries);
+static_assert(kGatherShm >= sizeof(int) * (9 * (size_t)kGatherMaxCand + 4), "the unstaged candidates fit");
 
 template <class FT>
 __device__ __forceinline__ void gather_body(const IBState &ib, const Geometry &g, int slot, FT *__restrict__ F, int mcap,
                                             int bid, int nblk) {
-  // LDS: delta factors and forces of the staged candidates, the sorted
-  // candidates' support starts and ids (x, y, z, id), the raw candidates'
-  // starts and the raw candidate ids (padded to a multiple of 4 for the
-  // 16-byte reads of the rank sort)
   extern __shared__ __attribute__((aligned(16))) double smem_d[];
-  double *sw = smem_d;                      // [kGatherStage][12] delta factors
-  double *se = sw + kGatherStage * 12;      // [kGatherStage][3] elastic force
-  int4 *sst = reinterpret_cast<int4 *>(se + kGatherStage * 3);
-  int4 *rst = sst + mcap;  // support starts of the raw candidates
-  int *raw = reinterpret_cast<int *>(rst + mcap);
+  // staged: the sorted candidates' delta factors, forces, support starts and
+  // ids (x, y, z, id), and the ids of the entries that are candidates
+  double *sw = smem_d;                        // [kGatherStage + 1][12] delta factors
+  double *se = sw + (kGatherStage + 1) * 12;  // [kGatherStage + 1][3] elastic force
+  int *raw = reinterpret_cast<int *>(smem_d + (kGatherStage + 1) * 15 + 1);
+  int4 *sst = reinterpret_cast<int4 *>(raw + kGatherEntries);
+  // not staged: the raw candidates' starts, the sorted ones, and the raw ids
+  // (padded to a multiple of 4 for the 16-byte reads of the rank sort)
+  int4 *rst = reinterpret_cast<int4 *>(smem_d), *ust = rst + mcap;
+  int *uraw = reinterpret_cast<int *>(ust + mcap);
   __shared__ int s_tot;
   const int M = ib.nnodes;
   const double cf = 1.0 / (64.0 * 1.0 * 1.0 * 1.0);  // lbm_ib.c:1357
@@ -334,10 +343,11 @@ __device__ __forceinline__ void gather_body(const IBState &ib, const Geometry &g
     // a node with support start j0 reaches rows j0..j0+3, so tile rows
     // kTile*ty .. kTile*ty+kTile-1 need j0 in [kTile*ty-3, kTile*ty+kTile-1]:
     // bins kTileBins*ty-1 .. kTileBins*ty+kTileBins-1.  Of those, only the
-    // nodes whose x support [i0, i0+3] meets the box's x range reach a cell
-    // of the tile (the others, e.g. of another sheet in the same (y, z)
-    // bins, add nothing); they are gathered in any order and rank-sorted
-    // below, so each cell still sums its contributions in node order.
+    // nodes whose support meets the box's x range and the tile's rows reach a
+    // cell of the tile (49 of 64 at unit spacing; the others, e.g. of another
+    // sheet in the same (y, z) bins, add nothing, and are left out where their
+    // number is small); they are gathered in any order and rank-sorted below,
+    // so each cell still sums its contributions in node order.
     // The bins' counts are loaded together, then every lane takes candidates
     // of the concatenated bin lists, so that the list reads of all bins are
     // in flight at once.
@@ -358,100 +368,172 @@ __device__ __forceinline__ void gather_body(const IBState &ib, const Geometry &g
       cnt[k] = seen;  // becomes the bin's offset in the concatenation
       seen += c;
     }
-    if (threadIdx.x == 0) s_tot = 0;
-    __syncthreads();
-    for (int e = threadIdx.x; e < seen; e += blockDim.x) {
+    const auto entry = [&](int e) {
       int bin = bins[0], off = 0;  // the last bin whose offset is <= e (empty bins share the next offset)
 #pragma unroll
       for (int j = 1; j < kNB; ++j)
         if (e >= cnt[j]) { bin = bins[j]; off = cnt[j]; }
-      const int4 q = ib.bin_list[(long)bin * ib.cap + (e - off)];  // id, support start
-      if (q.y <= x1 && q.y + 3 >= x0) {
-        const int k = atomicAdd(&s_tot, 1);
-        if (k < mcap) {  // LDS holds up to mcap candidates; more is reported
-          raw[k] = q.x;
-          rst[k] = make_int4(q.y, q.z, q.w, q.x);
+      return ib.bin_list[(long)bin * ib.cap + (e - off)];  // id, support start
+    };
+    const auto meets_x = [&](const int4 &q) { return q.y <= x1 && q.y + 3 >= x0; };
+    bool staged = seen <= kGatherEntries;
+    int tot = 0;
+    if (staged) {
+      // up to two entries per thread, the candidates' factors and forces read
+      // into registers while the ranks (ascending node id: the order of
+      // (sheet, row, col)) are counted
+      constexpr int kPer = kGatherEntries / kGatherThreads;
+      int4 q[kPer];
+      bool cand[kPer];
+      double w[kPer][12], f[kPer][3];
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        const int e = threadIdx.x + u * kGatherThreads;
+        q[u] = make_int4(INT_MAX, 0, 0, 0);
+        if (e < seen) q[u] = entry(e);
+      }
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        const int e = threadIdx.x + u * kGatherThreads;
+        cand[u] = e < seen && meets_x(q[u]) && q[u].z + 3 >= kTile * ty && q[u].w + 3 >= kTile * tz;
+        raw[e] = cand[u] ? q[u].x : INT_MAX;
+        if (cand[u]) {
+          for (int a = 0; a < 12; ++a) w[u][a] = ib.wgt[a * (long)M + q[u].x];
+          for (int a = 0; a < 3; ++a) f[u][a] = ib.frc[(NF_EX + a) * (long)M + q[u].x];
         }
       }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && s_tot > mcap) atomicOr(ib.err, DERR_BIN_OVERFLOW);
-    const int tot = min(s_tot, mcap), tot4 = (tot + 3) & ~3;
-    const bool staged = tot <= kGatherStage;
-    if ((int)threadIdx.x < tot4 - tot) {
-      // padding up to a multiple of 4: an id above every id for the rank
-      // sort; a support start far from every cell and zero factors and
-      // forces for the unrolled sum
-      const int k = tot + threadIdx.x;
-      raw[k] = INT_MAX;
+      __syncthreads();
+      int r[kPer] = {};
+      const int4 *raw4 = reinterpret_cast<const int4 *>(raw);
+#pragma unroll 4
+      for (int k = 0; k < (seen + 3) / 4; ++k) {
+        const int4 p = raw4[k];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) r[u] += (p.x < q[u].x) + (p.y < q[u].x) + (p.z < q[u].x) + (p.w < q[u].x);
+        tot += (p.x != INT_MAX) + (p.y != INT_MAX) + (p.z != INT_MAX) + (p.w != INT_MAX);
+      }
+      staged = tot <= kGatherStage;
       if (staged) {
-        sst[k] = make_int4(-(1 << 28), -(1 << 28), -(1 << 28), 0);
-        for (int a = 0; a < 12; ++a) sw[k * 12 + a] = 0.0;
-        for (int a = 0; a < 3; ++a) se[k * 3 + a] = 0.0;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+          if (cand[u]) {
+            sst[r[u]] = make_int4(q[u].y, q[u].z, q[u].w, q[u].x);
+            for (int a = 0; a < 12; ++a) sw[r[u] * 12 + a] = w[u][a];
+            for (int a = 0; a < 3; ++a) se[r[u] * 3 + a] = f[u][a];
+          }
+        // the zero entry: a support start far from every cell, zero factors
+        // and forces
+        if (threadIdx.x == 0) sst[kGatherStage] = make_int4(-(1 << 28), -(1 << 28), -(1 << 28), 0);
+        if (threadIdx.x < 12) sw[kGatherStage * 12 + threadIdx.x] = 0.0;
+        if (threadIdx.x < 3) se[kGatherStage * 3 + threadIdx.x] = 0.0;
+      } else {
+        __syncthreads();  // the ids' readers are done
       }
     }
-    __syncthreads();
-    // rank sort (node ids are distinct): ascending (sheet, row, col) order
-    const int4 *raw4 = reinterpret_cast<const int4 *>(raw);
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-      const int v = raw[e];
-      int r = 0;
-      for (int k = 0; k < tot4 / 4; ++k) {
-        const int4 q = raw4[k];
-        r += (q.x < v) + (q.y < v) + (q.z < v) + (q.w < v);
+    if (!staged) {
+      if (threadIdx.x == 0) s_tot = 0;
+      __syncthreads();
+      for (int e = threadIdx.x; e < seen; e += blockDim.x) {
+        const int4 q = entry(e);
+        if (meets_x(q)) {
+          const int k = atomicAdd(&s_tot, 1);
+          if (k < mcap) {  // LDS holds up to mcap candidates; more is reported
+            uraw[k] = q.x;
+            rst[k] = make_int4(q.y, q.z, q.w, q.x);
+          }
+        }
       }
-      sst[r] = rst[e];  // starts and id
-      if (staged) {
-        for (int a = 0; a < 12; ++a) sw[r * 12 + a] = ib.wgt[a * (long)M + v];
-        for (int a = 0; a < 3; ++a) se[r * 3 + a] = ib.frc[(NF_EX + a) * (long)M + v];
+      __syncthreads();
+      if (threadIdx.x == 0 && s_tot > mcap) atomicOr(ib.err, DERR_BIN_OVERFLOW);
+      tot = min(s_tot, mcap);
+      const int tot4 = (tot + 3) & ~3;
+      if ((int)threadIdx.x < tot4 - tot) uraw[tot + threadIdx.x] = INT_MAX;  // above every id
+      __syncthreads();
+      const int4 *raw4 = reinterpret_cast<const int4 *>(uraw);
+      for (int e = threadIdx.x; e < tot; e += blockDim.x) {
+        const int v = uraw[e];
+        int r = 0;
+        for (int k = 0; k < tot4 / 4; ++k) {
+          const int4 q = raw4[k];
+          r += (q.x < v) + (q.y < v) + (q.z < v) + (q.w < v);
+        }
+        ust[r] = rst[e];  // starts and id
       }
     }
     __syncthreads();
     const int y0 = max(kTile * ty, bybox0), y1 = min(kTile * ty + kTile - 1, bybox1);
     const int z0 = max(kTile * tz, bzbox0), z1 = min(kTile * tz + kTile - 1, bzbox1);
-    const int nxs = x1 - x0 + 1, nys = y1 - y0 + 1, nzs = z1 - z0 + 1;
-    const int ncell = nxs * nys * nzs;
-    for (int e = threadIdx.x; e < ncell; e += blockDim.x) {
-      const int x = x0 + e % nxs, y = y0 + (e / nxs) % nys, z = z0 + e / (nxs * nys);
-      double ax = 0.0, ay = 0.0, az = 0.0;
-      if (staged) {
-        // branch-free over the candidates, four at a time, so that their LDS
-        // reads are all in flight together (the empty asm keeps the force
-        // reads unconditional): a candidate whose support misses the cell
-        // adds fma(0, w, a) = a (w is a finite factor read at an in-range
-        // index; a sum that starts at +0 is never -0), so each cell still
-        // adds exactly its own contributions in node order
-        for (int k = 0; k < tot4; k += 4) {
-          int4 st[4];
+    const auto put = [&](int x, int y, int z, double ax, double ay, double az) {
+      const long c0 = (long)x + (long)g.nx * ((long)y + (long)g.ny * z);
+      F[c0] = (FT)ax;
+      F[g.n + c0] = (FT)ay;
+      F[2 * g.n + c0] = (FT)az;
+    };
+    if (staged) {
+      // Eight lanes along x per (y, z) column.  A column meets 16 of the 49
+      // candidates at unit spacing: two ballots per column give the set of its
+      // candidates, whose bits its lanes walk in ascending rank, four at a
+      // time, so that their LDS reads are in flight together (every cell
+      // testing every candidate: two sheets of 128 x 128 nodes 31 us, now 26).  A
+      // candidate whose support misses the cell's x, and the zero entry that
+      // fills up the last four, add fma(0, w, a) = a (w is a finite factor read
+      // at an in-range index; a sum that starts at +0 is never -0), so each
+      // cell still adds exactly its own contributions in node order.
+      const int lane = threadIdx.x & 63, c_0 = (threadIdx.x >> 6) * 8;
+      const int4 sa = sst[lane < tot ? lane : kGatherStage], sb = sst[64 + lane < tot ? 64 + lane : kGatherStage];
+      unsigned long long m0 = 0, m1 = 0;
 #pragma unroll
-          for (int u = 0; u < 4; ++u) st[u] = sst[k + u];
-          bool hit[4];
-          double wa[4], wb[4], wc[4], ex[4], ey[4], ez[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int ix = x - st[u].x, iy = y - st[u].y, iz = z - st[u].z;
-            hit[u] = (unsigned)ix <= 3u && (unsigned)iy <= 3u && (unsigned)iz <= 3u;
-            const double *w = sw + (k + u) * 12;
-            wa[u] = w[ix & 3];
-            wb[u] = w[4 + (iy & 3)];
-            wc[u] = w[8 + (iz & 3)];
-            ex[u] = se[(k + u) * 3];
-            ey[u] = se[(k + u) * 3 + 1];
-            ez[u] = se[(k + u) * 3 + 2];
-          }
-          asm volatile("" : "+v"(ex[0]), "+v"(ey[0]), "+v"(ez[0]), "+v"(ex[1]), "+v"(ey[1]), "+v"(ez[1]),
-                       "+v"(ex[2]), "+v"(ey[2]), "+v"(ez[2]), "+v"(ex[3]), "+v"(ey[3]), "+v"(ez[3]));
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const double wgt = cf * wa[u] * wb[u] * wc[u];
-            ax = fma(hit[u] ? ex[u] : 0.0, wgt, ax);
-            ay = fma(hit[u] ? ey[u] : 0.0, wgt, ay);
-            az = fma(hit[u] ? ez[u] : 0.0, wgt, az);
-          }
+      for (int j = 0; j < 8; ++j) {
+        const int yy = kTile * ty + ((c_0 + j) & 3), zz = kTile * tz + ((c_0 + j) >> 2);
+        const unsigned long long b0 = __ballot((unsigned)(yy - sa.y) <= 3u && (unsigned)(zz - sa.z) <= 3u);
+        const unsigned long long b1 = __ballot((unsigned)(yy - sb.y) <= 3u && (unsigned)(zz - sb.z) <= 3u);
+        if (lane >> 3 == j) {
+          m0 = b0;
+          m1 = b1;
         }
-      } else {
+      }
+      const int y = kTile * ty + ((threadIdx.x >> 3) & 3), z = kTile * tz + (threadIdx.x >> 5);
+      if (y >= y0 && y <= y1 && z >= z0 && z <= z1)
+        for (int x = x0 + (int)(threadIdx.x & 7); x <= x1; x += 8) {
+          double ax = 0.0, ay = 0.0, az = 0.0;
+          for (int h = 0; h < 2; ++h)
+            for (unsigned long long m = h ? m1 : m0; m;) {
+              int4 st[4];
+              int r[4];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                r[u] = m ? 64 * h + __builtin_ctzll(m) : kGatherStage;
+                m &= m - 1;
+                st[u] = sst[r[u]];
+              }
+              double wgt[4], ex[4], ey[4], ez[4];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                const int ix = x - st[u].x;
+                const bool hit = (unsigned)ix <= 3u;
+                const double *w = sw + r[u] * 12, *e = se + r[u] * 3;
+                wgt[u] = cf * w[ix & 3] * w[4 + ((y - st[u].y) & 3)] * w[8 + ((z - st[u].z) & 3)];
+                ex[u] = hit ? e[0] : 0.0;
+                ey[u] = hit ? e[1] : 0.0;
+                ez[u] = hit ? e[2] : 0.0;
+              }
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                ax = fma(ex[u], wgt[u], ax);
+                ay = fma(ey[u], wgt[u], ay);
+                az = fma(ez[u], wgt[u], az);
+              }
+            }
+          put(x, y, z, ax, ay, az);
+        }
+    } else {
+      const int nxs = x1 - x0 + 1, nys = y1 - y0 + 1, nzs = z1 - z0 + 1;
+      const int ncell = nxs * nys * nzs;
+      for (int e = threadIdx.x; e < ncell; e += blockDim.x) {
+        const int x = x0 + e % nxs, y = y0 + (e / nxs) % nys, z = z0 + e / (nxs * nys);
+        double ax = 0.0, ay = 0.0, az = 0.0;
         for (int k = 0; k < tot; ++k) {
-          const int4 st = sst[k];
+          const int4 st = ust[k];
           const int ix = x - st.x, iy = y - st.y, iz = z - st.z;
           if ((unsigned)ix > 3u || (unsigned)iy > 3u || (unsigned)iz > 3u) continue;
           const int n = st.w;
@@ -461,11 +543,8 @@ __device__ __forceinline__ void gather_body(const IBState &ib, const Geometry &g
           ay = fma(ib.frc[NF_EY * (long)M + n], wgt, ay);
           az = fma(ib.frc[NF_EZ * (long)M + n], wgt, az);
         }
+        put(x, y, z, ax, ay, az);
       }
-      const long c0 = (long)x + (long)g.nx * ((long)y + (long)g.ny * z);
-      F[c0] = (FT)ax;
-      F[g.n + c0] = (FT)ay;
-      F[2 * g.n + c0] = (FT)az;
     }
     __syncthreads();
   }
@@ -638,7 +717,8 @@ __global__ void __launch_bounds__(kMoveThreads) k_move(IBState ib, Geometry g, i
 
 constexpr int kMvThreads = 256;
 constexpr int kMvCells = 1024;  // cells of u per slab: 24 KB
-static_assert(3 * kMvNodes * kMvNodes <= 64, "the tile's lanes fit in one wave");
+constexpr int kMvLanes = 3 * kMvNodes * kMvNodes;  // (node, component) lanes
+constexpr int kMvWaves = (kMvLanes + 63) / 64;
 
 template <int P>
 __global__ void __launch_bounds__(kMvThreads)
@@ -646,7 +726,7 @@ __global__ void __launch_bounds__(kMvThreads)
                  const typename Traits<P>::FT *__restrict__ F, double u0x, double u0y, double u0z, double gz,
                  const double *__restrict__ ref, typename Traits<P>::T b1, typename Traits<P>::T b2, int reset_slot) {
   __shared__ double su[3][kMvCells];
-  __shared__ int s_box[6];
+  __shared__ int s_box[kMvWaves][6];
   const int tid = threadIdx.x;
   const int M = ib.nnodes;
   {
@@ -673,7 +753,7 @@ __global__ void __launch_bounds__(kMvThreads)
   const int pr = tid / 3, comp = tid % 3;
   const int i = (w / tcols) * kMvNodes + pr / kMvNodes, j = (w % tcols) * kMvNodes + pr % kMvNodes;
   const int n = sd.off + i * sd.cols + j;
-  bool act = tid < 3 * kMvNodes * kMvNodes && i < sd.rows && j < sd.cols;
+  bool act = tid < kMvLanes && i < sd.rows && j < sd.cols;
   int st[3] = {0, 0, 0};
   double wx[4], wy[4], wz[4], X = 0.0;
   if (act) {
@@ -688,22 +768,29 @@ __global__ void __launch_bounds__(kMvThreads)
     X = ib.pos[(long)comp * M + n];
     act = st[0] >= 0;  // start -1: support off the grid (error latched), not moved
   }
-  if (tid < 64) {
+  if (tid < 64 * kMvWaves) {
     int lo[3], hi[3];
     for (int d = 0; d < 3; ++d) {
       lo[d] = wave_min(act ? st[d] : INT_MAX);
       hi[d] = wave_max(act ? st[d] + 3 : INT_MIN);
     }
-    if (tid == 0)
+    if ((tid & 63) == 0)
       for (int d = 0; d < 3; ++d) {
-        s_box[2 * d] = lo[d];
-        s_box[2 * d + 1] = hi[d];
+        s_box[tid >> 6][2 * d] = lo[d];
+        s_box[tid >> 6][2 * d + 1] = hi[d];
       }
   }
   __syncthreads();
-  const int xlo = s_box[0], xhi = s_box[1], ylo = s_box[2], zlo = s_box[4];
+  int bx[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    bx[k] = s_box[0][k];
+#pragma unroll
+    for (int v = 1; v < kMvWaves; ++v) bx[k] = k & 1 ? max(bx[k], s_box[v][k]) : min(bx[k], s_box[v][k]);
+  }
+  const int xlo = bx[0], xhi = bx[1], ylo = bx[2], zlo = bx[4];
   if (xlo > xhi) return;  // no node of the tile is moved
-  const int nyr = s_box[3] - ylo + 1, nzr = s_box[5] - zlo + 1;
+  const int nyr = bx[3] - ylo + 1, nzr = bx[5] - zlo + 1;
   const double c_64 = 1.0 / (6.4e1);
   double acc = 0;
   if (nyr * nzr <= kMvCells) {
@@ -851,10 +938,9 @@ int launch_fiber(const IBState &ib, const Geometry &g, int mask, int slot, hipSt
 int launch_gather(int prec, const IBState &ib, const Geometry &g, int slot, void *F, hipStream_t s) {
   if (ib.nnodes <= 0) return LBMIB_OK;
   const int mcap = gather_mcap(ib.cap);
-  const size_t shm = gather_shm_bytes(mcap);
   const int blocks = gather_blocks(ib.nnodes);
-  if (prec == LBMIB_F64) k_gather<double><<<blocks, kGatherThreads, shm, s>>>(ib, g, slot, (double *)F, mcap);
-  else k_gather<float><<<blocks, kGatherThreads, shm, s>>>(ib, g, slot, (float *)F, mcap);
+  if (prec == LBMIB_F64) k_gather<double><<<blocks, kGatherThreads, kGatherShm, s>>>(ib, g, slot, (double *)F, mcap);
+  else k_gather<float><<<blocks, kGatherThreads, kGatherShm, s>>>(ib, g, slot, (float *)F, mcap);
   return hipGetLastError() == hipSuccess ? LBMIB_OK : LBMIB_ERR_HIP;
 }
 
@@ -949,12 +1035,10 @@ int launch_fiber_batch(const BatchDesc *d, const int *map, int nblocks, int slot
   k_fiber_batch<<<nblocks, kFiberThreads, 0, s>>>(d, map, slot);
   return hipGetLastError() == hipSuccess ? LBMIB_OK : LBMIB_ERR_HIP;
 }
-int launch_gather_batch(int prec, const BatchDesc *d, const int *map, int nblocks, int slot, int mcap_max,
-                        hipStream_t s) {
+int launch_gather_batch(int prec, const BatchDesc *d, const int *map, int nblocks, int slot, hipStream_t s) {
   if (nblocks <= 0) return LBMIB_OK;
-  const size_t shm = gather_shm_bytes(mcap_max);
-  if (prec == LBMIB_F64) k_gather_batch<double><<<nblocks, kGatherThreads, shm, s>>>(d, map, slot);
-  else k_gather_batch<float><<<nblocks, kGatherThreads, shm, s>>>(d, map, slot);
+  if (prec == LBMIB_F64) k_gather_batch<double><<<nblocks, kGatherThreads, kGatherShm, s>>>(d, map, slot);
+  else k_gather_batch<float><<<nblocks, kGatherThreads, kGatherShm, s>>>(d, map, slot);
   return hipGetLastError() == hipSuccess ? LBMIB_OK : LBMIB_ERR_HIP;
 }
 int launch_band_u_batch(int prec, const BatchDesc *d, const int *map, int nblocks, int cur_new, int slot,

@@ -129,10 +129,10 @@ struct IBState {
 
 // host-side launchers (defined in lbmib_fluid.hip / lbmib_ib.hip)
 
-// k_fiber: four lanes per node, kFiberThreads per block; each block folds its
-// nodes' support boxes into the box slot with atomic min/max.
-constexpr int kFiberThreads = 256;  // four lanes per node: 64 nodes per block
-__host__ __device__ inline int fiber_blocks(int nnodes) { return (4 * nnodes + kFiberThreads - 1) / kFiberThreads; }
+// k_fiber: five waves per 64 nodes; each wave folds its nodes' supports into
+// the box slot with atomic min/max.
+constexpr int kFiberThreads = 320;
+__host__ __device__ inline int fiber_blocks(int nnodes) { return (nnodes + 63) / 64; }
 // Grids of the other IB kernels for a sheet set of nnodes nodes (the kernels
 // stride over any further work).
 __host__ __device__ inline int gather_blocks(int nnodes) {
@@ -181,8 +181,7 @@ int box_rows_auto(const ::lbmib_ctx *ctx);
 int launch_collide_batch(int prec, const BatchDesc *d, const int *map, int nblocks, int wpb, int cur, int own,
                          int slot, int nt_mask, int rows, int box_rows_cached, hipStream_t s);
 int launch_fiber_batch(const BatchDesc *d, const int *map, int nblocks, int slot, hipStream_t s);
-int launch_gather_batch(int prec, const BatchDesc *d, const int *map, int nblocks, int slot, int mcap_max,
-                        hipStream_t s);
+int launch_gather_batch(int prec, const BatchDesc *d, const int *map, int nblocks, int slot, hipStream_t s);
 int launch_band_u_batch(int prec, const BatchDesc *d, const int *map, int nblocks, int cur_new, int slot,
                         hipStream_t s);
 int launch_move_batch(const BatchDesc *d, const int *map, int nblocks, int reset_slot, hipStream_t s);
