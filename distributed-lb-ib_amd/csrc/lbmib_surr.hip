@@ -1137,14 +1137,83 @@ int conv_fwd(const void *x, const void *w, const float *bias, const void *mask, 
 }
 
 // wt[ci][26 - t][co] = w[co][t][ci]
-__global__ void k_flip(const uint16_t *__restrict__ w, uint16_t *__restrict__ wt, int Cin, int Cout) {
-  const long n = (long)Cout * 27 * Cin;
-  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
-    const int ci = (int)(e % Cin);
-    const long r = e / Cin;
-    const int t = (int)(r % 27), co = (int)(r / 27);
-    wt[((long)ci * 27 + (26 - t)) * Cout + co] = w[e];
+// One 64 x 64 tile of one tap: rows of w come and rows of wt go in 16-byte
+// pieces through LDS (one element per lane wrote wt in 2-byte pieces, 27 Cout
+// apart: 15.3 us for 256 x 256 channels, and 83 us in a launch for each of a
+// network's 14 layers; 7.5 us now, in one launch for the list).
+constexpr int kFlipTile = 64;
+constexpr int kFlipMax = 32;  // layers per launch
+struct FlipItem {
+  const uint16_t *w;
+  uint16_t *wt;
+  int Cin, Cout, first, vec;  // first block; both pointers on 16 bytes
+};
+struct FlipList {
+  FlipItem it[kFlipMax];
+  int n;
+};
+
+static inline int flip_blocks(int Cin, int Cout) {
+  return 27 * ((Cin + kFlipTile - 1) / kFlipTile) * ((Cout + kFlipTile - 1) / kFlipTile);
+}
+
+__global__ void __launch_bounds__(256) k_flip(FlipList l) {
+  __shared__ uint16_t tile[kFlipTile][kFlipTile + 2];
+  int k = 0;
+  while (k + 1 < l.n && (int)blockIdx.x >= l.it[k + 1].first) ++k;
+  const FlipItem it = l.it[k];
+  const int Cin = it.Cin, Cout = it.Cout;
+  const int nci = (Cin + kFlipTile - 1) / kFlipTile;
+  int b = blockIdx.x - it.first;
+  const int t = b % 27;
+  b /= 27;
+  const int ci0 = b % nci * kFlipTile, co0 = b / nci * kFlipTile;
+  for (int e = threadIdx.x; e < kFlipTile * kFlipTile / 8; e += 256) {
+    const int co = e / 8, ci = e % 8 * 8;
+    if (co0 + co >= Cout || ci0 + ci >= Cin) continue;
+    const uint16_t *src = it.w + ((long)(co0 + co) * 27 + t) * Cin + ci0 + ci;
+    alignas(16) uint16_t v[8];
+    if (it.vec) {
+      *(u32x4 *)v = *(const u32x4 *)src;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = src[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tile[co][ci + j] = v[j];
   }
+  __syncthreads();
+  for (int e = threadIdx.x; e < kFlipTile * kFlipTile / 8; e += 256) {
+    const int ci = e / 8, co = e % 8 * 8;
+    if (co0 + co >= Cout || ci0 + ci >= Cin) continue;
+    uint16_t *dst = it.wt + ((long)(ci0 + ci) * 27 + (26 - t)) * Cout + co0 + co;
+    alignas(16) uint16_t v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = tile[co + j][ci];
+    if (it.vec) {
+      *(u32x4 *)dst = *(const u32x4 *)v;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) dst[j] = v[j];
+    }
+  }
+}
+
+static int flip_list(int n, const lbmib_sg_flip_item *items, hipStream_t s) {
+  for (int k0 = 0; k0 < n; k0 += kFlipMax) {
+    FlipList l;
+    l.n = n - k0 < kFlipMax ? n - k0 : kFlipMax;
+    int blocks = 0;
+    for (int k = 0; k < l.n; ++k) {
+      const lbmib_sg_flip_item &q = items[k0 + k];
+      l.it[k] = FlipItem{(const uint16_t *)q.w, (uint16_t *)q.wt, q.Cin, q.Cout, blocks,
+                         (((uintptr_t)q.w | (uintptr_t)q.wt) & 15) == 0};
+      blocks += flip_blocks(q.Cin, q.Cout);
+    }
+    k_flip<<<blocks, 256, 0, s>>>(l);
+    HIPCHK(hipGetLastError());
+  }
+  return LBMIB_OK;
 }
 
 // ----------------------------------------------------------- weight grad
@@ -1683,23 +1752,24 @@ int sq_partials(void **out) {
 //
 // One thread per (voxel, 8-channel piece); C is a multiple of 16.
 
-__global__ void k_pool2(const uint16_t *__restrict__ x, uint16_t *__restrict__ y, int D, int H, int W, int C, long n) {
-  const int P = C / 8;
-  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
-    const int q = (int)(e % P);
-    long r = e / P;
-    const int ox = (int)(r % W);
+template <class I>
+__global__ void k_pool2(const uint16_t *__restrict__ x, uint16_t *__restrict__ y, unsigned D, unsigned H, unsigned W, unsigned C, I n) {
+  const I P = C / 8;
+  for (I e = (I)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (I)gridDim.x * blockDim.x) {
+    const I q = e % P;
+    I r = e / P;
+    const I ox = r % W;
     r /= W;
-    const int oy = (int)(r % H);
+    const I oy = r % H;
     r /= H;
-    const int oz = (int)(r % D);
-    const long b = r / D;
+    const I oz = r % D;
+    const I b = r / D;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      const long iz = 2 * oz + (c >> 2), iy = 2 * oy + ((c >> 1) & 1), ix = 2 * ox + (c & 1);
-      const long v = ((b * 2 * D + iz) * 2 * H + iy) * 2 * W + ix;
-      const u32x4 val = *(const u32x4 *)(x + v * C + q * 8);
+      const I iz = 2 * oz + (c >> 2), iy = 2 * oy + ((c >> 1) & 1), ix = 2 * ox + (c & 1);
+      const I v = ((b * 2 * D + iz) * 2 * H + iy) * 2 * W + ix;
+      const u32x4 val = *(const u32x4 *)(x + (size_t)v * C + q * 8);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         acc[2 * k] += bf2f((uint16_t)(val[k] & 0xffff));
@@ -1710,7 +1780,7 @@ __global__ void k_pool2(const uint16_t *__restrict__ x, uint16_t *__restrict__ y
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       o[k] = (uint32_t)f2bf(acc[2 * k] * 0.125f) | ((uint32_t)f2bf(acc[2 * k + 1] * 0.125f) << 16);
-    *(u32x4 *)(y + e * 8) = o;
+    *(u32x4 *)(y + (size_t)e * 8) = o;
   }
 }
 
@@ -1729,89 +1799,93 @@ __device__ __forceinline__ u32x4 pack8(const float f[8]) {
 }
 
 // voxel index of the parent (D, H, W fine dims) of fine voxel v
-__device__ __forceinline__ long parent_of(long v, int D, int H, int W) {
-  const int x = (int)(v % W);
-  long r = v / W;
-  const int y = (int)(r % H);
+template <class I>
+__device__ __forceinline__ I parent_of(I v, unsigned D, unsigned H, unsigned W) {
+  const I x = v % W;
+  I r = v / W;
+  const I y = r % H;
   r /= H;
-  const int z = (int)(r % D);
-  const long b = r / D;
+  const I z = r % D;
+  const I b = r / D;
   return ((b * (D / 2) + z / 2) * (H / 2) + y / 2) * (W / 2) + x / 2;
 }
 
+template <class I>
 __global__ void k_up2_add(const uint16_t *__restrict__ c, const uint16_t *__restrict__ e, uint16_t *__restrict__ s,
-                          int D, int H, int W, int C, long n) {
-  const int P = C / 8;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int q = (int)(i % P);
-    const long v = i / P;
-    const long u = parent_of(v, D, H, W);
+                          unsigned D, unsigned H, unsigned W, unsigned C, I n) {
+  const I P = C / 8;
+  for (I i = (I)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (I)gridDim.x * blockDim.x) {
+    const I q = i % P;
+    const I v = i / P;
+    const I u = parent_of<I>(v, D, H, W);
     float a[8], b[8];
-    unpack8(*(const u32x4 *)(c + u * C + q * 8), a);
+    unpack8(*(const u32x4 *)(c + (size_t)u * C + q * 8), a);
     if (e) {
-      unpack8(*(const u32x4 *)(e + i * 8), b);
+      unpack8(*(const u32x4 *)(e + (size_t)i * 8), b);
 #pragma unroll
       for (int k = 0; k < 8; ++k) a[k] += b[k];
     }
-    *(u32x4 *)(s + i * 8) = pack8(a);
+    *(u32x4 *)(s + (size_t)i * 8) = pack8(a);
   }
 }
 
+template <class I>
 __global__ void k_pool2_bwd(const uint16_t *__restrict__ a, const uint16_t *__restrict__ g,
-                            const uint16_t *__restrict__ mask, uint16_t *__restrict__ out, int D, int H, int W, int C,
-                            long n) {
-  const int P = C / 8;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int q = (int)(i % P);
-    const long v = i / P;
-    const long u = parent_of(v, D, H, W);
+                            const uint16_t *__restrict__ mask, uint16_t *__restrict__ out, unsigned D, unsigned H, unsigned W, unsigned C,
+                            I n) {
+  const I P = C / 8;
+  for (I i = (I)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (I)gridDim.x * blockDim.x) {
+    const I q = i % P;
+    const I v = i / P;
+    const I u = parent_of<I>(v, D, H, W);
     float f[8], t[8];
-    unpack8(*(const u32x4 *)(g + u * C + q * 8), f);
+    unpack8(*(const u32x4 *)(g + (size_t)u * C + q * 8), f);
 #pragma unroll
     for (int k = 0; k < 8; ++k) f[k] *= 0.125f;
     if (a) {
-      unpack8(*(const u32x4 *)(a + i * 8), t);
+      unpack8(*(const u32x4 *)(a + (size_t)i * 8), t);
 #pragma unroll
       for (int k = 0; k < 8; ++k) f[k] += t[k];
     }
     if (mask) {
-      unpack8(*(const u32x4 *)(mask + i * 8), t);
+      unpack8(*(const u32x4 *)(mask + (size_t)i * 8), t);
 #pragma unroll
       for (int k = 0; k < 8; ++k)
         if (!(t[k] > 0.f)) f[k] = 0.f;
     }
-    *(u32x4 *)(out + i * 8) = pack8(f);
+    *(u32x4 *)(out + (size_t)i * 8) = pack8(f);
   }
 }
 
+template <class I>
 __global__ void k_up2_bwd(const uint16_t *__restrict__ ds, const uint16_t *__restrict__ mask,
-                          uint16_t *__restrict__ out, int D, int H, int W, int C, long n) {
-  const int P = C / 8;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int q = (int)(i % P);
-    long r = i / P;
-    const int ox = (int)(r % W);
+                          uint16_t *__restrict__ out, unsigned D, unsigned H, unsigned W, unsigned C, I n) {
+  const I P = C / 8;
+  for (I i = (I)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (I)gridDim.x * blockDim.x) {
+    const I q = i % P;
+    I r = i / P;
+    const I ox = r % W;
     r /= W;
-    const int oy = (int)(r % H);
+    const I oy = r % H;
     r /= H;
-    const int oz = (int)(r % D);
-    const long b = r / D;
+    const I oz = r % D;
+    const I b = r / D;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, t[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      const long iz = 2 * oz + (c >> 2), iy = 2 * oy + ((c >> 1) & 1), ix = 2 * ox + (c & 1);
-      const long v = ((b * 2 * D + iz) * 2 * H + iy) * 2 * W + ix;
-      unpack8(*(const u32x4 *)(ds + v * C + q * 8), t);
+      const I iz = 2 * oz + (c >> 2), iy = 2 * oy + ((c >> 1) & 1), ix = 2 * ox + (c & 1);
+      const I v = ((b * 2 * D + iz) * 2 * H + iy) * 2 * W + ix;
+      unpack8(*(const u32x4 *)(ds + (size_t)v * C + q * 8), t);
 #pragma unroll
       for (int k = 0; k < 8; ++k) acc[k] += t[k];
     }
     if (mask) {
-      unpack8(*(const u32x4 *)(mask + i * 8), t);
+      unpack8(*(const u32x4 *)(mask + (size_t)i * 8), t);
 #pragma unroll
       for (int k = 0; k < 8; ++k)
         if (!(t[k] > 0.f)) acc[k] = 0.f;
     }
-    *(u32x4 *)(out + i * 8) = pack8(acc);
+    *(u32x4 *)(out + (size_t)i * 8) = pack8(acc);
   }
 }
 
@@ -1856,19 +1930,119 @@ __global__ void __launch_bounds__(256) k_final_sum(const float *__restrict__ par
   if (threadIdx.x == 0) *out = r[0] * scale;
 }
 
-__global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m, float *__restrict__ v,
-                       uint16_t *__restrict__ w16, long n, float lr, float b1, float b2, float eps, float c1,
-                       float c2) {
-  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
-    const float gr = g[e];
-    const float mm = b1 * m[e] + (1.f - b1) * gr;
-    const float vv = b2 * v[e] + (1.f - b2) * gr * gr;
-    m[e] = mm;
-    v[e] = vv;
-    const float pn = p[e] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
-    p[e] = pn;
-    if (w16) w16[e] = f2bf(pn);
+// The same for C a multiple of 8 and 16-byte pointers: one lane takes 8
+// channels (one element per lane and 64-bit divisions took 47.7 us for 4 x 64^3
+// voxels of 16 channels, 22.6 now).
+__global__ void __launch_bounds__(256) k_mse8(const uint16_t *__restrict__ out, const float *__restrict__ tgt,
+                                              uint16_t *__restrict__ dout, float *__restrict__ part, unsigned n,
+                                              unsigned P, int nl, float gscale) {
+  __shared__ float red[256];
+  float s = 0.f;
+  for (unsigned e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
+    const unsigned v = e / P;
+    const int c0 = (int)(e - v * P) * 8;
+    float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (c0 < nl) {
+      unpack8(*(const u32x4 *)(out + (size_t)e * 8), f);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        float d = 0.f;
+        if (c0 + k < nl) d = f[k] - tgt[(size_t)v * nl + c0 + k];
+        s += d * d;
+        f[k] = gscale * d;
+      }
+    }
+    *(u32x4 *)(dout + (size_t)e * 8) = pack8(f);
   }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+
+// Adam on a list of tensors in one launch (a launch per tensor took 3 to 11 us
+// for each of a network's 30, 106 us in all; 28 now, 7.4 TB/s): every block takes
+// 1024 elements of one tensor, 16 bytes per lane where its pointers allow.
+constexpr int kAdamMax = 32;  // tensors per launch
+struct AdamItem {
+  float *p;
+  const float *g;
+  float *m, *v;
+  uint16_t *w16;
+  long n;
+  unsigned first;  // first block
+  int vec;         // every pointer on 16 bytes (w16: 8)
+};
+struct AdamList {
+  AdamItem it[kAdamMax];
+  int n;
+};
+
+__device__ __forceinline__ float adam_one(float p, float gr, float &m, float &v, float lr, float b1, float b2,
+                                          float eps, float c1, float c2) {
+  m = b1 * m + (1.f - b1) * gr;
+  v = b2 * v + (1.f - b2) * gr * gr;
+  return p - lr * (m / c1) / (sqrtf(v / c2) + eps);
+}
+
+__global__ void __launch_bounds__(256) k_adam(AdamList l, float lr, float b1, float b2, float eps, float c1,
+                                              float c2) {
+  int k = 0;
+  while (k + 1 < l.n && blockIdx.x >= l.it[k + 1].first) ++k;
+  const AdamItem it = l.it[k];
+  const long e0 = (long)(blockIdx.x - it.first) * 1024 + threadIdx.x * 4;
+  if (it.vec && e0 + 4 <= it.n) {
+    f32x4 p = *(const f32x4 *)(it.p + e0), m = *(const f32x4 *)(it.m + e0), v = *(const f32x4 *)(it.v + e0);
+    const f32x4 g = *(const f32x4 *)(it.g + e0);
+    uint16_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float mj = m[j], vj = v[j];
+      p[j] = adam_one(p[j], g[j], mj, vj, lr, b1, b2, eps, c1, c2);
+      m[j] = mj;
+      v[j] = vj;
+      w[j] = f2bf(p[j]);
+    }
+    *(f32x4 *)(it.m + e0) = m;
+    *(f32x4 *)(it.v + e0) = v;
+    *(f32x4 *)(it.p + e0) = p;
+    if (it.w16) *(uint2 *)(it.w16 + e0) = make_uint2(w[0] | (uint32_t)w[1] << 16, w[2] | (uint32_t)w[3] << 16);
+    return;
+  }
+  for (long e = e0; e < it.n && e < e0 + 4; ++e) {
+    float m = it.m[e], v = it.v[e];
+    const float p = adam_one(it.p[e], it.g[e], m, v, lr, b1, b2, eps, c1, c2);
+    it.m[e] = m;
+    it.v[e] = v;
+    it.p[e] = p;
+    if (it.w16) it.w16[e] = f2bf(p);
+  }
+}
+
+static int adam_list(int n, const lbmib_sg_adam_item *items, float lr, float b1, float b2, float eps, int t,
+                     hipStream_t s) {
+  const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
+  for (int k = 0; k < n;) {
+    AdamList l;
+    l.n = 0;
+    long blocks = 0;
+    for (; k < n && l.n < kAdamMax; ++k) {
+      const lbmib_sg_adam_item &q = items[k];
+      const long nb = (q.n + 1023) / 1024;
+      if (nb > 0x7fffffffL) return LBMIB_ERR_ARG;
+      if (blocks + nb > 0x7fffffffL) break;
+      const uintptr_t bits = (uintptr_t)q.p | (uintptr_t)q.g | (uintptr_t)q.m | (uintptr_t)q.v;
+      l.it[l.n++] = AdamItem{q.p, q.g, q.m, q.v, (uint16_t *)q.w16, q.n, (unsigned)blocks,
+                             (bits & 15) == 0 && ((uintptr_t)q.w16 & 7) == 0};
+      blocks += nb;
+    }
+    k_adam<<<(unsigned)blocks, 256, 0, s>>>(l, lr, b1, b2, eps, c1, c2);
+    HIPCHK(hipGetLastError());
+  }
+  return LBMIB_OK;
 }
 
 __global__ void k_cast(const float *__restrict__ src, uint16_t *__restrict__ dst, long n) {
@@ -1969,6 +2143,15 @@ __global__ void __launch_bounds__(256) k_sqdiff_final(const double *__restrict__
   }
 }
 
+// Launches a kernel over n 8-channel pieces with a 32-bit index where the
+// indices of the finer grid fit too, for the divisions that place a piece
+// (up2_add of 4 x 32^3 x 64 channels 9.5 -> 8.1 us, of 64^3 x 32 10.2 -> 9.0).
+template <class Fn>
+void pool_launch(long n, Fn fn) {
+  if (n < (1L << 29)) fn((unsigned)n);
+  else fn(n);
+}
+
 unsigned grid_for(long n, int per_block = 256, long cap = 8192) {
   long g = (n + per_block - 1) / per_block;
   if (g > cap) g = cap;
@@ -2001,10 +2184,25 @@ extern "C" int lbmib_sg_conv3d_bwd_data(const void *dy, const void *w, void *wt,
   if (!shape_ok(B, D, H, W, Cout, Cin) || Cin % 16) return LBMIB_ERR_ARG;
   if (Cout & (Cout - 1)) return LBMIB_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
-  const long n = (long)Cout * 27 * Cin;
-  k_flip<<<grid_for(n), 256, 0, s>>>((const uint16_t *)w, (uint16_t *)wt, Cin, Cout);
-  HIPCHK(hipGetLastError());
+  const lbmib_sg_flip_item item = {w, wt, Cin, Cout};
+  const int rc = flip_list(1, &item, s);
+  if (rc) return rc;
   return conv_fwd(dy, wt, nullptr, mask, dx, B, D, H, W, Cout, Cin, 0, s);
+}
+
+extern "C" int lbmib_sg_flip_many(int n, const lbmib_sg_flip_item *items, void *stream) {
+  if (n < 1 || !items) return LBMIB_ERR_ARG;
+  for (int k = 0; k < n; ++k) {
+    const lbmib_sg_flip_item &q = items[k];
+    if (!q.w || !q.wt || !shape_ok(1, 1, 1, 1, q.Cout, q.Cin)) return LBMIB_ERR_ARG;
+  }
+  return flip_list(n, items, (hipStream_t)stream);
+}
+
+extern "C" int lbmib_sg_conv3d_bwd_data_flipped(const void *dy, const void *wt, const void *mask, void *dx, int B,
+                                                int D, int H, int W, int Cin, int Cout, void *stream) {
+  if (!dy || !wt || !dx || !shape_ok(B, D, H, W, Cout, Cin)) return LBMIB_ERR_ARG;
+  return conv_fwd(dy, wt, nullptr, mask, dx, B, D, H, W, Cout, Cin, 0, (hipStream_t)stream);
 }
 
 extern "C" int lbmib_sg_conv3d_bwd_weight(const void *x, const void *dy, float *dw, float *db, int B, int D, int H,
@@ -2031,7 +2229,9 @@ extern "C" int lbmib_sg_conv3d_bwd_weight_noalloc(const void *x, const void *dy,
 extern "C" int lbmib_sg_pool2(const void *x, void *y, int B, int D, int H, int W, int C, void *stream) {
   if (!x || !y || B < 1 || D < 1 || H < 1 || W < 1 || C < 8 || C % 8) return LBMIB_ERR_ARG;
   const long n = (long)B * D * H * W * (C / 8);
-  k_pool2<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)x, (uint16_t *)y, D, H, W, C, n);
+  pool_launch(n, [&](auto nn) {
+    k_pool2<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)x, (uint16_t *)y, D, H, W, C, nn);
+  });
   HIPCHK(hipGetLastError());
   return LBMIB_OK;
 }
@@ -2040,8 +2240,9 @@ extern "C" int lbmib_sg_up2_add(const void *c, const void *e, void *s, int B, in
                                 void *stream) {
   if (!c || !s || B < 1 || D < 2 || H < 2 || W < 2 || (D | H | W) & 1 || C < 8 || C % 8) return LBMIB_ERR_ARG;
   const long n = (long)B * D * H * W * (C / 8);
-  k_up2_add<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)c, (const uint16_t *)e, (uint16_t *)s, D,
-                                                          H, W, C, n);
+  pool_launch(n, [&](auto nn) {
+    k_up2_add<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)c, (const uint16_t *)e, (uint16_t *)s, D, H, W, C, nn);
+  });
   HIPCHK(hipGetLastError());
   return LBMIB_OK;
 }
@@ -2050,8 +2251,9 @@ extern "C" int lbmib_sg_pool2_bwd(const void *a, const void *g, const void *mask
                                   int C, void *stream) {
   if (!g || !out || B < 1 || D < 2 || H < 2 || W < 2 || (D | H | W) & 1 || C < 8 || C % 8) return LBMIB_ERR_ARG;
   const long n = (long)B * D * H * W * (C / 8);
-  k_pool2_bwd<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)a, (const uint16_t *)g,
-                                                            (const uint16_t *)mask, (uint16_t *)out, D, H, W, C, n);
+  pool_launch(n, [&](auto nn) {
+    k_pool2_bwd<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)a, (const uint16_t *)g, (const uint16_t *)mask, (uint16_t *)out, D, H, W, C, nn);
+  });
   HIPCHK(hipGetLastError());
   return LBMIB_OK;
 }
@@ -2060,8 +2262,9 @@ extern "C" int lbmib_sg_up2_bwd(const void *ds, const void *mask, void *out, int
                                 void *stream) {
   if (!ds || !out || B < 1 || D < 1 || H < 1 || W < 1 || C < 8 || C % 8) return LBMIB_ERR_ARG;
   const long n = (long)B * D * H * W * (C / 8);
-  k_up2_bwd<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)ds, (const uint16_t *)mask,
-                                                          (uint16_t *)out, D, H, W, C, n);
+  pool_launch(n, [&](auto nn) {
+    k_up2_bwd<<<grid_for(n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)ds, (const uint16_t *)mask, (uint16_t *)out, D, H, W, C, nn);
+  });
   HIPCHK(hipGetLastError());
   return LBMIB_OK;
 }
@@ -2073,9 +2276,14 @@ extern "C" int lbmib_sg_mse(const void *out, const float *tgt, void *dout, float
   const int rc = workspace(&ws);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const unsigned nb = grid_for(M * C, 256, 1024);
   const float denom = (float)((double)M * nl);
-  k_mse<<<nb, 256, 0, s>>>((const uint16_t *)out, tgt, (uint16_t *)dout, (float *)ws, M, C, nl, 2.0f / denom);
+  const bool wide = C % 8 == 0 && M * (C / 8) < (1L << 31) && (((uintptr_t)out | (uintptr_t)dout) & 15) == 0;
+  const unsigned nb = grid_for(wide ? M * (C / 8) : M * C, 256, 1024);
+  if (wide)
+    k_mse8<<<nb, 256, 0, s>>>((const uint16_t *)out, tgt, (uint16_t *)dout, (float *)ws, (unsigned)(M * (C / 8)),
+                              (unsigned)(C / 8), nl, 2.0f / denom);
+  else
+    k_mse<<<nb, 256, 0, s>>>((const uint16_t *)out, tgt, (uint16_t *)dout, (float *)ws, M, C, nl, 2.0f / denom);
   HIPCHK(hipGetLastError());
   k_final_sum<<<1, 256, 0, s>>>((const float *)ws, (int)nb, 1.0f / denom, loss);
   HIPCHK(hipGetLastError());
@@ -2085,10 +2293,18 @@ extern "C" int lbmib_sg_mse(const void *out, const float *tgt, void *dout, float
 extern "C" int lbmib_sg_adam(float *p, const float *g, float *m, float *v, void *w16, long n, float lr, float beta1,
                              float beta2, float eps, int t, void *stream) {
   if (!p || !g || !m || !v || n < 1 || t < 1) return LBMIB_ERR_ARG;
-  const float c1 = 1.f - powf(beta1, (float)t), c2 = 1.f - powf(beta2, (float)t);
-  k_adam<<<grid_for(n), 256, 0, (hipStream_t)stream>>>(p, g, m, v, (uint16_t *)w16, n, lr, beta1, beta2, eps, c1, c2);
-  HIPCHK(hipGetLastError());
-  return LBMIB_OK;
+  const lbmib_sg_adam_item item = {p, g, m, v, w16, n};
+  return adam_list(1, &item, lr, beta1, beta2, eps, t, (hipStream_t)stream);
+}
+
+extern "C" int lbmib_sg_adam_many(int n, const lbmib_sg_adam_item *items, float lr, float beta1, float beta2,
+                                  float eps, int t, void *stream) {
+  if (n < 1 || !items || t < 1) return LBMIB_ERR_ARG;
+  for (int k = 0; k < n; ++k) {
+    const lbmib_sg_adam_item &q = items[k];
+    if (!q.p || !q.g || !q.m || !q.v || q.n < 1) return LBMIB_ERR_ARG;
+  }
+  return adam_list(n, items, lr, beta1, beta2, eps, t, (hipStream_t)stream);
 }
 
 extern "C" int lbmib_sg_cast_bf16(const float *src, void *dst, long n, void *stream) {

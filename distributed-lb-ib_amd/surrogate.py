@@ -23,6 +23,16 @@ import lbmib
 CHANS = (32, 64, 128, 256)
 
 
+class AdamItem(ctypes.Structure):
+    """lbmib_sg_adam_item"""
+    _fields_ = [(k, ctypes.c_void_p) for k in ("p", "g", "m", "v", "w16")] + [("n", ctypes.c_long)]
+
+
+class FlipItem(ctypes.Structure):
+    """lbmib_sg_flip_item"""
+    _fields_ = [("w", ctypes.c_void_p), ("wt", ctypes.c_void_p), ("Cin", ctypes.c_int), ("Cout", ctypes.c_int)]
+
+
 def _bind():
     L = lbmib.load_library()
     if getattr(L, "_sg_bound", False):
@@ -39,6 +49,9 @@ def _bind():
     L.lbmib_sg_up2_bwd.argtypes = [vp, vp, vp, i, i, i, i, i, vp]
     L.lbmib_sg_mse.argtypes = [vp, vp, vp, vp, l, i, i, vp]
     L.lbmib_sg_adam.argtypes = [vp, vp, vp, vp, vp, l, f, f, f, f, i, vp]
+    L.lbmib_sg_adam_many.argtypes = [i, ctypes.POINTER(AdamItem), f, f, f, f, i, vp]
+    L.lbmib_sg_flip_many.argtypes = [i, ctypes.POINTER(FlipItem), vp]
+    L.lbmib_sg_conv3d_bwd_data_flipped.argtypes = [vp, vp, vp, vp, i, i, i, i, i, i, vp]
     L.lbmib_sg_pack.argtypes = [vp, i, dp, dp, i, dp, vp, l, i, vp]
     L.lbmib_sg_target.argtypes = [vp, vp, i, dp, dp, vp, l, vp]
     L.lbmib_sg_unpack.argtypes = [vp, i, i, dp, dp, vp, l, vp]
@@ -53,7 +66,8 @@ def _bind():
 SG_SYMBOLS = ("lbmib_sg_conv3d_fwd", "lbmib_sg_conv3d_bwd_data", "lbmib_sg_conv3d_bwd_weight", "lbmib_sg_pool2",
               "lbmib_sg_up2_add", "lbmib_sg_pool2_bwd", "lbmib_sg_up2_bwd", "lbmib_sg_mse", "lbmib_sg_adam",
               "lbmib_sg_pack", "lbmib_sg_target", "lbmib_sg_unpack", "lbmib_sg_sqdiff", "lbmib_sg_cast_bf16",
-              "lbmib_sg_conv3d_bwd_weight_noalloc")
+              "lbmib_sg_conv3d_bwd_weight_noalloc", "lbmib_sg_conv3d_bwd_data_flipped", "lbmib_sg_flip_many",
+              "lbmib_sg_adam_many")
 
 
 def check(rc, where):
@@ -218,8 +232,15 @@ class Net:
     def _dgrad(self, name, dy, dx, mask, dims):
         _, ci, co, _, _ = next(l for l in self.layers if l[0] == name)
         self._timed("dgrad", name, lambda: check(
-            self.L.lbmib_sg_conv3d_bwd_data(ptr(dy), ptr(self.w16[name]), ptr(self.wt[name]), ptr(mask), ptr(dx),
-                                            *dims, ci, co, stream()), "conv3d_bwd_data " + name))
+            self.L.lbmib_sg_conv3d_bwd_data_flipped(ptr(dy), ptr(self.wt[name]), ptr(mask), ptr(dx), *dims, ci, co,
+                                                    stream()), "conv3d_bwd_data " + name))
+
+    def _flip(self):
+        """The transposed weights that the data gradients read, of every layer but the first."""
+        items = (FlipItem * (len(self.layers) - 1))()
+        for k, (name, ci, co, _, _) in enumerate(self.layers[1:]):
+            items[k] = FlipItem(self.w16[name].data_ptr(), self.wt[name].data_ptr(), ci, co)
+        check(self.L.lbmib_sg_flip_many(len(items), items, stream()), "flip_many")
 
     def backward(self, dout):
         """Parameter gradients (FP32, overwritten) for the output gradient
@@ -228,6 +249,7 @@ class Net:
         B, D, H, W = self.dims
         n = len(self.chans)
         dims = lambda lvl: (B, D >> lvl, H >> lvl, W >> lvl)  # noqa: E731
+        self._flip()
         self._wgrad("out", a["dec0b"], dout, dims(0))
         g = self._buf("g0", dims(0) + (self.chans[0],))
         self._dgrad("out", dout, g, a["dec0b"], dims(0))
@@ -276,12 +298,13 @@ class Net:
 
     def adam_step(self, lr, b1=0.9, b2=0.999, eps=1e-8):
         self.t += 1
-        for name in self.p:
-            check(self.L.lbmib_sg_adam(ptr(self.p[name]), ptr(self.g[name]), ptr(self.m[name]), ptr(self.v[name]),
-                                       ptr(self.w16[name]), self.p[name].numel(), lr, b1, b2, eps, self.t, stream()),
-                  "adam")
-            check(self.L.lbmib_sg_adam(ptr(self.b[name]), ptr(self.gb[name]), ptr(self.mb[name]), ptr(self.vb[name]),
-                                       None, self.b[name].numel(), lr, b1, b2, eps, self.t, stream()), "adam bias")
+        items = (AdamItem * (2 * len(self.p)))()
+        for k, name in enumerate(self.p):
+            for j, (p, g, m, v, w16) in enumerate(((self.p, self.g, self.m, self.v, self.w16[name].data_ptr()),
+                                                   (self.b, self.gb, self.mb, self.vb, None))):
+                items[2 * k + j] = AdamItem(p[name].data_ptr(), g[name].data_ptr(), m[name].data_ptr(),
+                                            v[name].data_ptr(), w16, p[name].numel())
+        check(self.L.lbmib_sg_adam_many(len(items), items, lr, b1, b2, eps, self.t, stream()), "adam")
 
     def train_step(self, x, tgt, lr):
         out = self.forward(x)

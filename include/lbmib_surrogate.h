@@ -48,6 +48,16 @@ int lbmib_sg_conv3d_fwd(const void *x, const void *w, const float *bias, const v
  * output, so that dx is the gradient at the previous layer's pre-activation. */
 int lbmib_sg_conv3d_bwd_data(const void *dy, const void *w, void *wt, const void *mask, void *dx, int B, int D, int H,
                              int W, int Cin, int Cout, void *stream);
+/* Its two parts: wt[ci][26 - t][co] = w[co][t][ci] of n layers in one launch,
+ * and the data gradient from a layer's wt. */
+typedef struct {
+  const void *w;
+  void *wt;
+  int Cin, Cout;
+} lbmib_sg_flip_item;
+int lbmib_sg_flip_many(int n, const lbmib_sg_flip_item *items, void *stream);
+int lbmib_sg_conv3d_bwd_data_flipped(const void *dy, const void *wt, const void *mask, void *dx, int B, int D, int H,
+                                     int W, int Cin, int Cout, void *stream);
 
 /* Weight and bias gradients: dw[co][t][ci] = sum_v dy[v][co] x[v + o(t)][ci],
  * db[co] = sum_v dy[v][co] (db nullable), FP32, overwritten.  The sum over
@@ -97,6 +107,16 @@ int lbmib_sg_mse(const void *out, const float *tgt, void *dout, float *loss, lon
  * the BF16 copy w16 (nullable) that the convolutions read. */
 int lbmib_sg_adam(float *p, const float *g, float *m, float *v, void *w16, long n, float lr, float beta1, float beta2,
                   float eps, int t, void *stream);
+/* The same on n tensors in one launch, with the same results. */
+typedef struct {
+  float *p;
+  const float *g;
+  float *m, *v;
+  void *w16; /* or NULL */
+  long n;
+} lbmib_sg_adam_item;
+int lbmib_sg_adam_many(int n, const lbmib_sg_adam_item *items, float lr, float beta1, float beta2, float eps, int t,
+                       void *stream);
 
 /* BF16 copy (round to nearest even) of n FP32 values. */
 int lbmib_sg_cast_bf16(const float *src, void *dst, long n, void *stream);
