@@ -587,6 +587,71 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
+// The moments of lbmib_get_macroscopic on every cell (the coupling's read at
+// factor 1): the row form's loads, one block per (y, z) row, so that they are
+// whole lines with a scalar offset per population; the tiles of the coarser
+// factors read 64-cell pieces and meet at barriers (256^3 FP32 330 us, now 252,
+// 6.1 TB/s; 512 x 256 x 256 FP64 1127, now 980).  The arithmetic and its
+// order are those of the tiles.
+template <int P, bool NTL, int ADDR>
+__global__ void __launch_bounds__(1024)
+    k_moments_rows(Geometry g, const typename Traits<P>::S *__restrict__ f, int own,
+                   KConsts<typename Traits<P>::T> c, double rhor, double mrx, double rho0, double u0x, double u0y,
+                   double u0z, double gz, int nsheets, const int *__restrict__ box,
+                   const typename Traits<P>::FT *__restrict__ F, const uint32_t *__restrict__ rowtab,
+                   float *__restrict__ out) {
+  using T = typename Traits<P>::T;
+  using S = typename Traits<P>::S;
+  using A = JumpT<P>;
+  const int x = threadIdx.x, row = blockIdx.x;
+  if (x >= g.nx) return;
+  const int y = row % g.ny, z = row / g.ny;
+  const auto acc = [&] {
+    if constexpr (ADDR == kRowsBuf) return BufRows<P>{make_rsrc(f), make_rsrc(f)};
+    else return PtrRows<P>{f, nullptr};
+  }();
+  A r = (A)rho0, ux = (A)u0x, uy = (A)u0y, uz = (A)u0z;
+  const long c0 = (long)x + (long)g.nx * row;
+  // the moment box, which lies in the active one and leaves out the frozen
+  // planes; on the first step every cell keeps the initial values
+  if (!own && y >= g.mlo[1] && y <= g.mhi[1] && z >= g.mlo[2] && z <= g.mhi[2] && x >= g.mlo[0] && x <= g.mhi[0]) {
+    const uint32_t *rt = rowtab + (long)row * kRowTabStride;
+    uint32_t so[19];
+    T v[19];
+#pragma unroll
+    for (int q = 0; q < 19; ++q) so[q] = ldc(rt + q);
+#pragma unroll
+    for (int q = 0; q < 19; ++q) v[q] = acc.template ld<NTL>((uint32_t)x * (uint32_t)sizeof(S), so[q]);
+    const uint32_t bbm = ldc(rt + 19);
+    const auto row_u = (uint32_t)row * ((uint32_t)g.prow * decltype(acc)::unit);
+    x_edge_sources<P, NTL>(g, acc, x, so, bbm, row_u, c.br[1], c.br[2], v);
+    bounce_fix<P>(bbm, c.br[1], c.br[2], v);
+    A fx = 0, fy = 0, fz = 0;
+    if (in_any_box(box, nsheets, x, y, z)) { fx = (A)F[c0]; fy = (A)F[g.n + c0]; fz = (A)F[2 * g.n + c0]; }
+    A s1 = 0, s2 = 0, s3 = 0, s4 = 0;
+#pragma unroll
+    for (int q = 0; q < 19; ++q) {
+      const A fq = (A)(v[q] * Traits<P>::inv_scale);
+      s1 += fq;
+      s2 = add_c(s2, kCX[q], fq);
+      s3 = add_c(s3, kCY[q], fq);
+      s4 = add_c(s4, kCZ[q], fq);
+    }
+    if (Traits<P>::dev) {  // sum r = rho_r, sum c r = rho_r u_r e_x
+      s1 += (A)rhor;
+      s2 += (A)mrx;
+    }
+    r = s1;
+    ux = (s2 + (A)0.5 * fx) / s1;
+    uy = (s3 + (A)0.5 * fy) / s1;
+    uz = (s4 + (A)0.5 * (fz + r * (A)gz)) / s1;
+  }
+  __builtin_nontemporal_store((float)r, out + c0);
+  __builtin_nontemporal_store((float)ux, out + g.n + c0);
+  __builtin_nontemporal_store((float)uy, out + 2 * g.n + c0);
+  __builtin_nontemporal_store((float)uz, out + 3 * g.n + c0);
+}
+
 // Two consecutive cells of a row per lane (the buffer-addressed path with
 // loads and stores twice as wide): lane t updates x = 2t and 2t + 1.  A pair
 // load of plane q reads the two sources (x - c_x, x + 1 - c_x), which are
@@ -1458,6 +1523,23 @@ int launch_collide_stream(int prec, const Geometry &g, const void *fin, void *fo
   LBMIB_DISPATCH(prec, ({
     if (nt) launch_any<P, true>(v, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, s);
     else launch_any<P, false>(v, g, fin, fout, own_mode, c, nsheets, box_cur, box_prev, Fcur, Fprev, s);
+  }));
+  return hipGetLastError() == hipSuccess ? LBMIB_OK : LBMIB_ERR_HIP;
+}
+
+int launch_moments_rows(int prec, const Geometry &g, const void *f, int own, const FluidConsts<double> &c, int nsheets,
+                        const int *box, const void *F, const uint32_t *rowtab, const uint32_t *rowtab_elems,
+                        float *out, hipStream_t s) {
+  const bool ntl = fused_shape(prec, g, rowtab != nullptr, 1, -1).nt & 2;
+  LBMIB_DISPATCH(prec, ({
+    auto go = [&](auto kern, const uint32_t *tab) {
+      kern<<<g.ny * g.nz, row_block(g), 0, s>>>(g, (const typename Traits<P>::S *)f, own, kconsts<P>(c), c.rhor,
+                                                c.rhor * c.urx, c.rho0, c.u0x, c.u0y, c.u0z, c.g, nsheets, box,
+                                                (const typename Traits<P>::FT *)F, tab, out);
+    };
+    if (!rowtab) go(k_moments_rows<P, true, kRowsPtr>, rowtab_elems);
+    else if (ntl) go(k_moments_rows<P, true, kRowsBuf>, rowtab);
+    else go(k_moments_rows<P, false, kRowsBuf>, rowtab);
   }));
   return hipGetLastError() == hipSuccess ? LBMIB_OK : LBMIB_ERR_HIP;
 }

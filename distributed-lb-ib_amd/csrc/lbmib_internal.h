@@ -242,6 +242,11 @@ bool row_path_elems(const Geometry &g);
 // A fused step that also writes the coarse stored-moment planes of the state
 // it writes (lbmib_step_coarse): whether it applies, and its launch
 // (LBMIB_ERR_ARG where it does not apply).
+// The moments of every cell into four planes of g.n floats, by rows; needs one
+// of the two row source tables.
+int launch_moments_rows(int prec, const Geometry &g, const void *f, int own, const FluidConsts<double> &c, int nsheets,
+                        const int *box, const void *F, const uint32_t *rowtab, const uint32_t *rowtab_elems,
+                        float *out, hipStream_t s);
 bool collide_coarse_ok(const Geometry &g, size_t es, bool rowtab, int F);
 int launch_collide_coarse(int prec, const Geometry &g, const void *fin, void *fout, int own_mode,
                           const FluidConsts<double> &c, int nsheets, const int *box_cur, const int *box_prev,
