@@ -221,8 +221,8 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const uint16_t *__restrict__ x
 // fragment order, and a ring of four z-planes holds the lines around the
 // block's (the next two planes are loaded into registers while these
 // multiply).  Each input voxel is thus staged once per (4 G + 2) / 4 G lines
-// and the weights once per block, where the box form below fetches 132 KB for
-// every 256 voxels.
+// and the weights once per block, where a box of 8 channels at a time took 132 KB
+// for every 256 voxels.
 //
 // A line's fragment of 16 voxels is read from LDS once for its three dx: the
 // products with the weights of each dx go to accumulators of their own, acc[dx][u]
@@ -237,7 +237,8 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const uint16_t *__restrict__ x
 //
 // The LDS holds one block, so two waves a SIMD: one's LDS reads and epilogue
 // run beside the other's products (with four waves and one plane at a time
-// they did not: 67 us where this takes 53).  Measured, with the box form's
+// they did not: 67 us where this takes 53).  Measured, with the former box
+// form's
 // times: 64^3 32 -> 32 at batch 4 53 us, 1089 TFLOP/s (92 us), at batch 1 18
 // us (31); 48^3 32 -> 32 12.5 us (27); 32^3 32 -> 64 at batch 4 16 us (27).
 // Matrix units are busy 43% of the time; the rest is the epilogue and, twice a
