@@ -388,6 +388,13 @@ __device__ __forceinline__ void gather_body(const IBState &ib, const Geometry &g
     static_assert(kNB == 4, "four bins");
     const auto bin4 = make_int4(bins[0], bins[1], bins[2], bins[3]), off4 = make_int4(0, cnt[1], cnt[2], cnt[3]);
     const auto meets_x = [&](const int4 &q) { return q.y <= x1 && q.y + 3 >= x0; };
+    // the zero entry: a support start far from every cell, zero factors and
+    // forces
+    const auto zero_entry = [&] {
+      if (threadIdx.x == 0) sst[kGatherStage] = make_int4(-(1 << 28), -(1 << 28), -(1 << 28), 0);
+      if (threadIdx.x < 12) sw[kGatherStage * 12 + threadIdx.x] = 0.0;
+      if (threadIdx.x < 3) se[kGatherStage * 3 + threadIdx.x] = 0.0;
+    };
     bool staged = seen <= kGatherEntries;
     int tot = 0;
     if (staged) {
@@ -436,11 +443,7 @@ __device__ __forceinline__ void gather_body(const IBState &ib, const Geometry &g
           for (int a = 0; a < 12; ++a) sw[r[1] * 12 + a] = ib.wgt[a * (long)M + q[1].x];
           for (int a = 0; a < 3; ++a) se[r[1] * 3 + a] = ib.frc[(NF_EX + a) * (long)M + q[1].x];
         }
-        // the zero entry: a support start far from every cell, zero factors
-        // and forces
-        if (threadIdx.x == 0) sst[kGatherStage] = make_int4(-(1 << 28), -(1 << 28), -(1 << 28), 0);
-        if (threadIdx.x < 12) sw[kGatherStage * 12 + threadIdx.x] = 0.0;
-        if (threadIdx.x < 3) se[kGatherStage * 3 + threadIdx.x] = 0.0;
+        zero_entry();
       } else {
         __syncthreads();  // the ids' readers are done
       }
@@ -465,14 +468,34 @@ __device__ __forceinline__ void gather_body(const IBState &ib, const Geometry &g
       if ((int)threadIdx.x < tot4 - tot) uraw[tot + threadIdx.x] = INT_MAX;  // above every id
       __syncthreads();
       const int4 *raw4 = reinterpret_cast<const int4 *>(uraw);
-      for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-        const int v = uraw[e];
+      const auto rank = [&](int v) {
         int r = 0;
         for (int k = 0; k < tot4 / 4; ++k) {
           const int4 q = raw4[k];
           r += (q.x < v) + (q.y < v) + (q.z < v) + (q.w < v);
         }
-        ust[r] = rst[e];  // starts and id
+        return r;
+      };
+      staged = tot <= kGatherStage;
+      if (staged) {
+        // few of many entries (sheets one behind the other): one candidate per
+        // thread, kept over the change of layout
+        const int e = threadIdx.x;
+        int4 q = make_int4(0, 0, 0, 0);
+        int r = 0;
+        if (e < tot) {
+          q = rst[e];
+          r = rank(q.w);
+        }
+        __syncthreads();
+        if (e < tot) {
+          sst[r] = q;
+          for (int a = 0; a < 12; ++a) sw[r * 12 + a] = ib.wgt[a * (long)M + q.w];
+          for (int a = 0; a < 3; ++a) se[r * 3 + a] = ib.frc[(NF_EX + a) * (long)M + q.w];
+        }
+        zero_entry();
+      } else {
+        for (int e = threadIdx.x; e < tot; e += kGatherThreads) ust[rank(uraw[e])] = rst[e];  // starts and id
       }
     }
     __syncthreads();

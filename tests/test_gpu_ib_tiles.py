@@ -39,6 +39,8 @@ CASES = {
                            _sheet(5, 4, 1.0, 26.0, y=28.0, seed=3), _sheet(6, 11, 1.0, 32.0, seed=4)],
     "behind_each_other": [_sheet(20, 21, 1.0, 18.0, seed=5), _sheet(20, 21, 1.0, 20.5, seed=6),
                           _sheet(20, 21, 1.0, 30.0, seed=7)],
+    "six_behind_each_other": [_sheet(14, 15, 1.0, 9.0 + 5.0 * k, seed=8 + k) for k in range(6)],
+    "six_close": [_sheet(14, 15, 1.0, 14.0 + 2.0 * k, seed=20 + k) for k in range(6)],
     "leaning": [_sheet(21, 18, 1.0, 23.0, lean=0.9)],
     "dense": [_sheet(24, 25, 0.55, 20.0)],
     "very_dense": [_sheet(30, 30, 0.45, 20.0)],
