@@ -21,6 +21,9 @@
 
 #include "../../include/lbmib.h"
 #include "../../include/lbmib_surrogate.h"
+#include "lbmib_conv_plan.h"
+
+using namespace lbmib;
 
 namespace {
 
@@ -51,12 +54,6 @@ __device__ __forceinline__ bf16x8 zero8() { return __builtin_bit_cast(bf16x8, u3
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-__host__ __device__ inline int ilog2(int v) {
-  int r = 0;
-  while ((1 << r) < v) ++r;
-  return r;
 }
 
 // ---------------------------------------------------------------- forward
@@ -243,12 +240,6 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const uint16_t *__restrict__ x
 // us (31); 48^3 32 -> 32 12.5 us (27); 32^3 32 -> 64 at batch 4 16 us (27).
 // Matrix units are busy 43% of the time; the rest is the epilogue and, twice a
 // step, the barriers around the exchange of planes.
-struct MarchGeo {
-  int G, nyb, zc, zs, cot;  // lines per wave; line groups, planes per block, z ranges, channel tiles
-  int plane_bytes;          // of one ring slot
-  long jobs;
-};
-
 // v of another lane of the row of 16, zero where there is none: the next
 // lane's, the previous one's; lane 0's at lane 15 alone, lane 15's at lane 0
 // alone.  Added to a sum, each is one v_add_f32 with a DPP operand.
@@ -467,35 +458,6 @@ __global__ void __launch_bounds__(512, 2)
   }
 }
 
-// Where the march applies, and its shape.
-bool march_geo(int B, int D, int H, int W, int Cin, int Cout, int *wm, MarchGeo *q) {
-  if ((Cin != 16 && Cin != 32) || W < 8 || W > 64) return false;
-  const long HW = (long)H * W;
-  if (HW * (Cin > Cout ? Cin : Cout) * 2 >= (1L << 31)) return false;
-  // positions per wave: the multiple of 16 that whole lines fill best
-  const int g4 = 64 / W, g3 = 48 / W;
-  *wm = g3 && g3 * W * 4 > g4 * W * 3 ? 3 : 4;
-  q->G = *wm == 3 ? g3 : g4;
-  q->nyb = (H + 4 * q->G - 1) / (4 * q->G);
-  q->plane_bytes = ((4 * q->G + 2) * W * 2 * Cin + 1023) / 1024 * 1024;
-  q->cot = (Cout + 31) / 32;
-  // z ranges: one block a CU (256), so the rounds of blocks times the plane
-  // pairs each takes (and about two for its weights and first planes) are least
-  const long cols = (long)B * q->nyb * q->cot;
-  long best = -1;
-  for (int zs = 1; zs <= D; ++zs) {
-    const int zc = (D + zs - 1) / zs, used = (D + zc - 1) / zc;
-    const long cost = (cols * used + 255) / 256 * ((zc + 1) / 2 + 2);
-    if (best < 0 || cost < best) {
-      best = cost;
-      q->zc = zc;
-      q->zs = used;
-    }
-  }
-  q->jobs = cols * q->zs;
-  return q->jobs < (1L << 30);
-}
-
 template <int WM, int WN, int CI>
 int launch_march(const MarchGeo &q, const void *x, const void *w, const float *bias, const void *mask, void *y, int D,
                  int H, int W, int Cout, int relu, hipStream_t s) {
@@ -550,14 +512,6 @@ int launch_march_any(int wm, const MarchGeo &q, const void *x, const void *w, co
 // (230).  The small ones are launch, first loads and the sum over KW; in the
 // large ones the loads of a block's box, which nothing overlaps (one block a
 // CU), and LDS reads beside the products.
-struct TileGeo {
-  int G, LP, PZ, nty, ntz, cot;  // lines per group; tile lines and planes; tiles in y and z; channel tiles
-  int cs, lgp;                   // channels staged at a time; log2 of their 16-byte pieces per voxel
-  int box, lds;                  // LDS bytes of the box, and of all
-  int mW, mLP;                   // 65536 / W + 1, 65536 / LP + 1: quotients of small numbers
-  long jobs;
-};
-
 template <int WM, int NC, int KW, int VG, bool WHOLE>
 __global__ void __launch_bounds__(512, 2)
     k_conv_tile(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
@@ -769,44 +723,6 @@ __global__ void __launch_bounds__(512, 2)
   }
 }
 
-// Shape of the tile form for 16 WM positions, NC channel groups, KW parts and
-// VG voxel groups; false where it does not apply.
-bool tile_geo(int B, int D, int H, int W, int Cin, int Cout, int wm, int nc, int kw, int vg, TileGeo *q) {
-  if (Cin < 32 || W > 16 * wm || W > 64) return false;
-  const long S = (long)D * H * W;
-  if (S * (Cin > Cout ? Cin : Cout) * 2 >= (1L << 31) || (long)Cout * 27 * Cin * 2 >= (1L << 31)) return false;
-  q->G = 16 * wm / W;
-  const int nl = q->G * vg;
-  // lines x planes: the fewest tiles, then the fewest lines in a tile's box
-  long best = -1;
-  for (int pz = 1; pz <= nl && pz <= D && pz <= 16; ++pz) {
-    const int lp = nl / pz < H ? nl / pz : H;
-    const long tiles = (long)((H + lp - 1) / lp) * ((D + pz - 1) / pz);
-    const long cost = tiles * 100000 + (long)(lp + 2) * (pz + 2);
-    if (best < 0 || cost < best) {
-      best = cost;
-      q->LP = lp;
-      q->PZ = pz;
-    }
-  }
-  q->nty = (H + q->LP - 1) / q->LP;
-  q->ntz = (D + q->PZ - 1) / q->PZ;
-  q->cot = (Cout + 16 * nc - 1) / (16 * nc);
-  q->mW = 65536 / W + 1;
-  q->mLP = 65536 / q->LP + 1;
-  const long vox = (long)(q->LP + 2) * (q->PZ + 2) * W;
-  q->cs = Cin;
-  const long most = 160 * 1024 - 8 * 3072;
-  while (q->cs > 32 && vox * (q->cs * 2 + 16) > most) q->cs /= 2;
-  const long box = vox * (q->cs * 2 + 16), red = kw > 1 ? 8L * wm * 1024 : 0;
-  if (box > most) return false;
-  q->box = (int)box;
-  q->lds = (int)(box + 8 * 3072 > red ? box + 8 * 3072 : red);
-  q->lgp = ilog2(q->cs / 8);
-  q->jobs = (long)B * q->nty * q->ntz * q->cot;
-  return q->jobs < (1L << 30);
-}
-
 template <int WM, int NC, int KW, int VG>
 int launch_tile(const TileGeo &q, const void *x, const void *w, const float *bias, const void *mask, void *y, int D,
                 int H, int W, int Cin, int Cout, int relu, hipStream_t s) {
@@ -819,42 +735,6 @@ int launch_tile(const TileGeo &q, const void *x, const void *w, const float *bia
   else go(k_conv_tile<WM, NC, KW, VG, false>);
   HIPCHK(hipGetLastError());
   return LBMIB_OK;
-}
-
-// The shape of least estimated time, in us: a block's first loads and box,
-// which take longer the more of the 256 CUs fetch at once, its items, and the
-// sum over KW.  The constants are a fit to 13 shapes on 70 layers (Cin 64 to
-// 256, and 32 below 4096 voxels; 4 to 64 voxels a side, Cout 16 to 256): 6.6%
-// rms, and the shape it picks takes 2% longer than the fastest on average.
-// The narrowest shape leaves room for two blocks a CU where its box is small.
-struct TileShape {
-  int wm, nc, kw, vg;
-};
-constexpr TileShape kTileShapes[] = {{8, 8, 1, 1}, {8, 4, 1, 2}, {8, 2, 1, 4}, {8, 4, 2, 1}, {8, 2, 4, 1}, {8, 1, 8, 1},
-                                     {4, 4, 2, 1}, {4, 2, 2, 2}, {4, 2, 4, 1}, {4, 1, 8, 1}, {2, 1, 8, 1}};
-
-bool tile_plan(int B, int D, int H, int W, int Cin, int Cout, int *shape, TileGeo *q) {
-  double best = 0;
-  bool any = false;
-  for (int k = 0; k < (int)(sizeof(kTileShapes) / sizeof(kTileShapes[0])); ++k) {
-    const TileShape &c = kTileShapes[k];
-    TileGeo g;
-    if (!tile_geo(B, D, H, W, Cin, Cout, c.wm, c.nc, c.kw, c.vg, &g)) continue;
-    const int per = c.wm == 2 && g.lds <= 80 * 1024 ? 2 : 1;
-    const long rounds = (g.jobs + 256 * per - 1) / (256 * per);
-    const double busy = g.jobs < 256 * per ? (double)g.jobs / (256 * per) : 1.0;
-    const int slices = Cin / g.cs, items = ((9 * g.cs / 32 + c.kw - 1) / c.kw + 1) / 2 * 2 * slices;
-    const double mb = (double)(g.LP + 2) * (g.PZ + 2) * W * (2 * Cin + 16) * 1e-6;
-    const double t = rounds * (2.0 * slices + 10.3 * mb * (0.28 + busy) +
-                               items * (0.073 * c.wm + 0.1) * (per == 2 ? 1.7 : 1.0) + (c.kw > 1 ? 2.1 : 0.0));
-    if (!any || t < best) {
-      any = true;
-      best = t;
-      *shape = k;
-      *q = g;
-    }
-  }
-  return any;
 }
 
 int launch_tile_any(int shape, const TileGeo &q, const void *x, const void *w, const float *bias, const void *mask,
@@ -1246,20 +1126,6 @@ static int flip_list(int n, const lbmib_sg_flip_item *items, hipStream_t s) {
 // Measured, against the form with one unit ahead through registers: 98 us
 // (593 TFLOP/s) for 139 at batch 4 x 64^3, 32 -> 32; 53 for 74 at 32^3, 64 ->
 // 64; 38 for 46 at 16^3, 128 -> 128; 203 for 275 at batch 2 x 24^3, 256 -> 256.
-constexpr int kWgRuns = 16;
-constexpr int kWgBufs = 3;      // units in LDS: one multiplies, two arrive
-constexpr int kWgMaxVox = 288;  // LDS voxels of a unit's x: three units and two blocks a CU in 160 KB
-
-struct WgGeo {
-  int TX, nr, R, P;  // voxels of a line segment, its runs of 8, lines per plane, planes
-  int halo;          // 1: segments of a longer line, loaded with their x neighbours
-  int LP;            // LDS voxels per line: index i is x = xs + i - 1
-  int nseg, nyb;     // segments per line, line groups per plane
-  int npg, nunits;     // plane groups, units
-  long planes;
-  int xbytes, ybytes;  // of one LDS buffer, multiples of 1024
-};
-
 // 16 bytes per lane from r + off to LDS at + 16 lane, without registers in
 // between; zeros where off lies past the resource.  Nothing waits: dma_wait.
 // (The builtin makes the compiler wait for every such load before the next LDS
@@ -1597,62 +1463,6 @@ __global__ void __launch_bounds__(256) k_wgrad_sum(const float *__restrict__ par
 #pragma unroll
   for (int r = 0; r < 4; ++r)
     if (co + r < Cout) dw[((long)(co + r) * 27 + t) * Cin + ci] = s[r];
-}
-
-// Units and split of the voxel reduction, from the shape only (so every entry
-// point that shares it gives the same bits), capped so that the partials fit
-// in `cap_bytes`.
-struct WgradPlan {
-  WgGeo q;
-  int ci_tiles, tiles, splits, na, nb, ups;  // ups: units per split
-  long n4;  // fragment quads of one split's partials
-  size_t lds, part_bytes;
-};
-
-WgradPlan wgrad_plan(int B, int D, int H, int W, int Cin, int Cout, size_t cap_bytes) {
-  WgradPlan p;
-  WgGeo &q = p.q;
-  // whole lines up to 64 voxels (an LDS line of at most 68), else 32-voxel
-  // segments: 64-voxel ones with their two neighbours need a fifth round of
-  // loads for 8 pieces
-  q.halo = W > 64;
-  q.TX = W > 64 ? 32 : (W + 7) / 8 * 8;
-  q.nr = q.TX / 8;
-  q.R = H < kWgRuns / q.nr ? H : kWgRuns / q.nr;
-  q.nseg = (W + q.TX - 1) / q.TX;
-  q.nyb = (H + q.R - 1) / q.R;
-  q.planes = (long)B * D;
-  q.P = 1;
-  if (q.R == H && q.nseg == 1) {  // whole planes: as many as the runs hold
-    const long fit = kWgRuns / (q.nr * q.R);
-    q.P = (int)(fit < q.planes ? fit : q.planes);
-    while (q.P > 1 && q.P * (q.R + 2) * (q.TX + 4) > kWgMaxVox) --q.P;
-  }
-  q.LP = q.TX + 4;
-  q.npg = (int)((q.planes + q.P - 1) / q.P);
-  q.nunits = q.npg * q.nyb * q.nseg;
-  p.na = Cout >= 32 ? 2 : 1;
-  p.nb = Cin >= 32 ? 2 : 1;
-  q.xbytes = (q.P * (q.R + 2) * q.LP * 32 * p.nb + 1023) / 1024 * 1024;
-  q.ybytes = kWgRuns * 8 * 32 * p.na;
-  p.lds = ((size_t)kWgBufs * (q.xbytes + q.ybytes) + 12 * 32 * p.nb + 1023) / 1024 * 1024 + 1024;
-  const size_t red = (size_t)4 * 3 * p.na * p.nb * 64 * sizeof(f32x4);
-  if (p.lds < red) p.lds = red;
-  p.ci_tiles = (Cin + 31) / 32;
-  p.tiles = p.ci_tiles * ((Cout + 31) / 32);
-  p.n4 = (long)p.tiles * 27 * p.na * p.nb * 64;
-  const size_t per_split = (size_t)p.n4 * 16 + (size_t)Cout * 4;
-  // about 512 blocks, one round at 2 per CU
-  long want = 512 / (3 * p.tiles);
-  if (want < 1) want = 1;
-  if (want > q.nunits) want = q.nunits;
-  const long cap = (long)(cap_bytes / per_split);
-  if (want > cap) want = cap;
-  if (want < 1) want = 1;
-  p.ups = (int)((q.nunits + want - 1) / want);
-  p.splits = (q.nunits + p.ups - 1) / p.ups;
-  p.part_bytes = per_split * p.splits;
-  return p;
 }
 
 template <int NA, int NB>
