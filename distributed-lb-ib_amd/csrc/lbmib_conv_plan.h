@@ -63,7 +63,7 @@ struct TileGeo {
   int G, LP, PZ, nty, ntz, cot;  // lines per group; tile lines and planes; tiles in y and z; channel tiles
   int cs, lgp;                   // channels staged at a time; log2 of their 16-byte pieces per voxel
   int box, lds;                  // LDS bytes of the box, and of all
-  int mW, mLP;                   // 65536 / W + 1, 65536 / LP + 1: quotients of small numbers
+  int mW, mLP;                   // 2^20 / W + 1, 2^20 / LP + 1: quotients (tile_pos)
   long jobs;
 };
 
@@ -90,8 +90,8 @@ inline bool tile_geo(int B, int D, int H, int W, int Cin, int Cout, int wm, int 
   q->nty = (H + q->LP - 1) / q->LP;
   q->ntz = (D + q->PZ - 1) / q->PZ;
   q->cot = (Cout + 16 * nc - 1) / (16 * nc);
-  q->mW = 65536 / W + 1;
-  q->mLP = 65536 / q->LP + 1;
+  q->mW = (1 << 20) / W + 1;
+  q->mLP = (1 << 20) / q->LP + 1;
   const long vox = (long)(q->LP + 2) * (q->PZ + 2) * W;
   q->cs = Cin;
   const long most = 160 * 1024 - 8 * 3072;
@@ -103,6 +103,24 @@ inline bool tile_geo(int B, int D, int H, int W, int Cin, int Cout, int wm, int 
   q->lgp = ilog2(q->cs / 8);
   q->jobs = (long)B * q->nty * q->ntz * q->cot;
   return q->jobs < (1L << 30);
+}
+
+// Position pos of voxel group vg: its plane and line in the tile, and its x.
+// n / d as n (2^20 / d + 1) >> 20, which is exact for n d < 2^20 and stays in
+// 31 bits: n <= 511 (the lines of a tile at W = 1) and d <= 512.  (With 2^16 the
+// last of 512 lines fell out of the tile and were not written.)
+struct TilePos {
+  int pz, ly, x;
+  bool in;
+};
+LBMIB_HD TilePos tile_pos(const TileGeo &q, int W, int vg, int pos) {
+  TilePos t;
+  const int l = (pos * q.mW) >> 20, lt = vg * q.G + l;
+  t.x = pos - l * W;
+  t.pz = (lt * q.mLP) >> 20;
+  t.ly = lt - t.pz * q.LP;
+  t.in = l < q.G && t.pz < q.PZ;
+  return t;
 }
 
 // The shape of least estimated time, in us: a block's first loads and box,

@@ -579,13 +579,12 @@ __global__ void __launch_bounds__(512, 2)
   bool nxt[WM], prv[WM];
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
-    const int pos = 16 * i + col, l = (pos * q.mW) >> 16, xx = pos - l * W, lt = vg * q.G + l;
-    const int pz = (lt * q.mLP) >> 16, ly = lt - pz * q.LP;
-    const bool in = l < q.G && pz < q.PZ, out = in && z0 + pz < D && y0 + ly < H;
-    at[i] = (in ? ((pz * BL + ly) * W + xx) * pitch : 0) + kq * 16;
-    yo[i] = out ? (uint32_t)(((((z0 + pz) * H + y0 + ly) * W + xx) * Cout + n0 + 4 * kq) * 2) : kNone;
-    nxt[i] = WHOLE ? (16 * i + 16) % W != 0 : xx < W - 1;
-    prv[i] = WHOLE ? 16 * i % W != 0 : xx > 0;
+    const TilePos t = tile_pos(q, W, vg, 16 * i + col);
+    const bool out = t.in && z0 + t.pz < D && y0 + t.ly < H;
+    at[i] = (t.in ? ((t.pz * BL + t.ly) * W + t.x) * pitch : 0) + kq * 16;
+    yo[i] = out ? (uint32_t)(((((z0 + t.pz) * H + y0 + t.ly) * W + t.x) * Cout + n0 + 4 * kq) * 2) : kNone;
+    nxt[i] = WHOLE ? (16 * i + 16) % W != 0 : t.x < W - 1;
+    prv[i] = WHOLE ? 16 * i % W != 0 : t.x > 0;
   }
   f32x4 acc[3][WM];
 #pragma unroll

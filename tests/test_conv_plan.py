@@ -1,0 +1,27 @@
+"""The shapes of the surrogate's convolution kernels (csrc/lbmib_conv_plan.h),
+walked on the host by tests/conv_plan_check.cpp."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("plan") / "conv_plan_check")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-Wall", "-o", exe,
+                           os.path.join(REPO, "tests", "conv_plan_check.cpp")])
+
+    def run(what):
+        r = subprocess.run([exe, what], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+def test_every_voxel_of_a_tile_has_one_position(check):
+    check("tiles")
