@@ -541,9 +541,10 @@ __global__ void __launch_bounds__(512, 2)
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(w), (short)0,
                                                                       Cout * 27 * Cin * 2, 0x00020000);
   // items of a slice: (dz, dy) times 32-channel blocks; this wave's are kg, kg
-  // + KW, ..., rounded up to pairs (weights past the end are zero)
+  // + KW, ...  Nothing past the end is multiplied: zero weights would turn an
+  // infinity of the voxels read in its place into NaN.
   const int lgc = q.lgp - 2, nitems = 9 << lgc;
-  const int nrounds = ((nitems + KW - 1) / KW + 1) / 2;
+  const int mine = (nitems - kg + KW - 1) / KW;
   const uint32_t wb = n0 < Cout ? (uint32_t)((n0 + (lane >> 2)) * 27 * Cin * 2 + (lane & 3) * 16) : kNone;
   u32x4 wf[2][3];
   auto load_w = [&](int s, int n, int c0) {
@@ -635,28 +636,36 @@ __global__ void __launch_bounds__(512, 2)
     }
     swap_w(0);
     load_w(0, 2, c0);
-    for (int rd = 0; rd < nrounds; ++rd) {
+    auto multiply = [&](int n, int s) {  // item n from wa[s] and bf; item n + 1 follows in wa[s ^ 1]
+      const int o = item_off(n + 1);
+      swap_w(s ^ 1);
+      load_w(s ^ 1, n + 3, c0);
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int o = item_off(rd * 2 + s + 1);
-        swap_w(s ^ 1);
-        load_w(s ^ 1, rd * 2 + s + 3, c0);
+      for (int i = 0; i < WM; ++i) {
 #pragma unroll
-        for (int i = 0; i < WM; ++i) {
-#pragma unroll
-          for (int dx = 0; dx < 3; ++dx) acc[dx][i] = mfma16(wa[s][dx], bf[i], acc[dx][i]);
-          bf[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(sm + at[i] + o));
-        }
-        __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x020, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-        for (int i = 1; i < WM; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
+        for (int dx = 0; dx < 3; ++dx) acc[dx][i] = mfma16(wa[s][dx], bf[i], acc[dx][i]);
+        bf[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(sm + at[i] + o));
       }
+      __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 3, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int i = 1; i < WM; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+    };
+    int n = 0;
+    for (; n + 1 < mine; n += 2) {
+      multiply(n, 0);
+      multiply(n + 1, 1);
+    }
+    if (n < mine) {
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) acc[dx][i] = mfma16(wa[0][dx], bf[i], acc[dx][i]);
     }
   }
 
