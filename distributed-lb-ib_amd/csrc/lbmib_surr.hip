@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const uint16_t *__restrict__ x
 //
 // Reduction slots 8 kq + e (kq = lane >> 4): CI = 32: channel 8 kq + e of one
 // (dz, dy); CI = 16: channel 8 (kq & 1) + e of (dz, dy) number 2 c + (kq >> 1)
-// in chunk c (the tenth is zero).
+// in chunk c (the tenth is zero in both operands).
 //
 // The LDS holds one block, so two waves a SIMD: one's LDS reads and epilogue
 // run beside the other's products (with four waves and one plane at a time
@@ -387,7 +387,10 @@ __global__ void __launch_bounds__(512, 2)
         }
         bf16x8 bf[WM];
 #pragma unroll
-        for (int i = 0; i < WM; ++i) bf[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(p + i * 16 * VX));
+        for (int i = 0; i < WM; ++i) {
+          bf[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(p + i * 16 * VX));
+          if (CI == 16 && c == kChunks - 1 && kq >> 1) bf[i] = zero8();  // no tenth line: 0 times an infinity is NaN
+        }
 #pragma unroll
         for (int dx = 0; dx < 3; ++dx)
 #pragma unroll

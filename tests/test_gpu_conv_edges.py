@@ -101,3 +101,14 @@ def _with_infinities(case, relu):
 ], ids=lambda c: "x".join(map(str, c)))
 def test_tile_keeps_an_infinity(case, relu):
     _with_infinities(case, relu)
+
+
+@pytest.mark.parametrize("relu", [0, 1])
+@pytest.mark.parametrize("case", [
+    (2, 12, 33, 33, 16, 32),
+    (3, 7, 40, 31, 16, 16),
+    (1, 8, 64, 64, 16, 48),
+    (1, 6, 64, 64, 32, 32),
+], ids=lambda c: "x".join(map(str, c)))
+def test_march_keeps_an_infinity(case, relu):
+    _with_infinities(case, relu)
