@@ -175,6 +175,36 @@ struct WgGeo {
   int xbytes, ybytes;  // of one LDS buffer, multiples of 1024
 };
 
+// Piece e (16 bytes, 8 channels) of a unit's x or dy in LDS, packed: its line,
+// plane and x in the unit (x: of the loaded lines, which begin one voxel and
+// one line before it), which 16 of a voxel's 32 channels, and bit 31 where
+// there is nothing to load.  The half alternates with the 8-voxel block and
+// the line, or the run, so that two runs' reads fall on distinct banks.
+constexpr uint32_t kWgNoPiece = 0x80000000u;
+LBMIB_HD uint32_t wg_pack(int l, int p, int ix, int h) { return (uint32_t)(l | p << 5 | ix << 10 | h << 17); }
+LBMIB_HD int wg_line(uint32_t v) { return (int)(v & 31); }
+LBMIB_HD int wg_plane(uint32_t v) { return (int)(v >> 5 & 31); }
+LBMIB_HD int wg_x(uint32_t v) { return (int)(v >> 10 & 127); }
+LBMIB_HD int wg_half(uint32_t v) { return (int)(v >> 17 & 1); }
+LBMIB_HD uint32_t wg_x_piece(const WgGeo &q, int nb, int e) {
+  const int pc = e & (2 * nb - 1), v = e / (2 * nb);
+  const int i = v % q.LP, L = v / q.LP, l = L % (q.R + 2), p = L / (q.R + 2);
+  if (p >= q.P) return kWgNoPiece;
+  return wg_pack(l, p, i, nb == 2 ? (pc >> 1) ^ (((i >> 3) + L) & 1) : 0);
+}
+LBMIB_HD uint32_t wg_dy_piece(const WgGeo &q, int na, int e, int channels) {
+  const int pc = e & (2 * na - 1), v = e / (2 * na), run = v >> 3;
+  const int ix = (run % q.nr) * 8 + (v & 7), l = (run / q.nr) % q.R, p = run / (q.nr * q.R);
+  const int h = na == 2 ? (pc >> 1) ^ (run & 1) : 0;
+  return p < q.P && h * 16 < channels ? wg_pack(l, p, ix, h) : kWgNoPiece;
+}
+// Its element offset from the unit's first voxel in a tensor of C channels.
+// (The half comes from its own bit: the offset's holds it only where voxels are
+// whole 64-byte pieces, and dy has any multiple of 16 channels.)
+LBMIB_HD long wg_piece_at(uint32_t v, int e, int H, int W, int C) {
+  return (((long)wg_plane(v) * H + wg_line(v)) * W + wg_x(v)) * C + wg_half(v) * 16 + (e & 1) * 8;
+}
+
 // Units and split of the voxel reduction, from the shape only (so every entry
 // point that shares it gives the same bits), capped so that the partials fit
 // in `cap_bytes`.

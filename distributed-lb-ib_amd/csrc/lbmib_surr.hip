@@ -1195,29 +1195,20 @@ __global__ void __launch_bounds__(256, 2)
 
   // Instruction k of a wave fills the 1024 bytes number wave + 4 k of a
   // buffer's x (and of its dy): this lane's piece of it, where it lies in
-  // memory relative to the unit, and (in one register) line, plane and x,
-  // which decide whether it exists
+  // memory relative to the unit, and (in one register, wg_x_piece) line, plane,
+  // x and half, which decide whether it exists
   uint32_t xo[KX], yo[KY], xl[KX], yl[KY];
-  constexpr uint32_t kNoPiece = 0x80000000u;
-  auto pack = [](int l, int p, int ix) { return (uint32_t)(l | p << 5 | ix << 10); };
-  auto line_of = [](uint32_t v) { return (int)(v & 31); };
-  auto plane_of = [](uint32_t v) { return (int)(v >> 5 & 31); };
-  auto x_of = [](uint32_t v) { return (int)(v >> 10 & 127); };
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
-    const int e = (wave + 4 * k) * 64 + lane, pc = e & (2 * NB - 1), v = e / (2 * NB);
-    const int i = v % q.LP, L = v / q.LP, l = L % (q.R + 2), p = L / (q.R + 2);
-    const int h = NB == 2 ? (pc >> 1) ^ (((i >> 3) + L) & 1) : 0;
-    xo[k] = (uint32_t)((((long)p * H + l) * W + i) * Cin * 2 + h * 32 + (pc & 1) * 16);
-    xl[k] = p < q.P ? pack(l, p, i) : kNoPiece;
+    const int e = (wave + 4 * k) * 64 + lane;
+    xl[k] = wg_x_piece(q, NB, e);
+    xo[k] = (uint32_t)(wg_piece_at(xl[k], e, H, W, Cin) * 2);
   }
 #pragma unroll
   for (int k = 0; k < KY; ++k) {
-    const int e = (wave + 4 * k) * 64 + lane, pc = e & (2 * NA - 1), v = e / (2 * NA);
-    const int run = v >> 3, ix = (run % q.nr) * 8 + (v & 7), l = (run / q.nr) % q.R, p = run / (q.nr * q.R);
-    const int h = NA == 2 ? (pc >> 1) ^ (run & 1) : 0, ch = h * 16 + (pc & 1) * 8;
-    yo[k] = (uint32_t)((((long)p * H + l) * W + ix) * Cout * 2 + ch * 2);
-    yl[k] = p < q.P && co0 + ch < Cout ? pack(l, p, ix) : kNoPiece;
+    const int e = (wave + 4 * k) * 64 + lane;
+    yl[k] = wg_dy_piece(q, NA, e, Cout - co0);
+    yo[k] = (uint32_t)(wg_piece_at(yl[k], e, H, W, Cout) * 2);
   }
   // this lane's run: LDS addresses of its x (line dy = -1) and dy operands
   const int run = 4 * wave + kq, rx = run % q.nr, rl = (run / q.nr) % q.R, rp = run / (q.nr * q.R);
@@ -1273,12 +1264,11 @@ __global__ void __launch_bounds__(256, 2)
     const uint32_t at0 = lds0 + buf * buf_bytes;
 #pragma unroll
     for (int k = 0; k < KX; ++k) {
-      const int l = line_of(xl[k]), p = plane_of(xl[k]), ix = x_of(xl[k]), at = (wave + 4 * k) * 1024;
-      const bool ok = (xl[k] != kNoPiece) & ((unsigned)(y0 - 1 + l) < (unsigned)H) &
+      const int l = wg_line(xl[k]), p = wg_plane(xl[k]), ix = wg_x(xl[k]), at = (wave + 4 * k) * 1024;
+      const bool ok = !(xl[k] & kWgNoPiece) & ((unsigned)(y0 - 1 + l) < (unsigned)H) &
                       ((unsigned)(xs - 1 + ix) < (unsigned)W) & (bool)(zin >> p & 1);
       if constexpr (BIG) {
-        const int pc = lane & (2 * NB - 1), h = NB == 2 ? (xo[k] >> 5) & 1 : 0;
-        const uint16_t *src = ok ? bx + (((long)p * H + l) * W + ix) * Cin + h * 16 + (pc & 1) * 8 : x;
+        const uint16_t *src = ok ? bx + wg_piece_at(xl[k], lane, H, W, Cin) : x;
         const u32x4 v = ok ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
         if (at < q.xbytes) *(u32x4 *)(sm + buf * buf_bytes + at + lane * 16) = v;
       } else {
@@ -1287,11 +1277,10 @@ __global__ void __launch_bounds__(256, 2)
     }
 #pragma unroll
     for (int k = 0; k < KY; ++k) {
-      const int l = line_of(yl[k]), p = plane_of(yl[k]), ix = x_of(yl[k]), at = q.xbytes + (wave + 4 * k) * 1024;
-      const bool ok = (yl[k] != kNoPiece) & (y0 + l < H) & (xs + ix < W) & (bool)(yin >> p & 1);
+      const int l = wg_line(yl[k]), p = wg_plane(yl[k]), ix = wg_x(yl[k]), at = q.xbytes + (wave + 4 * k) * 1024;
+      const bool ok = !(yl[k] & kWgNoPiece) & (y0 + l < H) & (xs + ix < W) & (bool)(yin >> p & 1);
       if constexpr (BIG) {
-        const int pc = lane & (2 * NA - 1), h = NA == 2 ? (yo[k] >> 5) & 1 : 0;
-        const uint16_t *src = ok ? by + (((long)p * H + l) * W + ix) * Cout + h * 16 + (pc & 1) * 8 : dy;
+        const uint16_t *src = ok ? by + wg_piece_at(yl[k], lane, H, W, Cout) : dy;
         *(u32x4 *)(sm + buf * buf_bytes + at + lane * 16) = ok ? *(const u32x4 *)src : u32x4{0u, 0u, 0u, 0u};
       } else {
         dma16(ry_, ok ? yo[k] : kNone, at0 + at);

@@ -2,6 +2,8 @@
 //   tiles   every output voxel of a tile belongs to exactly one position of
 //           its waves, for every line width, tile shape and lines x planes
 //           that the plans give.
+//   pieces  every 16-byte piece of a weight-gradient unit comes from the voxel
+//           and channels that the LDS reads expect there.
 // Prints what it finds wrong and returns the number of wrong cases.
 #include <stdio.h>
 #include <string.h>
@@ -39,8 +41,46 @@ static int tiles() {
   return bad;
 }
 
+// What lies at byte 16 e of a unit's dy: run e / (16 na) of 8 voxels, 2 na
+// pieces each, the upper half first in odd runs.  x: lines of LP voxels.
+static int pieces() {
+  int bad = 0;
+  const int widths[] = {1, 3, 8, 13, 33, 64, 65, 300}, heights[] = {1, 2, 5, 16};
+  for (int W : widths)
+    for (int H : heights)
+      for (int C = 16; C <= 144; C += 16) {
+        const int cin = C >= 128 ? 128 : (C >= 64 ? 64 : (C >= 32 ? 32 : 16));
+        const WgradPlan p = wgrad_plan(2, 3, H, W, cin, C, 1 << 27);
+        const WgGeo &q = p.q;
+        for (int co0 = 0; co0 < C; co0 += 32)
+          for (int e = 0; e < kWgRuns * 8 * 2 * p.na; ++e) {
+            const int v = e / (2 * p.na), run = v / 8, second = p.na == 2 ? e / 2 % 2 : 0;
+            const int half = p.na == 2 && run % 2 ? 1 - second : second;
+            const int line = run / q.nr % q.R, plane = run / q.nr / q.R, x = run % q.nr * 8 + v % 8;
+            const uint32_t w = wg_dy_piece(q, p.na, e, C - co0);
+            const bool none = plane >= q.P || co0 + half * 16 >= C;
+            const long want = (((long)plane * H + line) * W + x) * C + half * 16 + e % 2 * 8;
+            if (none != (w == kWgNoPiece) || (!none && wg_piece_at(w, e, H, W, C) != want)) {
+              if (++bad <= 10) printf("pieces: dy, W %d, H %d, %d channels from %d, piece %d\n", W, H, C, co0, e);
+            }
+          }
+        for (int e = 0; e < q.xbytes / 16; ++e) {
+          const int v = e / (2 * p.nb), second = p.nb == 2 ? e / 2 % 2 : 0, i = v % q.LP, L = v / q.LP;
+          const int half = p.nb == 2 && (i / 8 + L) % 2 ? 1 - second : second;
+          const int line = L % (q.R + 2), plane = L / (q.R + 2);
+          const uint32_t w = wg_x_piece(q, p.nb, e);
+          const long want = (((long)plane * H + line) * W + i) * cin + half * 16 + e % 2 * 8;
+          if ((plane >= q.P) != (w == kWgNoPiece) || (plane < q.P && wg_piece_at(w, e, H, W, cin) != want)) {
+            if (++bad <= 10) printf("pieces: x, W %d, H %d, %d channels, piece %d\n", W, H, cin, e);
+          }
+        }
+      }
+  return bad;
+}
+
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "tiles")) return tiles() != 0;
+  if (!strcmp(what, "pieces")) return pieces() != 0;
   return 2;
 }

@@ -25,3 +25,7 @@ def check(tmp_path_factory):
 
 def test_every_voxel_of_a_tile_has_one_position(check):
     check("tiles")
+
+
+def test_every_piece_of_a_weight_gradient_unit_is_the_one_its_readers_expect(check):
+    check("pieces")
