@@ -1140,7 +1140,11 @@ static int flip_list(int n, const lbmib_sg_flip_item *items, hipStream_t s) {
 // 16 bytes per lane from r + off to LDS at + 16 lane, without registers in
 // between; zeros where off lies past the resource.  Nothing waits: dma_wait.
 // (The builtin makes the compiler wait for every such load before the next LDS
-// read, whichever buffer it reads.  The compiler keeps nothing in m0.)
+// read, whichever buffer it reads.  m0 is among the clobbers so that nothing
+// the compiler puts there is expected to survive; it warns that the register
+// is reserved.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(u32x4 r, uint32_t off, uint32_t at) {
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
@@ -1148,8 +1152,9 @@ __device__ __forceinline__ void dma16(u32x4 r, uint32_t off, uint32_t at) {
       "buffer_load_dwordx4 %1, %2, 0 offen lds"
       :
       : "s"(at), "v"(off), "s"(r)
-      : "memory");
+      : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // all but the last N loads have arrived, and this wave's LDS reads are done
 template <int N>
 __device__ __forceinline__ void dma_wait() {
