@@ -296,10 +296,15 @@ __device__ __forceinline__ bool tile_of(const IBState &ib, int slot, int w, int 
 
 constexpr int kGatherMaxCand = 384;         // candidates whose support meets the tile: 13.8 KB of LDS
 constexpr int kGatherEntries = 2 * kGatherThreads;  // bin entries taken at once: two per thread
-constexpr int kGatherStage = 96;            // candidates whose delta factors / forces are staged
+// Candidates whose delta factors / forces are staged: what two ballots cover,
+// and the two times 49 of two close sheets at unit spacing (with 96 those took
+// the unstaged path: two sheets of 90 x 90 nodes 3 cells apart 48 us, 22 now).
+constexpr int kGatherStage = 128;
+static_assert(kGatherStage >= 2 * 49, "two close sheets are staged");
 
 // LDS of a gather block: the staged candidates' factors, forces, starts and
-// ids and a zero entry, and the entries' ids (18.6 KB, so that 8 blocks share a CU), or in their place the starts and
+// ids and a zero entry, and the entries' ids (18.6 KB: 8 blocks share a CU, as
+// many as the kernel's registers allow), or in their place the starts and
 // ids of up to kGatherMaxCand candidates, raw and sorted (the layout of
 // gather_body).
 constexpr size_t kGatherShm =
