@@ -194,7 +194,7 @@ extern "C" int lbmib_batch_create(int n, const lbmib_fluid_params *fluids, const
   b->prec = fluids[0].precision;
   int rc = LBMIB_OK, off = 0;
   for (int i = 0; i < n && !rc; ++i) {
-    // the batched fused kernel has no x-edge pass: inlet/outlet x only
+    // the batched fused kernel leaves the x edges out: inlet/outlet x only
     if (fluids[i].precision != b->prec || fluids[i].bc_x != LBMIB_BC_INOUT || nsheets[i] < 0) rc = LBMIB_ERR_ARG;
     lbmib_ctx *c = nullptr;
     if (!rc) rc = lbmib_create(fluids + i, nsheets[i], nsheets[i] ? sheets + off : nullptr, &c);

@@ -385,10 +385,15 @@ struct NoSink {
 // table holds 32 bits: up to 2^32 elements), one 64-bit scalar address per
 // population; the cell-by-cell general path, which larger arrays took before,
 // ran the fused kernel at 4.7 TB/s at 512 x 256 x 256 in FP64 (2163 us; this form
-// 1948 us, 5.2 TB/s).
-template <int P>
+// 1948 us, 5.2 TB/s).  EDGES: a wall or periodic x axis, whose edge cells take
+// x_edge_sources; kernels of an inlet/outlet axis are built without it (with
+// the test in them they took 3 to 5% longer -- 192 x 204 x 204 FP64 409 -> 421
+// us, 8 x 64 x 64 30 -> 36 -- and FP64 pairs a register too many for three waves
+// a SIMD: 640 x 80 x 80 217 -> 277).
+template <int P, bool EDGES>
 struct BufRows {
   static constexpr uint32_t unit = sizeof(typename Traits<P>::S);
+  static constexpr bool edges = EDGES;
   __amdgpu_buffer_rsrc_t rin, rout;
   template <bool NTL>
   __device__ __forceinline__ typename Traits<P>::T ld(uint32_t vo, uint32_t so) const {
@@ -399,10 +404,11 @@ struct BufRows {
     bst_h<P, NT>(rout, vo, so, v);
   }
 };
-template <int P>
+template <int P, bool EDGES>
 struct PtrRows {
   using S = typename Traits<P>::S;
   static constexpr uint32_t unit = 1;
+  static constexpr bool edges = EDGES;
   const S *fin;
   S *fout;
   template <bool NTL>
@@ -425,8 +431,8 @@ template <int P, bool NTL, class A>
 __device__ __forceinline__ void x_edge_sources(const Geometry &g, const A &acc, int x, const uint32_t so[19],
                                                uint32_t mask, uint32_t row_u, typename Traits<P>::T b1,
                                                typename Traits<P>::T b2, typename Traits<P>::T v[19]) {
+  if constexpr (!A::edges) return;
   constexpr uint32_t es = sizeof(typename Traits<P>::S);
-  if (g.bc[0] == LBMIB_BC_INOUT) return;
   const uint32_t pitch_u = (uint32_t)g.pq * A::unit;
 #pragma unroll
   for (int side = -1; side <= 1; side += 2) {
@@ -553,10 +559,10 @@ __device__ __forceinline__ void row_cell(const Geometry &g, const A &acc, int ow
 // wave-uniform (SGPR) value and the 19 loads and 19 stores of a lane share one
 // VGPR offset, x * sizeof(S) (one cell per thread, blockDim.x >= nx).  Lanes
 // on the frozen inlet/outlet planes take the table; the two x-edge cells of a
-// row on a wall or periodic x axis take x_edge_sources.  kRowsGeneral: every
-// cell takes update_cell.
+// row on a wall or periodic x axis (EDGES) take x_edge_sources.  kRowsGeneral:
+// every cell takes update_cell.
 enum { kRowsGeneral = 0, kRowsBuf = 1, kRowsPtr = 2 };
-template <int P, bool NT, bool NTL, int ADDR>
+template <int P, bool NT, bool NTL, int ADDR, bool EDGES>
 __global__ void __launch_bounds__(1024)
     k_collide_stream_rows(Geometry g, const typename Traits<P>::S *__restrict__ fin,
                           typename Traits<P>::S *__restrict__ fout, int own, KConsts<typename Traits<P>::T> c,
@@ -577,8 +583,8 @@ __global__ void __launch_bounds__(1024)
     const int x = threadIdx.x;
     if (x >= g.nx) return;
     const auto acc = [&] {
-      if constexpr (ADDR == kRowsBuf) return BufRows<P>{make_rsrc(fin), make_rsrc(fout)};
-      else return PtrRows<P>{fin, fout};
+      if constexpr (ADDR == kRowsBuf) return BufRows<P, EDGES>{make_rsrc(fin), make_rsrc(fout)};
+      else return PtrRows<P, EDGES>{fin, fout};
     }();
     int row;
     for (long it = blockIdx.x; next_row(g, it, row); it += gridDim.x)
@@ -593,7 +599,7 @@ __global__ void __launch_bounds__(1024)
 // factors read 64-cell pieces and meet at barriers (256^3 FP32 330 us, now 252,
 // 6.1 TB/s; 512 x 256 x 256 FP64 1127, now 980).  The arithmetic and its
 // order are those of the tiles.
-template <int P, bool NTL, int ADDR>
+template <int P, bool NTL, int ADDR, bool EDGES>
 __global__ void __launch_bounds__(1024)
     k_moments_rows(Geometry g, const typename Traits<P>::S *__restrict__ f, int own,
                    KConsts<typename Traits<P>::T> c, double rhor, double mrx, double rho0, double u0x, double u0y,
@@ -607,8 +613,8 @@ __global__ void __launch_bounds__(1024)
   if (x >= g.nx) return;
   const int y = row % g.ny, z = row / g.ny;
   const auto acc = [&] {
-    if constexpr (ADDR == kRowsBuf) return BufRows<P>{make_rsrc(f), make_rsrc(f)};
-    else return PtrRows<P>{f, nullptr};
+    if constexpr (ADDR == kRowsBuf) return BufRows<P, EDGES>{make_rsrc(f), make_rsrc(f)};
+    else return PtrRows<P, EDGES>{f, nullptr};
   }();
   A r = (A)rho0, ux = (A)u0x, uy = (A)u0y, uz = (A)u0z;
   const long c0 = (long)x + (long)g.nx * row;
@@ -699,7 +705,7 @@ __device__ __forceinline__ void bst_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff
   else __builtin_amdgcn_raw_buffer_store_b32(u, r, voff, soff, aux);
 }
 
-template <int P, bool NT, bool NTL>
+template <int P, bool NT, bool NTL, bool EDGES>
 __global__ void __launch_bounds__(512)
     k_collide_stream_pairs(Geometry g, const typename Traits<P>::S *__restrict__ fin,
                            typename Traits<P>::S *__restrict__ fout, int own, KConsts<typename Traits<P>::T> c,
@@ -756,7 +762,7 @@ __global__ void __launch_bounds__(512)
         const uint32_t bbm = ldc(rt + 19);
 #pragma unroll
         for (int k = 0; k < 2; ++k)
-          x_edge_sources<P, NTL>(g, BufRows<P>{rin, rout}, x0 + k, so, bbm, row_b, c.br[1], c.br[2], v[k]);
+          x_edge_sources<P, NTL>(g, BufRows<P, EDGES>{rin, rout}, x0 + k, so, bbm, row_b, c.br[1], c.br[2], v[k]);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
           bounce_fix<P>(bbm, c.br[1], c.br[2], v[k]);
@@ -807,7 +813,7 @@ __global__ void __launch_bounds__(512)
 // independent sets of aligned buffer loads, which doubles the bytes each wave
 // keeps in flight.  Filler lanes (dead x) store zeros so that the rows' cache
 // lines are written whole.
-template <int P, bool NT, bool NTL>
+template <int P, bool NT, bool NTL, bool EDGES>
 __device__ __forceinline__ void row_pair_cell(const Geometry &g, __amdgpu_buffer_rsrc_t rin,
                                               __amdgpu_buffer_rsrc_t rout, int own,
                                               const KConsts<typename Traits<P>::T> &c, int nsheets,
@@ -865,7 +871,7 @@ __device__ __forceinline__ void row_pair_cell(const Geometry &g, __amdgpu_buffer
       for (int k = 0; k < 2; ++k) {
         const uint32_t bbm = ldc(rt + k * kRowTabStride + 19);
         if (live[k])  // (a dead row has no sources in the table)
-          x_edge_sources<P, NTL>(g, BufRows<P>{rin, rout}, x, so[k], bbm, (uint32_t)(row0 + k) * sy_b, c.br[1],
+          x_edge_sources<P, NTL>(g, BufRows<P, EDGES>{rin, rout}, x, so[k], bbm, (uint32_t)(row0 + k) * sy_b, c.br[1],
                                  c.br[2], v[k]);
         bounce_fix<P>(bbm, c.br[1], c.br[2], v[k]);
         const long ck = (long)x + (long)g.nx * (row0 + k);
@@ -918,7 +924,7 @@ __device__ __forceinline__ void row_pair_cell(const Geometry &g, __amdgpu_buffer
 // and (x, y + 1, z) (row_pair_cell), which doubles the bytes each wave keeps
 // in flight without the unaligned pair loads of k_collide_stream_pairs.
 // Requires ny even and blockDim.x >= nx.
-template <int P, bool NT, bool NTL>
+template <int P, bool NT, bool NTL, bool EDGES>
 __global__ void __launch_bounds__(512)
     k_collide_stream_rows2(Geometry g, const typename Traits<P>::S *__restrict__ fin,
                            typename Traits<P>::S *__restrict__ fout, int own, KConsts<typename Traits<P>::T> c,
@@ -931,16 +937,16 @@ __global__ void __launch_bounds__(512)
   const int x = threadIdx.x;
   if (x >= g.nx) return;
   for (int rp = blockIdx.x; rp < npairs; rp += gridDim.x)
-    row_pair_cell<P, NT, NTL>(g, rin, rout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, 2 * rp, x,
-                              box_rows_cached);
+    row_pair_cell<P, NT, NTL, EDGES>(g, rin, rout, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, 2 * rp, x,
+                                     box_rows_cached);
 }
 
 // Batched ensemble: every instance's rows in one launch.  Block b serves
 // instance map[b] >> kBatchShift; each wave of it one row (or one 64-lane x
 // chunk of a row wider than 64: wpr waves per row), so the row offsets stay
 // wave-uniform for any mix of grid sizes; wpb waves per block is the tile
-// shape of the launch.  Instances need an inlet/outlet x axis (no x-edge
-// kernel).
+// shape of the launch.  Instances need an inlet/outlet x axis (built without
+// x_edge_sources).
 template <int P, bool NT, bool NTL>
 __global__ void __launch_bounds__(512)
     k_collide_batch(const BatchDesc *__restrict__ descs, const int *__restrict__ map, int wpb, int cur, int own,
@@ -962,7 +968,7 @@ __global__ void __launch_bounds__(512)
   if (row >= nrows || x >= g.nx) return;
   const KConsts<T> c = ldc_obj(reinterpret_cast<const KConsts<T> *>(dp->kc));
   const int *box = ldc(&dp->ib.box);
-  row_cell<P, NT, NTL>(g, BufRows<P>{make_rsrc(ldc(&dp->f[cur])), make_rsrc(ldc(&dp->f[1 - cur]))}, own, c,
+  row_cell<P, NT, NTL>(g, BufRows<P, false>{make_rsrc(ldc(&dp->f[cur])), make_rsrc(ldc(&dp->f[1 - cur]))}, own, c,
                        ldc(&dp->nsheets),
                        box + slot * kMaxSheets * 6, box + (1 - slot) * kMaxSheets * 6,
                        (const FT *)ldc(&dp->F[slot]), (const FT *)ldc(&dp->F[1 - slot]), ldc(&dp->rowtab), row, x,
@@ -992,7 +998,7 @@ __global__ void __launch_bounds__(512)
   if (2 * rp >= nrows || x >= g.nx) return;
   const KConsts<T> c = ldc_obj(reinterpret_cast<const KConsts<T> *>(dp->kc));
   const int *box = ldc(&dp->ib.box);
-  row_pair_cell<P, NT, NTL>(g, make_rsrc(ldc(&dp->f[cur])), make_rsrc(ldc(&dp->f[1 - cur])), own, c,
+  row_pair_cell<P, NT, NTL, false>(g, make_rsrc(ldc(&dp->f[cur])), make_rsrc(ldc(&dp->f[1 - cur])), own, c,
                             ldc(&dp->nsheets), box + slot * kMaxSheets * 6, box + (1 - slot) * kMaxSheets * 6,
                             (const FT *)ldc(&dp->F[slot]), (const FT *)ldc(&dp->F[1 - slot]), ldc(&dp->rowtab),
                             2 * rp, x, box_rows_cached);
@@ -1347,9 +1353,12 @@ static void launch_rows2(int nblocks, const Geometry &g, const void *fin, void *
   const int npairs = g.ny * g.nz / 2;
   const dim3 b((unsigned)((g.nx + 63) / 64 * 64));
   const dim3 gr(nblocks < npairs ? nblocks : npairs);
-  k_collide_stream_rows2<P, NT, NTL><<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets,
-                                                      box_cur, box_prev, (const FT *)Fcur, (const FT *)Fprev, rowtab,
-                                                      box_rows_cached);
+  auto go = [&](auto kern) {
+    kern<<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets, box_cur, box_prev,
+                          (const FT *)Fcur, (const FT *)Fprev, rowtab, box_rows_cached);
+  };
+  if (g.bc[0] == LBMIB_BC_INOUT) go(k_collide_stream_rows2<P, NT, NTL, false>);
+  else go(k_collide_stream_rows2<P, NT, NTL, true>);
 }
 
 // Whether the two-rows-per-block path applies (see k_collide_stream_rows2).
@@ -1370,9 +1379,12 @@ static void launch_pairs(int nblocks, const Geometry &g, const void *fin, void *
   const int nrows = g.ny * g.nz;
   const dim3 b((unsigned)(((g.nx / 2) + 63) / 64 * 64));
   const dim3 gr(nblocks < nrows ? nblocks : nrows);
-  k_collide_stream_pairs<P, NT, NTL><<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets,
-                                                      box_cur, box_prev, (const FT *)Fcur, (const FT *)Fprev, rowtab,
-                                                      band, box_rows_cached);
+  auto go = [&](auto kern) {
+    kern<<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets, box_cur, box_prev,
+                          (const FT *)Fcur, (const FT *)Fprev, rowtab, band, box_rows_cached);
+  };
+  if (g.bc[0] == LBMIB_BC_INOUT) go(k_collide_stream_pairs<P, NT, NTL, false>);
+  else go(k_collide_stream_pairs<P, NT, NTL, true>);
 }
 
 template <int P, bool NT, bool NTL>
@@ -1389,9 +1401,16 @@ static void launch_rows(int nblocks, const Geometry &g, const void *fin, void *f
     kern<<<gr, b, 0, s>>>(g, (const S *)fin, (S *)fout, own, kconsts<P>(c), nsheets, box_cur, box_prev,
                           (const FT *)Fcur, (const FT *)Fprev, tab, band, box_rows_cached);
   };
-  if (rowtab && row_path_buffered(g, sizeof(S))) go(k_collide_stream_rows<P, NT, NTL, kRowsBuf>, rowtab);
-  else if (rowtab_elems) go(k_collide_stream_rows<P, NT, NTL, kRowsPtr>, rowtab_elems);
-  else go(k_collide_stream_rows<P, NT, NTL, kRowsGeneral>, nullptr);
+  const bool edges = g.bc[0] != LBMIB_BC_INOUT;
+  if (rowtab && row_path_buffered(g, sizeof(S))) {
+    if (edges) go(k_collide_stream_rows<P, NT, NTL, kRowsBuf, true>, rowtab);
+    else go(k_collide_stream_rows<P, NT, NTL, kRowsBuf, false>, rowtab);
+  } else if (rowtab_elems) {
+    if (edges) go(k_collide_stream_rows<P, NT, NTL, kRowsPtr, true>, rowtab_elems);
+    else go(k_collide_stream_rows<P, NT, NTL, kRowsPtr, false>, rowtab_elems);
+  } else {
+    go(k_collide_stream_rows<P, NT, NTL, kRowsGeneral, true>, nullptr);
+  }
 }
 
 template <int P, bool NT>
@@ -1537,9 +1556,14 @@ int launch_moments_rows(int prec, const Geometry &g, const void *f, int own, con
                                                 c.rhor * c.urx, c.rho0, c.u0x, c.u0y, c.u0z, c.g, nsheets, box,
                                                 (const typename Traits<P>::FT *)F, tab, out);
     };
-    if (!rowtab) go(k_moments_rows<P, true, kRowsPtr>, rowtab_elems);
-    else if (ntl) go(k_moments_rows<P, true, kRowsBuf>, rowtab);
-    else go(k_moments_rows<P, false, kRowsBuf>, rowtab);
+    auto pick = [&](auto edges) {
+      constexpr bool E = decltype(edges)::value;
+      if (!rowtab) go(k_moments_rows<P, true, kRowsPtr, E>, rowtab_elems);
+      else if (ntl) go(k_moments_rows<P, true, kRowsBuf, E>, rowtab);
+      else go(k_moments_rows<P, false, kRowsBuf, E>, rowtab);
+    };
+    if (g.bc[0] == LBMIB_BC_INOUT) pick(std::false_type{});
+    else pick(std::true_type{});
   }));
   return hipGetLastError() == hipSuccess ? LBMIB_OK : LBMIB_ERR_HIP;
 }
@@ -1553,8 +1577,7 @@ int launch_moments_rows(int prec, const Geometry &g, const void *f, int own, con
 // that are not updated report rho0/u0 like the stored read).  The planes are
 // lbmib_coarse_state's stored planes of the new state, bit for bit.  Needs
 // the buffer-addressed row path with a block as wide as the row, and an
-// inlet/outlet x axis (the x edges of other axes are updated by a second
-// launch, after the sums).
+// inlet/outlet x axis.
 template <int P, bool NT, bool NTL, int F>
 __global__ void __launch_bounds__(1024)
     k_collide_stream_rows_coarse(Geometry g, const typename Traits<P>::S *__restrict__ fin,
@@ -1573,7 +1596,7 @@ __global__ void __launch_bounds__(1024)
   int row;
   for (long it = blockIdx.x; next_row(g, it, row); it += gridDim.x) {
     A sr = (A)rho0, sx = (A)u0x, sy = (A)u0y, sz = (A)u0z;
-    row_cell<P, NT, NTL>(g, BufRows<P>{rin, rout}, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, row, x,
+    row_cell<P, NT, NTL>(g, BufRows<P, false>{rin, rout}, own, c, nsheets, box_cur, box_prev, Fcur, Fprev, rowtab, row, x,
                          nullptr, box_rows_cached, [&](const T *v) {
                            S h[19];
 #pragma unroll
