@@ -1432,29 +1432,35 @@ static void launch_any(int v, const Geometry &g, const void *fin, void *fout, in
 
 // Shape of the fused launch where the caller leaves it open (cpt 0, nt -1): x
 // pairs or one cell per lane, and which accesses are nontemporal.  Each side
-// was measured in the rows layout; times are the fused kernel's, in us.
+// was measured in the rows layout, with and without sheets, from 8 to 1024 cells
+// a row and 10 MB to 2.5 GB an array; times are a step's, in us.
 //  - Rows that are no whole number of 64-byte pieces: each row's first and
 //    last pieces are written by two waves, and nontemporal stores send them to
-//    memory in parts.  Default policy: 500 x 256 x 256 FP32 1314 -> 932, 250 x
-//    100 x 100 FP16 52 -> 36, 151 x 100 x 100 FP64 106 -> 90.  Rows of one wave
-//    in 32 or 64 bits keep nontemporal stores (60 x 280 x 280 FP32 130, 139
-//    with the default policy).
-//  - An array that the 256 MB Infinity Cache holds next to part of the other:
-//    default policy (192 x 100 x 100 FP32 54.1 -> 51.8, 128 x 100 x 100 FP32
-//    38.1 -> 35.2), except rows of one 128-byte line or less (64 x 100 x 100
-//    FP16 16.3, nontemporal 15.2).  Beyond it nontemporal loads and stores
-//    (256^3 FP32 446 -> 435).
+//    memory in parts.  Default policy: 100 x 412 x 412 FP32 777 -> 487, 151 x
+//    116 x 116 FP16 44.6 -> 25.3, FP64 145 -> 116.  Rows of one wave in 32 or 64
+//    bits keep nontemporal stores (50 x 400 x 400 FP32 211, 223 with the default
+//    policy), in 64 bits the loads too (33 x 348 x 348 265, 270).
+//  - The smallest arrays (24 MB, or 400 thousand cells): nontemporal, one cell
+//    per lane (192 x 36 x 36 FP16 6.8, 8.0 with the default policy, 128 x 44 x 44
+//    FP32 9.4 and 11.5, 640 x 24 x 24 FP64 21.8 and 23.2): what the L2s hold
+//    dirty is written back at each kernel's end.
+//  - Else an array that the 256 MB Infinity Cache holds next to part of the
+//    other: default policy (256 x 64 x 64 FP32 27.7 -> 21.7, 128 x 124 x 124 49.9
+//    -> 42.1), except rows of one 128-byte line or less, which stay nontemporal
+//    as on larger arrays (16 x 352 x 352 FP32 112, 118 with the default policy; 64
+//    x 252 x 252 FP16 50.8 and 51.6, though 26.6 and 22.2 at 64 x 176 x 176).
+//    Beyond it nontemporal loads and stores (128 x 252 x 252 FP32 219 -> 199).
 //  - Wall or periodic x: the edge lanes read lines that other lanes read too,
-//    so loads use the default policy (256^3 FP32 448 -> 434, 64 x 288 x 288 212 ->
-//    193); so does the path by scalar addresses (512 x 256 x 256 FP64 1944 ->
-//    1782).
-//  - Pairs: FP32 from 96 cells a row (256^3 435 -> 417, 192 x 256 x 256 325 ->
-//    315; 64 cells fill half a wave: 137 -> 177), FP64 where they fill their
-//    waves (128 x 288 x 288 568 -> 551; 192 x 256 x 256 672 -> 684), in 16 bits
-//    where they fill their waves or beyond 256 cells (288^3 426 -> 355; 192 x
-//    256 x 256 161, pairs 180; 64 x 100 x 100 15.2, pairs 21.8).  Not on small
-//    arrays, and on wall or periodic x only in 16 bits beyond 256 cells
-//    (256^3 FP32 448 -> 520; 288^3 FP16 613 -> 446).
+//    so loads use the default policy (256 x 256 x 256 FP32 469 -> 445, 64 x 252
+//    x 252 152 -> 123); so does the path by scalar addresses (512 x 256 x 256
+//    FP64 1944 -> 1782).
+//  - Pairs where their lanes fill the waves nearly as well as single cells do,
+//    in 32 bits up to 512 cells (256^3 432 -> 418; with a sheet 384 x 104 x 104
+//    129 -> 123, but 160 x 224 x 224 224 -> 252 and 640 x 112 x 112 227 -> 251), in
+//    16 bits there and beyond 256 cells whatever they fill (320 x 160 x 160 108
+//    -> 103; 192 x 296 x 296 209 -> 216); not in 64 bits (256 x 124 x 124 198 ->
+//    211).  Not on small arrays, and on wall or periodic x only in 16 bits beyond
+//    256 cells (256^3 FP32 448 -> 520; 288^3 FP16 613 -> 446).
 FusedShape fused_shape(int prec, const Geometry &g, bool buffered, int cpt_req, int nt_req) {
   const size_t es = prec == LBMIB_F64 ? 8 : (prec == LBMIB_F32 ? 4 : 2);
   const bool half = es == 2, rows = g.prow != g.nx;
@@ -1466,17 +1472,20 @@ FusedShape fused_shape(int prec, const Geometry &g, bool buffered, int cpt_req, 
     sh.cpt = half && buffered && pair_path_ok(g) ? 2 : 1;
   } else {
     const size_t row_bytes = g.nx * es;
-    const bool aligned = row_bytes % 64 == 0;
-    const bool small = 19.0 * g.n * es <= 160.0 * (1 << 20);
+    const double mb = 19.0 * g.n * es / (1 << 20);
+    const bool aligned = row_bytes % 64 == 0, tiny = mb <= 24 || g.n <= 400000;
+    const bool small = mb <= 160;
     bool nts;
-    if (small) nts = row_bytes <= 128;
+    if (small) nts = tiny || row_bytes <= 128;
     else nts = aligned || (g.nx <= 64 && !half);
-    const bool ntl = nts && (aligned || small) && !edges && buffered;
+    const bool ntl = nts && (aligned || small || es == 8) && !edges && buffered;
     sh.nt = (nts ? 1 : 0) | (ntl ? 2 : 0);
-    const bool full = g.nx % 128 == 0;  // pairs fill their waves
+    // lanes of the waves that hold a row: as single cells, as pairs
+    const int lanes1 = (g.nx + 63) / 64 * 64, lanes2 = (g.nx / 2 + 63) / 64 * 64;
+    const bool fills = g.nx >= 96 && 5 * lanes1 >= 4 * 2 * lanes2;
     bool pairs;
-    if (half) pairs = g.nx > 256 || (!edges && !small && full);
-    else pairs = !edges && !small && aligned && (prec == LBMIB_F32 ? g.nx >= 96 : full);
+    if (half) pairs = !tiny && (g.nx > 256 || (!edges && !small && fills));
+    else pairs = es == 4 && !edges && !small && aligned && fills && g.nx <= 512;
     sh.cpt = pairs && buffered && pair_path_ok(g) ? 2 : 1;
   }
   if (nt_req >= 0) sh.nt = nt_req;
