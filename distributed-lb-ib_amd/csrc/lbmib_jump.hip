@@ -155,9 +155,18 @@ __global__ void __launch_bounds__(256)
 // inlet/outlet planes), rho0/u0 elsewhere; the convention lbmib_jump reports
 // a jumped state in -- as per-row partial sums (lbmib_coarse.h): one block
 // per (y, z) row, blockDim.x a multiple of 64 dividing into nx in x steps.
-// The populations are read once, nontemporally: 256^3 FP32 287 -> 225 us (a jump,
-// whose stores rewrite what it reads, is slower so: 435 -> 538).
-template <int P, int F, bool BUF>
+// NTL: the populations, which are read once, come nontemporally (256^3 FP32 287
+// -> 225 us; a jump, whose stores rewrite what it reads, is slower so: 435 ->
+// 538) -- where the array is well beyond the 256 MB Infinity Cache.  One that a
+// step or an earlier read left there in part is read with the default policy
+// (factor 4: 640 x 96 x 96 FP16, 214 MB, 43.8 us, 54.6 nontemporal; 128^3 FP64,
+// 304 MB, 56.2 and 55.7; 64 x 200 x 200 FP64, 371 MB, 71.5 and 66.6).  At
+// factor 1 the planes it writes take their share of that cache: 200 MB is the
+// limit there (64 x 200 x 200 FP32, 186 MB, 50.5 and 53.6; 192^3 FP16, 257 MB,
+// 103 and 89).
+template <int F>
+constexpr double kStoredNtBytes = (F == 1 ? 200.0 : 320.0) * (1 << 20);
+template <int P, int F, bool BUF, bool NTL>
 __global__ void __launch_bounds__(1024)
     k_coarse_stored_rows(Geometry g, const typename Traits<P>::S *__restrict__ f, double rhor, double mrx,
                          double rho0, double u0x, double u0y, double u0z, float *__restrict__ part) {
@@ -176,7 +185,7 @@ __global__ void __launch_bounds__(1024)
         S h[19];
 #pragma unroll
         for (int q = 0; q < 19; ++q) {
-          if constexpr (BUF) h[q] = bld_raw<P, true>(rf, (uint32_t)(c * sizeof(S)), (uint32_t)(q * g.pq * sizeof(S)));
+          if constexpr (BUF) h[q] = bld_raw<P, NTL>(rf, (uint32_t)(c * sizeof(S)), (uint32_t)(q * g.pq * sizeof(S)));
           else h[q] = __builtin_nontemporal_load(f + q * g.pq + c);
         }
         stored_moments<P>(h, rhor, mrx, sr, sx, sy, sz);
@@ -500,10 +509,17 @@ int coarse_launch(lbmib_ctx *ctx, int F, float *out, float *stored) {
       kern<<<rows, row_threads(g, 1024), 0, ctx->stream>>>(g, fp, c.rhor, c.rhor * c.urx, c.rho0, c.u0x, c.u0y,
                                                             c.u0z, ctx->d_cpart);
     };
+    auto pick = [&](auto f) {
+      constexpr int FF = decltype(f)::value;
+      if (!buf) go(k_coarse_stored_rows<P, FF, false, true>);
+      else if (19.0 * g.n * sizeof(typename Traits<P>::S) > kStoredNtBytes<FF>)
+        go(k_coarse_stored_rows<P, FF, true, true>);
+      else go(k_coarse_stored_rows<P, FF, true, false>);
+    };
     switch (F) {
-      case 1: buf ? go(k_coarse_stored_rows<P, 1, true>) : go(k_coarse_stored_rows<P, 1, false>); break;
-      case 2: buf ? go(k_coarse_stored_rows<P, 2, true>) : go(k_coarse_stored_rows<P, 2, false>); break;
-      default: buf ? go(k_coarse_stored_rows<P, 4, true>) : go(k_coarse_stored_rows<P, 4, false>); break;
+      case 1: pick(std::integral_constant<int, 1>{}); break;
+      case 2: pick(std::integral_constant<int, 2>{}); break;
+      default: pick(std::integral_constant<int, 4>{}); break;
     }
     JHIPCHK(hipGetLastError());
     JHIPCHK(launch_coarse_rows(g, F, ctx->d_cpart, stored, ctx->stream));
