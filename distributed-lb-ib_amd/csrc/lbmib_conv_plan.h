@@ -20,6 +20,10 @@ LBMIB_HD int ilog2(int v) {
   return r;
 }
 
+// A launch has fewer than 2^32 threads along x: blocks of 512, rounded up to
+// eight.  Layers of more jobs (8 million samples) are left to the general form.
+constexpr long kMaxJobs = (1L << 23) - 8;
+
 // ------------------------------------------- forward: march (k_conv_march)
 
 struct MarchGeo {
@@ -54,7 +58,7 @@ inline bool march_geo(int B, int D, int H, int W, int Cin, int Cout, int *wm, Ma
     }
   }
   q->jobs = cols * q->zs;
-  return q->jobs < (1L << 30);
+  return q->jobs <= kMaxJobs;
 }
 
 // --------------------------------------------- forward: tile (k_conv_tile)
@@ -102,7 +106,7 @@ inline bool tile_geo(int B, int D, int H, int W, int Cin, int Cout, int wm, int 
   q->lds = (int)(box + 8 * 3072 > red ? box + 8 * 3072 : red);
   q->lgp = ilog2(q->cs / 8);
   q->jobs = (long)B * q->nty * q->ntz * q->cot;
-  return q->jobs < (1L << 30);
+  return q->jobs <= kMaxJobs;
 }
 
 // Position pos of voxel group vg: its plane and line in the tile, and its x.

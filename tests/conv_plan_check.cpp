@@ -2,6 +2,7 @@
 //   tiles   every output voxel of a tile belongs to exactly one position of
 //           its waves, for every line width, tile shape and lines x planes
 //           that the plans give.
+//   grids   every launch that a plan gives has fewer than 2^32 threads.
 //   pieces  every 16-byte piece of a weight-gradient unit comes from the voxel
 //           and channels that the LDS reads expect there.
 // Prints what it finds wrong and returns the number of wrong cases.
@@ -37,6 +38,24 @@ static int tiles() {
           if (out && ++bad <= 10)
             printf("tiles: W %d, H %d, D %d, shape %d %d %d %d, LP %d, PZ %d\n", W, H, D, c.wm, c.nc, c.kw, c.vg, q.LP,
                    q.PZ);
+        }
+  return bad;
+}
+
+static int grids() {
+  int bad = 0;
+  for (long B : {1L, 1000L, 8388600L, 8388601L, 8388608L, 8388616L, 16777216L, 500000000L})
+    for (int side : {1, 2, 8, 64})
+      for (int cin : {16, 32, 64, 256})
+        for (int cout : {16, 48, 256}) {
+          MarchGeo m = {};
+          TileGeo t = {};
+          int wm = 0, shape = 0;
+          const bool mo = march_geo((int)B, side, side, side, cin, cout, &wm, &m);
+          const bool to = tile_plan((int)B, side, side, side, cin, cout, &shape, &t);
+          const long jobs = (mo && m.jobs > t.jobs) || !to ? (mo ? m.jobs : 0) : t.jobs;
+          if ((jobs + 7) / 8 * 8 * 512 >= 1L << 32 && ++bad <= 10)
+            printf("grids: %ld samples of %d^3, %d -> %d channels: %ld jobs\n", B, side, cin, cout, jobs);
         }
   return bad;
 }
@@ -81,6 +100,7 @@ static int pieces() {
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "tiles")) return tiles() != 0;
+  if (!strcmp(what, "grids")) return grids() != 0;
   if (!strcmp(what, "pieces")) return pieces() != 0;
   return 2;
 }

@@ -29,3 +29,7 @@ def test_every_voxel_of_a_tile_has_one_position(check):
 
 def test_every_piece_of_a_weight_gradient_unit_is_the_one_its_readers_expect(check):
     check("pieces")
+
+
+def test_every_launch_has_fewer_threads_than_the_runtime_takes(check):
+    check("grids")

@@ -112,3 +112,23 @@ def test_tile_keeps_an_infinity(case, relu):
 ], ids=lambda c: "x".join(map(str, c)))
 def test_march_keeps_an_infinity(case, relu):
     _with_infinities(case, relu)
+
+
+def test_more_samples_than_a_launch_has_blocks():
+    """8.4 million samples of one voxel: each output is the centre tap's product."""
+    import surrogate as sg
+    B, ci, co = (1 << 23) + 16, 64, 16
+    print(f"conv samples {B}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(33)
+    x = torch.randn((B, ci), generator=gen, device="cuda", dtype=torch.bfloat16)
+    w = (torch.randn((co, 27, ci), generator=gen, device="cuda") / 8).to(torch.bfloat16)
+    y = torch.full((B, co), 7.0, dtype=torch.bfloat16, device="cuda")
+    sg.check(sg._bind().lbmib_sg_conv3d_fwd(sg.ptr(x), sg.ptr(w), None, None, sg.ptr(y), B, 1, 1, 1, ci, co, 0,
+                                            sg.stream()), "conv fwd")
+    torch.cuda.synchronize()
+    wc = w[:, 13].double()
+    for b in (0, B // 2 - 100000, B - 100000):
+        xs = x[b:b + 100000].double()
+        ref, a = xs @ wc.T, 2.0 ** -16 * (xs.abs() @ wc.abs().T)
+        bad = (y[b:b + 100000].double() - ref).abs() > 2.0 ** -8 * (ref.abs() + a) + a
+        assert not bad.any(), (b, int(bad.sum()))
