@@ -3,11 +3,14 @@
 //           its waves, for every line width, tile shape and lines x planes
 //           that the plans give.
 //   grids   every launch that a plan gives has fewer than 2^32 threads.
+//   ranges  the march's z ranges are the best of all counts, found without
+//           trying each.
 //   pieces  every 16-byte piece of a weight-gradient unit comes from the voxel
 //           and channels that the LDS reads expect there.
 // Prints what it finds wrong and returns the number of wrong cases.
 #include <stdio.h>
 #include <string.h>
+#include <time.h>
 
 #include <vector>
 
@@ -60,6 +63,42 @@ static int grids() {
   return bad;
 }
 
+static int ranges() {
+  int bad = 0;
+  for (int cin : {16, 32})
+    for (long cols : {1L, 3L, 17L, 64L, 255L, 256L, 1000L})
+      for (int D = 1; D <= 700; ++D) {
+        MarchGeo q = {};
+        int wm = 0, zc = 0, zs = 0;
+        if (!march_geo((int)cols, D, 4, 64, cin, 32, &wm, &q)) return 1;
+        long best = -1;
+        for (int n = 1; n <= D; ++n) {
+          const int c = (D + n - 1) / n, used = (D + c - 1) / c;
+          const long cost = (cols * used + 255) / 256 * ((c + 1) / 2 + 2);
+          if (best < 0 || cost < best) best = cost, zc = c, zs = used;
+        }
+        if ((q.zc != zc || q.zs != zs) && ++bad <= 10)
+          printf("ranges: %d planes, %ld columns: %d x %d, best %d x %d\n", D, cols, q.zs, q.zc, zs, zc);
+      }
+  // many planes: no more work for the host than for a few
+  const auto spent = [](int D) {
+    MarchGeo q = {};
+    int wm = 0;
+    const clock_t t0 = clock();
+    volatile int used = 0;
+    for (int k = 0; k < 200; ++k) {
+      march_geo(1, D + k % 2, 1, 16, 16, 16, &wm, &q);
+      used = used + q.zc;
+    }
+    return (double)(clock() - t0) / CLOCKS_PER_SEC / 200;
+  };
+  if (spent(1 << 16) > 2e-5 + 50 * spent(1 << 8)) {
+    printf("ranges: %g s for 65,536 planes\n", spent(1 << 16));
+    ++bad;
+  }
+  return bad;
+}
+
 // What lies at byte 16 e of a unit's dy: run e / (16 na) of 8 voxels, 2 na
 // pieces each, the upper half first in odd runs.  x: lines of LP voxels.
 static int pieces() {
@@ -100,6 +139,7 @@ static int pieces() {
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "tiles")) return tiles() != 0;
+  if (!strcmp(what, "ranges")) return ranges() != 0;
   if (!strcmp(what, "grids")) return grids() != 0;
   if (!strcmp(what, "pieces")) return pieces() != 0;
   return 2;

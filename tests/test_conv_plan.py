@@ -33,3 +33,7 @@ def test_every_piece_of_a_weight_gradient_unit_is_the_one_its_readers_expect(che
 
 def test_every_launch_has_fewer_threads_than_the_runtime_takes(check):
     check("grids")
+
+
+def test_z_ranges_are_the_best_and_quickly_found(check):
+    check("ranges")
