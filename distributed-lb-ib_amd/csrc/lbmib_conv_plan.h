@@ -65,6 +65,12 @@ inline bool march_geo(int B, int D, int H, int W, int Cin, int Cout, int *wm, Ma
   return q->jobs <= kMaxJobs;
 }
 
+// Positions that the march computes for each voxel: those of lines past the
+// plane's end, past a line's and of an odd last plane.
+inline double march_fill(const MarchGeo &q, int wm, int D, int H, int W) {
+  return (double)q.nyb * 4 * 16 * wm * q.zs * ((q.zc + 1) / 2 * 2) / ((double)D * H * W);
+}
+
 // --------------------------------------------- forward: tile (k_conv_tile)
 
 struct TileGeo {
@@ -165,6 +171,43 @@ inline bool tile_plan(int B, int D, int H, int W, int Cin, int Cout, int *shape,
     }
   }
   return any;
+}
+
+// Positions that the tiles of a shape compute for each voxel.
+inline double tile_fill(const TileGeo &q, int shape, int D, int H, int W) {
+  const TileShape &c = kTileShapes[shape];
+  return (double)q.nty * q.ntz * 16 * c.wm * c.vg / ((double)D * H * W);
+}
+
+// Which form a layer takes.  The march and the tile work on one sample at a
+// time, on whole lines; the forms below them (k_conv_fwd, k_conv_fwd_kw) on the
+// voxels in linear order, with no position to spare.
+//
+// Few input channels: the march, from where its ~9 us of first loads and
+// launch are no more than the small-grid forms take (16^3 at batch 4, 32 ->
+// 64: 9.2 against 10.6 us; 32 -> 32: 9.0 against 8.5), unless it computes four
+// positions for each voxel (4096 x 1 x 16, 32 -> 32: 40 us, general 15; 1024
+// samples of 8^3, 32 -> 32: 86 and 73; 64 of 10^3, 2.6 positions: 13 and 17).
+//
+// More channels, and few-channel grids too small for the forms below (8^3 at
+// batch 4, 32 -> 64: 6.7 us; from 4096 voxels on those are faster, 7.4 against
+// 7.6 us at 16^3): the tile, unless it takes more than two rounds of 256 blocks
+// and computes 1.5 positions for each voxel (4096 samples of 2^3, 128 -> 128:
+// 345 us, general 66; of 3^3, 64 -> 64: 133 and 59), or two and four (64 of 64 x
+// 1 x 1, 64 -> 256: 33 and 19).  Below that its time is a block's, which the
+// general forms do not reach (64 of 2^3, 256 -> 64: 9 us, general 23).
+enum class ConvForm { march, tile, general };
+inline ConvForm conv_form(int B, int D, int H, int W, int Cin, int Cout, int *wm, MarchGeo *m, int *shape,
+                          TileGeo *t) {
+  const long M = (long)B * D * H * W;
+  if ((M >= 24576 || (M >= 16384 && M * Cout >= 1L << 20)) && march_geo(B, D, H, W, Cin, Cout, wm, m) &&
+      march_fill(*m, *wm, D, H, W) < 4)
+    return ConvForm::march;
+  if ((Cin >= 64 || (Cin == 32 && M < 4096)) && tile_plan(B, D, H, W, Cin, Cout, shape, t)) {
+    const double fill = tile_fill(*t, *shape, D, H, W);
+    if (t->jobs < 512 || (t->jobs == 512 ? fill < 4 : fill < 1.5)) return ConvForm::tile;
+  }
+  return ConvForm::general;
 }
 
 // --------------------------------------------- weight gradient (k_conv_wgrad)

@@ -980,21 +980,18 @@ int conv_fwd(const void *x, const void *w, const float *bias, const void *mask, 
   if (!x || !w || !y || !shape_ok(B, D, H, W, Cin, Cout)) return LBMIB_ERR_ARG;
   const long M = (long)B * D * H * W;
   MarchGeo mg;
-  int wm = 4;
-  // few input channels: the march, from where its ~9 us of first loads and
-  // launch are no more than the small-grid forms take (16^3 at batch 4, 32 ->
-  // 64: 9.2 against 10.6 us; 32 -> 32: 9.0 against 8.5)
-  if ((M >= 24576 || (M >= 16384 && M * Cout >= 1L << 20)) && march_geo(B, D, H, W, Cin, Cout, &wm, &mg))
-    return Cin == 32 ? launch_march_any<32>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s)
-                     : launch_march_any<16>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s);
-  // more channels, and few-channel grids too small for the forms below (8^3
-  // at batch 4, 32 -> 64: 6.7 us; from 4096 voxels on those are faster, 7.4
-  // against 7.6 us at 16^3)
   TileGeo tg;
-  int shape = 0;
-  if ((Cin >= 64 || (Cin == 32 && M < 4096)) && tile_plan(B, D, H, W, Cin, Cout, &shape, &tg))
-    return launch_tile_any(shape, tg, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
-  // lines longer than 64 voxels, and few channels on small grids.  Wave
+  int wm = 4, shape = 0;
+  switch (conv_form(B, D, H, W, Cin, Cout, &wm, &mg, &shape, &tg)) {
+    case ConvForm::march:
+      return Cin == 32 ? launch_march_any<32>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s)
+                       : launch_march_any<16>(wm, mg, x, w, bias, mask, y, D, H, W, Cout, relu, s);
+    case ConvForm::tile:
+      return launch_tile_any(shape, tg, x, w, bias, mask, y, D, H, W, Cin, Cout, relu, s);
+    case ConvForm::general: break;
+  }
+  // lines longer than 64 voxels, few channels on small grids, and many samples
+  // or planes too narrow for the forms above.  Wave
   // tiles: 4 x 16 voxels when the grid is large, fewer when the voxel count
   // alone cannot fill the device; 64 channels per block (32 / 16 for the
   // narrow layers)

@@ -5,6 +5,8 @@
 //   grids   every launch that a plan gives has fewer than 2^32 threads.
 //   ranges  the march's z ranges are the best of all counts, found without
 //           trying each.
+//   forms   a pyramid's layers take the march and the tile; layers of many
+//           narrow samples, on which those mostly compute nothing, do not.
 //   pieces  every 16-byte piece of a weight-gradient unit comes from the voxel
 //           and channels that the LDS reads expect there.
 // Prints what it finds wrong and returns the number of wrong cases.
@@ -99,6 +101,34 @@ static int ranges() {
   return bad;
 }
 
+static int forms() {
+  int bad = 0, wm = 0, shape = 0;
+  MarchGeo m = {};
+  TileGeo t = {};
+  const auto expect = [&](ConvForm want, int B, int D, int H, int W, int cin, int cout) {
+    if (conv_form(B, D, H, W, cin, cout, &wm, &m, &shape, &t) == want) return;
+    printf("forms: %d x %d x %d x %d, %d -> %d channels\n", B, D, H, W, cin, cout);
+    ++bad;
+  };
+  for (int B : {1, 2, 4}) {
+    expect(ConvForm::march, B, 64, 64, 64, 16, 32);
+    expect(ConvForm::march, B, 64, 64, 64, 32, 32);
+    expect(ConvForm::tile, B, 64, 64, 64, 64, 32);
+    for (int side : {2, 4, 8, 16, 32})
+      for (int c : {64, 128, 256}) expect(ConvForm::tile, B, side, side, side, c, c);
+  }
+  for (int c : {64, 128, 256})
+    for (int side : {1, 2}) expect(ConvForm::general, 4096, side, side, side, c, c);
+  expect(ConvForm::general, 4096, 3, 3, 3, 64, 64);
+  expect(ConvForm::general, 64, 64, 1, 1, 64, 256);
+  for (int c : {16, 32}) {
+    expect(ConvForm::general, 1, 4096, 1, 16, c, 32);
+    expect(ConvForm::general, 4096, 2, 4, 8, c, 64);
+    expect(ConvForm::general, 4096, 8, 8, 8, c, 32);
+  }
+  return bad;
+}
+
 // What lies at byte 16 e of a unit's dy: run e / (16 na) of 8 voxels, 2 na
 // pieces each, the upper half first in odd runs.  x: lines of LP voxels.
 static int pieces() {
@@ -139,6 +169,7 @@ static int pieces() {
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "tiles")) return tiles() != 0;
+  if (!strcmp(what, "forms")) return forms() != 0;
   if (!strcmp(what, "ranges")) return ranges() != 0;
   if (!strcmp(what, "grids")) return grids() != 0;
   if (!strcmp(what, "pieces")) return pieces() != 0;

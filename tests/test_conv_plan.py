@@ -37,3 +37,7 @@ def test_every_launch_has_fewer_threads_than_the_runtime_takes(check):
 
 def test_z_ranges_are_the_best_and_quickly_found(check):
     check("ranges")
+
+
+def test_layers_take_the_form_that_suits_them(check):
+    check("forms")

@@ -41,6 +41,22 @@ def _conv(x, w, b, relu):
     (1, 3, 511, 1, 128, 48),
 ], ids=lambda c: "x".join(map(str, c)))
 def test_lines_of_one_voxel(case):
+    _against_oracle(case)
+
+
+@pytest.mark.parametrize("case", [
+    (600, 2, 2, 2, 64, 128),    # the general forms: many samples of few voxels
+    (2500, 1, 1, 1, 256, 64),
+    (70, 64, 1, 1, 64, 256),
+    (1, 1700, 1, 16, 32, 48),   # one line a plane
+    (200, 8, 8, 8, 16, 16),
+    (40, 2, 2, 2, 64, 128),     # the tile: few samples of few voxels
+], ids=lambda c: "x".join(map(str, c)))
+def test_narrow_samples(case):
+    _against_oracle(case)
+
+
+def _against_oracle(case):
     B, D, H, W, ci, co = case
     print(f"conv edges {case}", flush=True)
     rng = np.random.default_rng(31)
