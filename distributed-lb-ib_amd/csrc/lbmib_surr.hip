@@ -1433,7 +1433,7 @@ __global__ void __launch_bounds__(256, 2)
 template <int NA, int NB>
 __global__ void __launch_bounds__(256) k_wgrad_sum(const float *__restrict__ part, const float *__restrict__ bpart,
                                                    float *__restrict__ dw, float *__restrict__ db, int splits, int Cin,
-                                                   int Cout, int ci_tiles, long n4) {
+                                                   int Cout, int ci_tiles, long n4, int taps) {
   __shared__ f32x4 red[16][17];
   const int tid = threadIdx.x, el = tid & 15, g = tid >> 4;
   const long e = (long)blockIdx.x * 16 + el;
@@ -1458,7 +1458,9 @@ __global__ void __launch_bounds__(256) k_wgrad_sum(const float *__restrict__ par
     if (e - n4 < Cout) db[e - n4] = s[0];
     return;
   }
-  const int lane = (int)(e & 63), f = (int)(e >> 6), b = f % NB, a = f / NB % NA, t = f / (NB * NA) % 27;
+  const int lane = (int)(e & 63), f = (int)(e >> 6), b = f % NB, a = f / NB % NA, tv = f / (NB * NA) % 27;
+  const int tl = wgrad_tap(taps, tv), t = tl < 0 ? tv : tl;
+  if (tl < 0) s = f32x4{0.f, 0.f, 0.f, 0.f};
   const int tile = f / (27 * NA * NB);
   const int ci = (tile % ci_tiles) * 32 + 16 * b + (lane & 15);
   const int co = (tile / ci_tiles) * 32 + 16 * a + 4 * (lane >> 4);
@@ -1468,8 +1470,9 @@ __global__ void __launch_bounds__(256) k_wgrad_sum(const float *__restrict__ par
 }
 
 template <int NA, int NB>
-int launch_wgrad(const WgradPlan &p, const void *x, const void *dy, float *dw, float *db, int D, int H, int W, int Cin,
+int launch_wgrad(const WgradPlan &p, const void *x, const void *dy, float *dw, float *db, const WgView &v, int Cin,
                  int Cout, float *part, hipStream_t s) {
+  const int D = v.D, H = v.H, W = v.W;
   float *bpart = db ? part + (size_t)p.n4 * 4 * p.splits : nullptr;
   const int jobs = p.tiles * 3 * p.splits;
   auto go = [&](auto kern) {
@@ -1482,20 +1485,22 @@ int launch_wgrad(const WgradPlan &p, const void *x, const void *dy, float *dw, f
   else go(k_conv_wgrad<NA, NB, true>);
   HIPCHK(hipGetLastError());
   const unsigned nb = (unsigned)(p.n4 / 16 + (db ? (Cout + 15) / 16 : 0));
-  k_wgrad_sum<NA, NB><<<nb, 256, 0, s>>>(part, bpart, dw, db, p.splits, Cin, Cout, p.ci_tiles, p.n4);
+  k_wgrad_sum<NA, NB><<<nb, 256, 0, s>>>(part, bpart, dw, db, p.splits, Cin, Cout, p.ci_tiles, p.n4,
+                                          v.taps);
   HIPCHK(hipGetLastError());
   return LBMIB_OK;
 }
 
 int wgrad_with(const void *x, const void *dy, float *dw, float *db, int B, int D, int H, int W, int Cin, int Cout,
                void *ws, size_t ws_bytes, hipStream_t s) {
-  const WgradPlan p = wgrad_plan(B, D, H, W, Cin, Cout, ws_bytes);
+  const WgView v = wgrad_view(B, D, H, W);
+  const WgradPlan p = wgrad_plan(v.B, v.D, v.H, v.W, Cin, Cout, ws_bytes);
   if (p.part_bytes > ws_bytes || p.q.nunits < 1) return LBMIB_ERR_ARG;
   float *part = (float *)ws;
-  if (p.na == 2 && p.nb == 2) return launch_wgrad<2, 2>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
-  if (p.na == 2) return launch_wgrad<2, 1>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
-  if (p.nb == 2) return launch_wgrad<1, 2>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
-  return launch_wgrad<1, 1>(p, x, dy, dw, db, D, H, W, Cin, Cout, part, s);
+  if (p.na == 2 && p.nb == 2) return launch_wgrad<2, 2>(p, x, dy, dw, db, v, Cin, Cout, part, s);
+  if (p.na == 2) return launch_wgrad<2, 1>(p, x, dy, dw, db, v, Cin, Cout, part, s);
+  if (p.nb == 2) return launch_wgrad<1, 2>(p, x, dy, dw, db, v, Cin, Cout, part, s);
+  return launch_wgrad<1, 1>(p, x, dy, dw, db, v, Cin, Cout, part, s);
 }
 
 // The library's workspace: one buffer per device, allocated on first use.

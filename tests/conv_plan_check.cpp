@@ -7,6 +7,7 @@
 //           trying each.
 //   forms   a pyramid's layers take the march and the tile; layers of many
 //           narrow samples, on which those mostly compute nothing, do not.
+//   views   the weight gradient of a view of a volume is the volume's.
 //   pieces  every 16-byte piece of a weight-gradient unit comes from the voxel
 //           and channels that the LDS reads expect there.
 // Prints what it finds wrong and returns the number of wrong cases.
@@ -129,6 +130,43 @@ static int forms() {
   return bad;
 }
 
+// The weight gradient of one channel over a volume: dw[t] = sum of dy[v] x[v + o(t)].
+static std::vector<long> gradient(const std::vector<int> &x, const std::vector<int> &dy, int B, int D, int H, int W) {
+  std::vector<long> dw(27, 0);
+  for (int b = 0; b < B; ++b)
+    for (int z = 0; z < D; ++z)
+      for (int y = 0; y < H; ++y)
+        for (int i = 0; i < W; ++i)
+          for (int t = 0; t < 27; ++t) {
+            const int zz = z + t / 9 - 1, yy = y + t / 3 % 3 - 1, xx = i + t % 3 - 1;
+            if (zz < 0 || zz >= D || yy < 0 || yy >= H || xx < 0 || xx >= W) continue;
+            dw[t] += (long)dy[((size_t)(b * D + z) * H + y) * W + i] * x[((size_t)(b * D + zz) * H + yy) * W + xx];
+          }
+  return dw;
+}
+
+static int views() {
+  int bad = 0;
+  for (int B : {1, 2, 7, 24, 64, 97, 130})
+    for (int D : {1, 2, 5, 70})
+      for (int H : {1, 3, 9, 66})
+        for (int W : {1, 2}) {
+          std::vector<int> x((size_t)B * D * H * W), dy(x.size());
+          for (size_t k = 0; k < x.size(); ++k) x[k] = (int)(k * 7 % 23) - 9, dy[k] = (int)(k * 5 % 19) - 8;
+          const WgView v = wgrad_view(B, D, H, W);
+          const std::vector<long> want = gradient(x, dy, B, D, H, W), seen = gradient(x, dy, v.B, v.D, v.H, v.W);
+          std::vector<long> got(27, -1);
+          for (int t = 0; t < 27; ++t) {
+            const int l = wgrad_tap(v.taps, t);
+            got[l < 0 ? t : l] = l < 0 ? 0 : seen[t];
+          }
+          const bool narrow = W == 1 && v.W == 1 && (long)B * D * H > 1;
+          if (((long)v.B * v.D * v.H * v.W != (long)x.size() || got != want || narrow) && ++bad <= 10)
+            printf("views: %d x %d x %d x %d as %d x %d x %d x %d\n", B, D, H, W, v.B, v.D, v.H, v.W);
+        }
+  return bad;
+}
+
 // What lies at byte 16 e of a unit's dy: run e / (16 na) of 8 voxels, 2 na
 // pieces each, the upper half first in odd runs.  x: lines of LP voxels.
 static int pieces() {
@@ -169,6 +207,7 @@ static int pieces() {
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "tiles")) return tiles() != 0;
+  if (!strcmp(what, "views")) return views() != 0;
   if (!strcmp(what, "forms")) return forms() != 0;
   if (!strcmp(what, "ranges")) return ranges() != 0;
   if (!strcmp(what, "grids")) return grids() != 0;

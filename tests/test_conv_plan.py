@@ -41,3 +41,7 @@ def test_z_ranges_are_the_best_and_quickly_found(check):
 
 def test_layers_take_the_form_that_suits_them(check):
     check("forms")
+
+
+def test_the_gradient_of_a_view_is_the_volumes(check):
+    check("views")
