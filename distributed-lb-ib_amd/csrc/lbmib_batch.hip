@@ -83,13 +83,18 @@ static int batch_box_rows_auto(const lbmib_batch *b) {
 
 // Nontemporal loads and stores, unless most cells lie in rows that are no
 // whole number of 64-byte pieces, as fused_shape decides for one grid: then
-// the default policy (8 x 100^3 FP32 343 -> 249 us, FP64 488 -> 450, FP16 180
-// -> 152), with nontemporal stores kept where the rows are one wave of 32 or
-// 64 bits (16 x 50^3 FP64 119.8, 129.7 with the default policy).
+// the default policy (8 x 100^3 FP32 364 -> 254 us, FP64 510 -> 456, FP16 212 ->
+// 155; with sheets over 0.4 of each side 337 -> 297, 512 -> 503, 207 -> 188), with
+// nontemporal stores kept where the rows are one wave of 32 or 64 bits (16 x
+// 50^3 FP64 130, 140 with the default policy).  Rows of 32 or 64 bits that fill
+// their waves badly stay nontemporal (12 x (65 x 64 x 64) with sheets FP32 173,
+// 198 with the default policy, FP64 222 and 251).
 static int batch_nt_auto(const lbmib_batch *b) {
   double plain = 0, wave = 0;
   for (const lbmib_ctx *c : b->inst) {
+    const int lanes = (c->g.nx + 63) / 64 * 64;
     if (c->g.nx * c->esz % 64 == 0) continue;
+    if (c->esz > 2 && c->g.nx > 64 && 5 * c->g.nx < 3 * lanes) continue;
     (c->g.nx > 64 || c->esz == 2 ? plain : wave) += (double)c->g.n;
   }
   if (plain > 0.5 * b->cells) return 0;
