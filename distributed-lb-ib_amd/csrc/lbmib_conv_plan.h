@@ -139,7 +139,7 @@ LBMIB_HD TilePos tile_pos(const TileGeo &q, int W, int vg, int pos) {
 
 // The shape of least estimated time, in us: a block's first loads and box,
 // which take longer the more of the 256 CUs fetch at once, its items, and the
-// sum over KW.  The constants are a fit to 13 shapes on 70 layers (Cin 64 to
+// sum over KW.  The constants are a fit to the shapes below on 70 layers (Cin 64 to
 // 256, and 32 below 4096 voxels; 4 to 64 voxels a side, Cout 16 to 256): 6.6%
 // rms, and the shape it picks takes 2% longer than the fastest on average.
 // The narrowest shape leaves room for two blocks a CU where its box is small.
