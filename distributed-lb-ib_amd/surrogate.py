@@ -367,7 +367,8 @@ def bench(batch=4, edge=64, warm=3, iters=10, predict_batch=1):
         out[name] = {"batch": b, "ms": round(ms, 4), "conv_gflop": round(flops / 1e9, 2),
                      "tflops": round(flops / (ms * 1e-3) / 1e12, 1)}
     # per layer and operation: one more pass of each with events around every
-    # convolution call (the calls' own launches, split-K reductions included)
+    # convolution call (the calls' own launches, split-K reductions included);
+    # the median of the calls, as a single one can read 25 ms (which, differs)
     for tag, fn, b in (("train", lambda: net.train_step(x, tgt, 1e-4), batch),
                        ("predict", lambda: net.forward(xp), predict_batch)):
         net.timing = {}
@@ -377,7 +378,7 @@ def bench(batch=4, edge=64, warm=3, iters=10, predict_batch=1):
         rows = []
         for (op, lname), evs in net.timing.items():
             _, ci, co, lvl, _ = next(l for l in net.layers if l[0] == lname)
-            ms = sum(e0.elapsed_time(e1) for e0, e1 in evs) / len(evs)
+            ms = float(np.median([e0.elapsed_time(e1) for e0, e1 in evs]))
             fl = 2 * b * (edge >> lvl) ** 3 * 27 * ci * co
             rows.append({"op": op, "layer": lname, "cin": ci, "cout": co, "grid": edge >> lvl, "us": round(ms * 1e3, 1),
                          "tflops": round(fl / (ms * 1e-3) / 1e12, 1)})
