@@ -488,7 +488,7 @@ int launch_march_any(int wm, const MarchGeo &q, const void *x, const void *w, co
 }
 
 // Forward convolution of 32 or more input channels on lines of at most 64
-// voxels.  A block owns a tile of LP lines x PZ planes (VG groups of G whole
+// voxels (which layers take it is conv_form's to say).  A block owns a tile of LP lines x PZ planes (VG groups of G whole
 // lines, 16 WM positions each) and 16 NC output channels.  It stages the box
 // around the tile, (LP + 2) x (PZ + 2) lines with zeros outside the volume,
 // for all input channels at once (or a slice at a time where that exceeds the

@@ -173,8 +173,8 @@ int lbmib_time_steps(lbmib_ctx *ctx, int nwarm, int nsteps, double *ms_total, do
  *   3 two rows (y, y+1) per block, one cell of each per lane (needs ny even);
  *   4, 8 x-vectors per lane (16 bytes per lane at most; one block per row,
  *     cached loads).
- * nontemporal: bit 0 stores, bit 1 loads; -1 automatic (both on large grids
- *   whose rows are whole 64-byte pieces; see fused_shape in lbmib_fluid.hip).
+ * nontemporal: bit 0 stores, bit 1 loads; -1 automatic (by array size, row
+ *   length and x boundary; the rule is fused_shape in lbmib_fluid.hip).
  * blocks_per_cu > 0: a persistent grid of that many blocks per compute unit
  * walking the rows (0 = one block per row or row pair).  Not in the
  * reference: the knobs bench.py's autotuning sweep sets.  Every variant
@@ -218,7 +218,8 @@ int lbmib_batch_init(lbmib_batch *b);
 int lbmib_batch_step(lbmib_batch *b, int nsteps);
 /* Tile shape of the batched fused launch: 64-lane waves per block (one row,
  * or 64-cell chunk of a row, per wave; a block holds whole rows) and the
- * nontemporal mask as in lbmib_set_kernel_variant.  bench.py autotunes it. */
+ * nontemporal mask as in lbmib_set_kernel_variant, -1 by the instances' rows
+ * (batch_nt_auto in lbmib_batch.hip).  bench.py autotunes it. */
 int lbmib_batch_set_tile(lbmib_batch *b, int waves_per_block, int nontemporal);
 /* Rows per lane of the batched fused launch: 1 (default) or 2, where each
  * lane updates one cell of two neighbouring rows (y, y + 1) of one z plane,
